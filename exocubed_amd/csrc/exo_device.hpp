@@ -137,19 +137,23 @@ EXO_HD double dpow(double x, double y) { return dexp(y * dlog(x)); }
 // smoothness indicators, eps 1e-6, linear weights 3/10, 6/10, 1/10 with the
 // 3/10 term summed first (tests/test_weno.cpp:20-29 returns 2.5000000000000004
 // for 1..5 only in that order).  Reconstruction::Weno5X* apply it per face.
-template <typename R>
-EXO_HD R weno5(R phim2, R phim1, R phi, R phip1, R phip2) {
-  R p0 = (R(1.) / R(3.)) * phi + (R(5.) / R(6.)) * phim1 - (R(1.) / R(6.)) * phim2;
-  R p1 = (R(-1.) / R(6.)) * phip1 + (R(5.) / R(6.)) * phi + (R(1.) / R(3.)) * phim1;
-  R p2 = (R(1.) / R(3.)) * phip2 - (R(7.) / R(6.)) * phip1 + (R(11.) / R(6.)) * phi;
-  R b0 = R(13.) / R(12.) * sqr(phi - R(2.) * phim1 + phim2) +
-         R(.25) * sqr(R(3.) * phi - R(4.) * phim1 + phim2);
-  R b1 = R(13.) / R(12.) * sqr(phip1 - R(2.) * phi + phim1) + R(.25) * sqr(phip1 - phim1);
-  R b2 = R(13.) / R(12.) * sqr(phip2 - R(2.) * phip1 + phi) +
-         R(.25) * sqr(phip2 - R(4.) * phip1 + R(3.) * phi);
-  R a0 = qdiv(R(.3), sqr(b0 + R(1e-6)));
-  R a1 = qdiv(R(.6), sqr(b1 + R(1e-6)));
-  R a2 = qdiv(R(.1), sqr(b2 + R(1e-6)));
+// The FP64 face kernels are bound by FP64 issue, and ten of these values are
+// most of a face.  A product by 2, 4 or 1/4 is exact, so a sum that takes it
+// through an FMA rounds as the separate product and sum do: eight instructions
+// fewer a value with the same bits.
+EXO_HD double weno5(double phim2, double phim1, double phi, double phip1, double phip2) {
+  double p0 = (1. / 3.) * phi + (5. / 6.) * phim1 - (1. / 6.) * phim2;
+  double p1 = (-1. / 6.) * phip1 + (5. / 6.) * phi + (1. / 3.) * phim1;
+  double p2 = (1. / 3.) * phip2 - (7. / 6.) * phip1 + (11. / 6.) * phi;
+  double phi3 = 3. * phi;
+  double b0 = fma(.25, sqr(fma(-4., phim1, phi3) + phim2),
+                  13. / 12. * sqr(fma(-2., phim1, phi) + phim2));
+  double b1 = fma(.25, sqr(phip1 - phim1), 13. / 12. * sqr(fma(-2., phi, phip1) + phim1));
+  double b2 = fma(.25, sqr(fma(-4., phip1, phip2) + phi3),
+                  13. / 12. * sqr(fma(-2., phip1, phip2) + phi));
+  double a0 = qdiv(.3, sqr(b0 + 1e-6));
+  double a1 = qdiv(.6, sqr(b1 + 1e-6));
+  double a2 = qdiv(.1, sqr(b2 + 1e-6));
   return qdiv(a0 * p0 + a1 * p1 + a2 * p2, a0 + a1 + a2);
 }
 

@@ -741,33 +741,44 @@ __device__ __forceinline__ void face_flux64(const DGrid &g, const DState &st, in
   riemann<double>(eos_of<E>(g), rs_of<RK>(g), dir == 1 ? IVY : IVZ, g.gamma, wl, wr, fl, cth, cosf, sinf, 0.);
 }
 
+// Face t of an instance's x2 (dir 1) or x3 (dir 2) faces: panel p, index kk
+// along the edge, level i, face index fa across it.  Lanes walk j in both
+// directions: x2 faces j fastest over N + 1 faces, then i and kk; x3 faces j
+// fastest over N cells, then the face index k, then i, so the six-row stencil
+// along k of consecutive faces is re-read within a few blocks, from L2.  The
+// quotients are 32-bit (an instance has fewer than 2^32 cells, ghosts
+// included, which launcher_setup checks, so fewer faces too): the compiler's
+// 64-bit ones are some 100 instructions each in kernels bound by issue.
+template <int dir>
+__device__ __forceinline__ void face_index(const DGrid &g, unsigned t, int &p, int &kk, int &i,
+                                           int &fa) {
+  unsigned N = g.N, na = N + 1, ni = g.nx1;
+  if (dir == 1) {
+    unsigned r = t / na;
+    fa = (int)(t - r * na);
+    unsigned q = r / ni;
+    i = g.is + (int)(r - q * ni);
+    p = (int)(q / N);
+    kk = (int)(q - p * N);
+  } else {
+    unsigned r = t / N;
+    kk = (int)(t - r * N);
+    unsigned q = r / na;
+    fa = (int)(r - q * na);
+    p = (int)(q / ni);
+    i = g.is + (int)(q - p * ni);
+  }
+}
+
 template <int dir, int EK = -1, int RK = -1>
 __device__ __forceinline__ void flux_h_body(const DGrid &g, const DState &st, int lb) {
   size_t t = (size_t)lb * BLK + threadIdx.x;
-  int N = g.N, ni = g.nx1;
+  int N = g.N;
   int na = N + 1;  // faces along the normal axis
-  size_t total = (size_t)6 * N * ni * na;
+  size_t total = (size_t)6 * N * g.nx1 * na;
   if (t >= total) return;
-  // lanes walk j in both directions: x2 faces (j fastest over N+1 faces),
-  // x3 faces (j fastest over N cells, then the face index k, then i)
   int kk, fa, i, p;
-  if (dir == 1) {
-    fa = (int)(t % na);
-    size_t r = t / na;
-    i = g.is + (int)(r % ni);
-    r /= ni;
-    kk = (int)(r % N);
-    p = (int)(r / N);
-  } else {
-    // j fastest, then the face index k, then i: the six-row stencil along k
-    // of consecutive faces is re-read within a few blocks, from L2
-    kk = (int)(t % N);
-    size_t r = t / N;
-    fa = (int)(r % na);
-    r /= na;
-    i = g.is + (int)(r % ni);
-    p = (int)(r / ni);
-  }
+  face_index<dir>(g, (unsigned)t, p, kk, i, fa);
   int k, j;
   if (dir == 1) { k = g.ks + kk; j = g.js + fa; }
   else { k = g.ks + fa; j = g.js + kk; }
@@ -1212,12 +1223,8 @@ __device__ __forceinline__ void face2_update_body(const DGrid &g, const DState &
   int lane = threadIdx.x & 63;
   size_t F = ((size_t)lb * (BLK / 64) + (threadIdx.x >> 6)) * F2_FACES + lane;
   bool act = F < total;
-  size_t r = act ? F : total - 1;
-  int fa = (int)(r % na);
-  r /= na;
-  int i = g.is + (int)(r % ni);
-  r /= ni;
-  int kk = (int)(r % N), p = (int)(r / N);
+  int fa, i, kk, p;
+  face_index<1>(g, (unsigned)(act ? F : total - 1), p, kk, i, fa);
   int k = g.ks + kk, j = g.js + fa;
   bool cell = act && lane < F2_FACES && fa < N;
   // the update's x1 face fluxes (FP64 form), loaded before the face
@@ -2433,23 +2440,7 @@ __device__ __forceinline__ void flux_h_mix_body(const DGrid &g, const DState &st
   size_t total = (size_t)6 * N * ni * na;
   if (t >= total) return;
   int kk, fa, i, p;
-  if (dir == 1) {
-    fa = (int)(t % na);
-    size_t r = t / na;
-    i = g.is + (int)(r % ni);
-    r /= ni;
-    kk = (int)(r % N);
-    p = (int)(r / N);
-  } else {
-    // j fastest, then the face index k, then i: the six-row stencil along k
-    // of consecutive faces is re-read within a few blocks, from L2
-    kk = (int)(t % N);
-    size_t r = t / N;
-    fa = (int)(r % na);
-    r /= na;
-    i = g.is + (int)(r % ni);
-    p = (int)(r / ni);
-  }
+  face_index<dir>(g, (unsigned)t, p, kk, i, fa);
   int k = dir == 1 ? g.ks + kk : g.ks + fa;
   int j = dir == 1 ? g.js + fa : g.js + kk;
   if (!SW) {
