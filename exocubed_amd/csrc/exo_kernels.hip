@@ -2667,6 +2667,39 @@ __global__ void __launch_bounds__(256) k_out_fields(Grid g, OutMap m, const doub
   }
 }
 
+// ---------------------------------------------------------------------------
+// Planes (p, n, k) of the host MeshBlock layout [p][n][k][j][i] to (TO_DEV) or
+// from the device layout [n][p][k][i][j]: blockIdx.z is the plane q0 + z of the
+// staging buffer `host`, whose planes of nc2 x nc1 doubles follow each other.
+// 32 x 32 tiles through LDS, so both sides move whole lines.  Bound by the
+// copy across the bus beside it: 8 MiB take 6 us here, 0.3 ms there.
+constexpr int XT = 32;
+template <bool TO_DEV>
+__global__ void __launch_bounds__(256) k_layout(Grid g, double *host, double *dev, int nvar,
+                                                unsigned q0) {
+  __shared__ double tile[XT][XT + 1];
+  unsigned q = q0 + blockIdx.z;
+  unsigned k = q % (unsigned)g.nc3, r = q / (unsigned)g.nc3;
+  int n = (int)(r % (unsigned)nvar), p = (int)(r / (unsigned)nvar);
+  double *H = host + (size_t)blockIdx.z * g.nc2 * g.nc1;
+  double *D = dev + g.c(n, p, (int)k, 0, 0);
+  int lx = threadIdx.x % XT, ly = threadIdx.x / XT;
+  int i0 = blockIdx.y * XT, j0 = blockIdx.x * XT;
+  for (int t = ly; t < XT; t += 256 / XT) {  // rows of the source: j (host) or i (device)
+    int i = TO_DEV ? i0 + lx : i0 + t, j = TO_DEV ? j0 + t : j0 + lx;
+    if (i < g.nc1 && j < g.nc2)
+      tile[t][lx] = TO_DEV ? H[(size_t)j * g.nc1 + i] : D[(size_t)i * g.jp + j];
+  }
+  __syncthreads();
+  for (int t = ly; t < XT; t += 256 / XT) {  // rows of the target
+    int i = TO_DEV ? i0 + t : i0 + lx, j = TO_DEV ? j0 + lx : j0 + t;
+    if (i < g.nc1 && j < g.nc2) {
+      if (TO_DEV) D[(size_t)i * g.jp + j] = tile[lx][t];
+      else H[(size_t)j * g.nc1 + i] = tile[lx][t];
+    }
+  }
+}
+
 }  // namespace
 
 // ===========================================================================
@@ -2746,6 +2779,7 @@ struct exo_handle {
   EdgeDesc *d_edge = nullptr;
   double *d_x1 = nullptr, *d_tab = nullptr;
   double *d_sums = nullptr;     // [5] totals of exo_conserved_sums
+  double *d_stage = nullptr;    // stage_doubles(g): pieces of host transfers
   double *d_uov = nullptr;      // per-column factors of the "uov" output (first use)
   float *d_out = nullptr;       // output fields (grown on demand)
   size_t out_cap = 0;           // floats in d_out
@@ -2965,6 +2999,14 @@ void make_grid(const Setup &s, Grid &g) {
   g.t2stride = (size_t)6 * g.nc3 * g.nc2;
 }
 
+// Doubles of the staging buffer of host transfers: whole (p, n, k) planes, at
+// most 8 MiB of them (one plane at least).  Larger pieces copy no faster, and
+// the buffer stays small beside the instance.
+size_t stage_doubles(const Grid &g) {
+  size_t plane = (size_t)g.nc2 * g.nc1, planes = (size_t)6 * std::max(g.nv, g.nt) * g.nc3;
+  return plane * std::max<size_t>(1, std::min(planes, ((size_t)1 << 20) / plane));
+}
+
 // Device bytes one instance allocates (the list init_handle allocates, each
 // rounded up to the allocation granule), for admission by memory footprint.
 size_t footprint_bytes(const Setup &s) {
@@ -3007,6 +3049,7 @@ size_t footprint_bytes(const Setup &s) {
   add(sizeof(int));
   add((size_t)grid1((size_t)6 * g.N * g.N * g.nx1) * 10 * sizeof(double));
   add(5 * sizeof(double));
+  add(stage_doubles(g) * sizeof(double));
   add(sizeof(Inst));
   add(sizeof(int) * K_NKIND * 2);
   return tot;
@@ -3091,6 +3134,7 @@ void init_handle(exo_handle *h) {
   st.bad = (int *)h->dalloc(sizeof(int));
   st.part = (double *)h->dalloc((size_t)grid1((size_t)6 * g.N * g.N * g.nx1) * 10 * sizeof(double));
   h->d_sums = (double *)h->dalloc(5 * sizeof(double));
+  h->d_stage = (double *)h->dalloc(stage_doubles(g) * sizeof(double));
   double dt0[2] = {0., DBL_MAX * 0.4};
   HIPCHK(hipMemcpyAsync(st.dtv, dt0, sizeof(dt0), hipMemcpyHostToDevice, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
@@ -3361,36 +3405,41 @@ void tune_launcher(Launcher &L, int reps) {
   HIPCHK(hipGetLastError());
 }
 
-// copy between the host MeshBlock layout (p, n, k, j, i) and the device
-// layout (n, p, k, i, j)
-void host_to_dev(exo_handle *h, const double *src, double *dst, int nvar) {
-  Grid &g = h->g;
-  std::vector<double> buf((size_t)nvar * g.vstride, 0.);
-  for (int p = 0; p < 6; ++p)
-    for (int n = 0; n < nvar; ++n)
-      for (int k = 0; k < g.nc3; ++k)
-        for (int j = 0; j < g.nc2; ++j)
-          for (int i = 0; i < g.nc1; ++i)
-            buf[g.c(n, p, k, i, j)] =
-                src[((((size_t)p * nvar + n) * g.nc3 + k) * g.nc2 + j) * g.nc1 + i];
-  HIPCHK(hipMemcpyAsync(dst, buf.data(), buf.size() * sizeof(double), hipMemcpyHostToDevice,
-                        h->stream));
+// Copy between the host MeshBlock layout (p, n, k, j, i) and the device layout
+// (n, p, k, i, j): pieces of whole planes cross the bus as they are and the
+// device transposes them (k_layout).  Transposing on the host, one double at a
+// time into another host array, took 55 / 63 ms in / out for 6 x 96 x 96 x 64
+// cells.  All cells are copied, ghosts and corners included.
+template <bool TO_DEV, typename H>
+void transfer(exo_handle *h, H *host, double *dev, int nvar) {
+  const Grid &g = h->g;
+  size_t plane = (size_t)g.nc2 * g.nc1, planes = (size_t)6 * nvar * g.nc3;
+  size_t per = std::min<size_t>(stage_doubles(g) / plane, 32768);  // grid z limit
+  dim3 tiles((g.nc2 + XT - 1) / XT, (g.nc1 + XT - 1) / XT);
+  for (size_t q = 0; q < planes; q += per) {
+    unsigned np = (unsigned)std::min(per, planes - q);
+    dim3 grid(tiles.x, tiles.y, np);
+    size_t bytes = np * plane * sizeof(double);
+    if constexpr (TO_DEV) {
+      HIPCHK(hipMemcpyAsync(h->d_stage, host + q * plane, bytes, hipMemcpyHostToDevice,
+                            h->stream));
+      k_layout<true><<<grid, 256, 0, h->stream>>>(g, h->d_stage, dev, nvar, (unsigned)q);
+    } else {
+      k_layout<false><<<grid, 256, 0, h->stream>>>(g, h->d_stage, dev, nvar, (unsigned)q);
+      HIPCHK(hipMemcpyAsync(host + q * plane, h->d_stage, bytes, hipMemcpyDeviceToHost,
+                            h->stream));
+    }
+  }
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->stream));
 }
 
+void host_to_dev(exo_handle *h, const double *src, double *dst, int nvar) {
+  transfer<true>(h, src, dst, nvar);
+}
+
 void dev_to_host(exo_handle *h, const double *src, double *dst, int nvar) {
-  Grid &g = h->g;
-  std::vector<double> buf((size_t)nvar * g.vstride);
-  HIPCHK(hipMemcpyAsync(buf.data(), src, buf.size() * sizeof(double), hipMemcpyDeviceToHost,
-                        h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
-  for (int p = 0; p < 6; ++p)
-    for (int n = 0; n < nvar; ++n)
-      for (int k = 0; k < g.nc3; ++k)
-        for (int j = 0; j < g.nc2; ++j)
-          for (int i = 0; i < g.nc1; ++i)
-            dst[((((size_t)p * nvar + n) * g.nc3 + k) * g.nc2 + j) * g.nc1 + i] =
-                buf[g.c(n, p, k, i, j)];
+  transfer<false>(h, dst, const_cast<double *>(src), nvar);
 }
 
 // Per-level reference of the mixed path: the horizontal mean of the uploaded
@@ -3402,20 +3451,24 @@ void set_reference(exo_handle *h, const double *u) {
   int nv = g.nv, nc1 = g.nc1, nc2 = g.nc2, nc3 = g.nc3;
   std::vector<double> ref(3 * (size_t)nc1, 0.), pr(nc1, 0.), rh(nc1, 0.);
   double gm1 = g.gamma - 1.0;
+  // one pass over the array in its own order; every level's sum still takes
+  // its cells in the order (p, k, j), so it rounds as a pass for each level does
+  for (int p = 0; p < 6; ++p)
+    for (int k = g.ks; k <= g.ke; ++k)
+      for (int j = g.js; j <= g.je; ++j) {
+        const double *c[5];
+        for (int n = 0; n < nv; ++n)
+          c[n] = u + ((((size_t)p * nv + n) * nc3 + k) * nc2 + j) * nc1;
+        for (int i = g.is; i <= g.ie; ++i) rh[i] += c[IDN][i];
+        if (g.eos == EOS_IDEAL)
+          for (int i = g.is; i <= g.ie; ++i)
+            pr[i] += gm1 * (c[IEN][i] - 0.5 * (c[IVX][i] * c[IVX][i] + c[IVY][i] * c[IVY][i] +
+                                               c[IVZ][i] * c[IVZ][i]) / c[IDN][i]);
+      }
+  double cnt = 6.0 * g.N * g.N;
   for (int i = g.is; i <= g.ie; ++i) {
-    double sp = 0., sr = 0.;
-    for (int p = 0; p < 6; ++p)
-      for (int k = g.ks; k <= g.ke; ++k)
-        for (int j = g.js; j <= g.je; ++j) {
-          auto U = [&](int n) { return u[((((size_t)p * nv + n) * nc3 + k) * nc2 + j) * nc1 + i]; };
-          double d = U(IDN);
-          sr += d;
-          if (g.eos == EOS_IDEAL)
-            sp += gm1 * (U(IEN) - 0.5 * (U(IVX) * U(IVX) + U(IVY) * U(IVY) + U(IVZ) * U(IVZ)) / d);
-        }
-    double cnt = 6.0 * g.N * g.N;
-    rh[i] = sr / cnt;
-    pr[i] = sp / cnt;
+    rh[i] = rh[i] / cnt;
+    pr[i] = pr[i] / cnt;
   }
   for (int i = 0; i < nc1; ++i) {
     int ii = std::min(std::max(i, g.is), g.ie);
