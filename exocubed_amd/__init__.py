@@ -28,7 +28,8 @@ LAUNCH_KINDS = ("prim", "ghost_u", "ghost_s", "x1", "x1_mix", "edge", "edge_mix"
                 "edge_flux", "face_mix_sw", "prim_rest", "prim_ghost", "implicit3",
                 "implicit_avg", "update_rs", "implicit3_avg",
                 "add_du_avg", "face2_update", "face_x2", "face2_update_s",
-                "face2_update_mix", "face2_update_mix_s")
+                "face2_update_mix", "face2_update_mix_s", "sw_stage", "sw_stage_mix", "sw_halo",
+                "sw_edge")
 
 
 def _tuning(caps):

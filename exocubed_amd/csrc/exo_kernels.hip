@@ -106,7 +106,8 @@ struct StateT {
   PTR(double) flx[3], sflx[3];          // face arrays
   PTR(double) edge;                     // [nv][6][4][N][nx1] ghost-side face states
   PTR(double) coef;                     // implicit column coefficients, 30 per cell
-  PTR(unsigned long long) dtbits;       // CFL minimum as ordered bits
+  PTR(unsigned long long) dtbits;       // CFL minimum as ordered bits and count of blocks,
+                                        // over all and DT_SLOTS times (k_dt)
   PTR(double) dtv;                      // [0] dt of the step, [1] previous dt
   // mixed precision: FP32 perturbation fluxes, FP64 reference parts
   PTR(float) fflx[3], fsflx[3];         // face fluxes without the reference pressure
@@ -178,6 +179,8 @@ struct Inst {
   State st;
   const GhostDesc *gd;
   const EdgeDesc *ed;
+  const int *gx;  // [6][4 sides][N][3 depths]: which of gd fills that ghost cell
+                  // (instances whose step is k_sw_stage's, else null)
   int ngd, ned;
 };
 
@@ -256,6 +259,20 @@ constexpr int eos_k() {
   return RK < 0 ? EK : RK <= RS_LMARS_SW ? EOS_SW : EOS_IDEAL;
 }
 
+// Shallow-water primitive state of one cell from its conserved values: depth
+// (raised to the floor; a NaN depth is too) and wind.  The four quotients by
+// sin^2 theta share one correctly rounded reciprocal.
+__device__ __forceinline__ void sw_prim(double &ud, double v, double ww, double cth, double dfloor,
+                                        double &w2, double &w3) {
+  if (!(ud > dfloor)) ud = dfloor;
+  double di = qdiv(1., ud);
+  double sth2 = 1. - cth * cth, ys = qdiv(1., sth2);
+  double wy = div_rn(v, sth2, ys) - div_rn(ww * cth, sth2, ys);
+  double wz = div_rn(-v * cth, sth2, ys) + div_rn(ww, sth2, ys);
+  w2 = wy * di;
+  w3 = wz * di;
+}
+
 // Primitive state of one cell (p, k, i, j) from its conserved values uv
 // (EquationOfState::ConservedToPrimitive of shallow_yz_hydro.cpp /
 // ideal_moist_hydro.cpp): w, the reflecting x1 mirrors and the scalar mixing
@@ -268,21 +285,12 @@ __device__ __forceinline__ void prim_from(const DGrid &g, const DState &st, int 
   double rho_c;
   if (eos_of<EK>(g) == EOS_SW) {
     double ud = uv[IDN];
-    if (!(ud > dfloor)) {  // the floor, written back only where it applies
-      ud = dfloor;
-      st.u[g.c(IDN, p, k, i, j)] = ud;
-    }
-    double v = uv[IVY], ww = uv[IVZ];
-    double di = qdiv(1., ud);
-    // the four quotients by sth2 share one correctly rounded reciprocal
-    double sth2 = 1. - cth * cth, ys = qdiv(1., sth2);
-    double wy = div_rn(v, sth2, ys) - div_rn(ww * cth, sth2, ys);
-    double wz = div_rn(-v * cth, sth2, ys) + div_rn(ww, sth2, ys);
+    // the floor, written back only where it applies
+    if (!(ud > dfloor)) st.u[g.c(IDN, p, k, i, j)] = dfloor;
+    sw_prim(ud, uv[IVY], uv[IVZ], cth, dfloor, wv[IVY], wv[IVZ]);
     rho_c = ud;
     wv[IDN] = ud;
     wv[IVX] = 0.;
-    wv[IVY] = wy * di;
-    wv[IVZ] = wz * di;
   } else {
     double gm1 = g.gamma - 1.0;
     double u_d = uv[IDN], u_m1 = uv[IVX];
@@ -415,6 +423,37 @@ __global__ void __launch_bounds__(BLK) k_prim_ghost(const Inst *__restrict__ I_,
 // Panel-edge ghost remap (CubedSphereUtility::PackData with InteprolateX2/X3,
 // cubed_sphere_utility.cpp:92-617): one thread per (ghost cell, i); the
 // descriptor carries the interpolation weights and vector-map points.
+__device__ __forceinline__ void ghost_source(const DGrid &g, const GhostDesc &d, int i, size_t &o0,
+                                             size_t &o1) {
+  int sp = d.src_panel;
+  if (d.along_x2) {
+    o0 = g.c(0, sp, d.src_row, i, d.src_a0);
+    o1 = g.c(0, sp, d.src_row, i, d.src_a0 + 1);
+  } else {
+    o0 = g.c(0, sp, d.src_a0, i, d.src_row);
+    o1 = g.c(0, sp, d.src_a0 + 1, i, d.src_row);
+  }
+}
+
+// the covariant x2 / x3 components of a ghost cell from the two source cells
+__device__ __forceinline__ void ghost_vector(const GhostDesc &d, double v1y, double v1z, double v2y,
+                                             double v2z, double &vy, double &vz) {
+  vy = qdiv(d.A * v1y + d.B * v2y, d.D);
+  vz = qdiv(d.A * v1z + d.B * v2z, d.D);
+  double sth = d.sth_s, cth = d.cth_s;
+  double vyt = vy, vzt = vz;
+  vy = qdiv(qdiv(vyt, sth), sth) - qdiv(qdiv(vzt * cth, sth), sth);
+  vz = qdiv(qdiv(vzt, sth), sth) - qdiv(qdiv(vyt * cth, sth), sth);
+  double U, V;
+  vec_rll_from_abp(d.src_cy, d.src_cz, d.src_block, vy, vz, &U, &V);
+  vec_abp_from_rll(d.tgt_cy, d.tgt_cz, d.tgt_block, U, V, &vy, &vz);
+  cth = d.cth_t;
+  vyt = vy;
+  vzt = vz;
+  vy = vyt + vzt * cth;
+  vz = vzt + vyt * cth;
+}
+
 __device__ __forceinline__ void ghost_body(const DGrid &g, int lb,
                                            const ADDR(1) GhostDesc *__restrict__ gd, int ndesc,
                                            ADDR(1) double *arr, int nvar, int vectors) {
@@ -423,15 +462,8 @@ __device__ __forceinline__ void ghost_body(const DGrid &g, int lb,
   if (t >= ndesc * ni) return;
   int di = t / ni, i = g.is + t % ni;
   GhostDesc d = *(const GhostDesc *)(gd + di);
-  int sp = d.src_panel;
   size_t o0, o1;
-  if (d.along_x2) {
-    o0 = g.c(0, sp, d.src_row, i, d.src_a0);
-    o1 = g.c(0, sp, d.src_row, i, d.src_a0 + 1);
-  } else {
-    o0 = g.c(0, sp, d.src_a0, i, d.src_row);
-    o1 = g.c(0, sp, d.src_a0 + 1, i, d.src_row);
-  }
+  ghost_source(g, d, i, o0, o1);
   size_t ot = g.c(0, d.tgt_panel, d.tgt_k, i, d.tgt_j);
   for (int n = 0; n < nvar; ++n) {
     if (vectors && (n == IVY || n == IVZ || g.skipv(n))) continue;
@@ -439,23 +471,9 @@ __device__ __forceinline__ void ghost_body(const DGrid &g, int lb,
     arr[n * g.vstride + ot] = qdiv(d.A * v1 + d.B * v2, d.D);
   }
   if (vectors) {
-    double v1y = arr[IVY * g.vstride + o0], v1z = arr[IVZ * g.vstride + o0];
-    double v2y = arr[IVY * g.vstride + o1], v2z = arr[IVZ * g.vstride + o1];
-    double vy = qdiv(d.A * v1y + d.B * v2y, d.D);
-    double vz = qdiv(d.A * v1z + d.B * v2z, d.D);
-    double sth = d.sth_s, cth = d.cth_s;
-    double vyt = vy, vzt = vz;
-    vy = qdiv(qdiv(vyt, sth), sth) - qdiv(qdiv(vzt * cth, sth), sth);
-    vz = qdiv(qdiv(vzt, sth), sth) - qdiv(qdiv(vyt * cth, sth), sth);
-    double U, V;
-    vec_rll_from_abp(d.src_cy, d.src_cz, d.src_block, vy, vz, &U, &V);
-    vec_abp_from_rll(d.tgt_cy, d.tgt_cz, d.tgt_block, U, V, &vy, &vz);
-    sth = d.sth_t;
-    cth = d.cth_t;
-    vyt = vy;
-    vzt = vz;
-    vy = vyt + vzt * cth;
-    vz = vzt + vyt * cth;
+    double vy, vz;
+    ghost_vector(d, arr[IVY * g.vstride + o0], arr[IVZ * g.vstride + o0],
+                 arr[IVY * g.vstride + o1], arr[IVZ * g.vstride + o1], vy, vz);
     arr[IVY * g.vstride + ot] = vy;
     arr[IVZ * g.vstride + ot] = vz;
   }
@@ -628,6 +646,21 @@ k_flux_x1(const Inst *__restrict__ I_, Work w) {
 // 326-576): the interior-side WENO state of each edge face, its IVY / IVZ
 // mapped through lat-lon into the neighbour's frame, stored in the
 // neighbour's ghost-side slot [n][panel][side][a][i].
+__device__ __forceinline__ void edge_store(const DGrid &g, const DState &st, const EdgeDesc &d,
+                                           int i, double *q) {
+  double U, V, vx, vy;
+  vec_rll_from_abp(d.x2s, d.x3s, d.src_block, q[IVY], q[IVZ], &U, &V);
+  vec_abp_from_rll(d.x2d, d.x3d, d.tgt_block, U, V, &vx, &vy);
+  q[IVY] = vx;
+  q[IVZ] = vy;
+  int ni = g.nx1;
+  size_t base = (((size_t)d.tgt_panel * 4 + d.tgt_dir) * g.N + d.tgt_a) * ni + (i - g.is);
+  size_t vs = (size_t)6 * 4 * g.N * ni;
+#pragma unroll
+  for (int n = 0; n < 5; ++n)
+    if (!g.skipv(n)) st.edge[n * vs + base] = q[n];
+}
+
 __device__ __forceinline__ void edge_body(const DGrid &g, const DState &st, int lb,
                                           const ADDR(1) EdgeDesc *__restrict__ ed, int nedge) {
   int t = lb * BLK + threadIdx.x;
@@ -659,16 +692,7 @@ __device__ __forceinline__ void edge_body(const DGrid &g, const DState &st, int 
                 st.w[g.c(n, p, k - 3, i, j)]);
     q[n] = v;
   }
-  double U, V, vx, vy;
-  vec_rll_from_abp(d.x2s, d.x3s, d.src_block, q[IVY], q[IVZ], &U, &V);
-  vec_abp_from_rll(d.x2d, d.x3d, d.tgt_block, U, V, &vx, &vy);
-  q[IVY] = vx;
-  q[IVZ] = vy;
-  size_t base = (((size_t)d.tgt_panel * 4 + d.tgt_dir) * g.N + d.tgt_a) * ni + (i - g.is);
-  size_t vs = (size_t)6 * 4 * g.N * ni;
-#pragma unroll
-  for (int n = 0; n < 5; ++n)
-    if (!g.skipv(n)) st.edge[n * vs + base] = q[n];
+  edge_store(g, st, d, i, q);
 }
 
 __global__ void __launch_bounds__(BLK) k_edge_states(const Inst *__restrict__ I_, Work w) {
@@ -678,37 +702,32 @@ __global__ void __launch_bounds__(BLK) k_edge_states(const Inst *__restrict__ I_
   }
 }
 
+// Value q - 3 places along the face's axis (dir 1: j, 2: k) from element c of a
+// cell array: one base and constant offsets, so that loads along j merge.
+template <int dir, typename P>
+__device__ __forceinline__ auto along(const DGrid &g, P a, size_t c, int q) {
+  return dir == 1 ? a[c + (q - 3)] : a[c + (ptrdiff_t)(q - 3) * (ptrdiff_t)g.plane];
+}
+
 // x2 faces (dir = 1) or x3 faces (dir = 2): WENO5 L/R of the face, the panel
 // edge's ghost side from the exchanged states, and Hydro::RiemannSolver with
 // the cubed-sphere frame maps.  One thread per (panel, k, i, j) face.
 // Hydro flux of the x2 (dir 1) or x3 (dir 2) face (p, k, i, j), j = js + fa
 // (x2) or k = ks + fa (x3), along-edge index kk: WENO5 L/R states, the
 // neighbour panel's state on a panel edge (fa = 0 or N), then riemann().
-template <int dir, int EK = -1, int RK = -1>
+// cell(n, q): variable n of the stencil cell q - 3 places along the face's
+// axis from the cell right of the face.
+template <int dir, int EK = -1, int RK = -1, typename C>
 __device__ __forceinline__ void face_flux64(const DGrid &g, const DState &st, int p, int kk, int fa,
-                                            int i, int k, int j, double *fl) {
+                                            int i, int k, int j, C &&cell, double *fl) {
   constexpr int E = eos_k<EK, RK>();
   int N = g.N, ni = g.nx1;
   double wl[5] = {0, 0, 0, 0, 0}, wr[5] = {0, 0, 0, 0, 0};
 #pragma unroll
   for (int n = 0; n < 5; ++n) {
     if (skip_of<E>(g, n)) continue;
-    double m3, m2, m1, c0, p1, p2;
-    if (dir == 1) {
-      m3 = st.w[g.c(n, p, k, i, j - 3)];
-      m2 = st.w[g.c(n, p, k, i, j - 2)];
-      m1 = st.w[g.c(n, p, k, i, j - 1)];
-      c0 = st.w[g.c(n, p, k, i, j)];
-      p1 = st.w[g.c(n, p, k, i, j + 1)];
-      p2 = st.w[g.c(n, p, k, i, j + 2)];
-    } else {
-      m3 = st.w[g.c(n, p, k - 3, i, j)];
-      m2 = st.w[g.c(n, p, k - 2, i, j)];
-      m1 = st.w[g.c(n, p, k - 1, i, j)];
-      c0 = st.w[g.c(n, p, k, i, j)];
-      p1 = st.w[g.c(n, p, k + 1, i, j)];
-      p2 = st.w[g.c(n, p, k + 2, i, j)];
-    }
+    double m3 = cell(n, 0), m2 = cell(n, 1), m1 = cell(n, 2), c0 = cell(n, 3), p1 = cell(n, 4),
+           p2 = cell(n, 5);
     // on a panel edge the ghost side is the neighbour's state (below)
     if (fa != 0) wl[n] = weno5(p1, c0, m1, m2, m3);
     if (fa != N) wr[n] = weno5(m2, m1, c0, p1, p2);
@@ -739,6 +758,18 @@ __device__ __forceinline__ void face_flux64(const DGrid &g, const DState &st, in
     cth = g.T(T_CTH3, p, k, j);
   }
   riemann<double>(eos_of<E>(g), rs_of<RK>(g), dir == 1 ? IVY : IVZ, g.gamma, wl, wr, fl, cth, cosf, sinf, 0.);
+}
+
+// the same from the primitive state in memory
+template <int dir, int EK = -1, int RK = -1>
+__device__ __forceinline__ void face_flux64(const DGrid &g, const DState &st, int p, int kk, int fa,
+                                            int i, int k, int j, double *fl) {
+  face_flux64<dir, EK, RK>(
+      g, st, p, kk, fa, i, k, j,
+      [&](int n, int q) -> double {
+        return along<dir>(g, st.w, g.c(n, p, k, i, j), q);
+      },
+      fl);
 }
 
 // Face t of an instance's x2 (dir 1) or x3 (dir 2) faces: panel p, index kk
@@ -791,7 +822,7 @@ __device__ __forceinline__ void flux_h_body(const DGrid &g, const DState &st, in
   for (int n = 0; n < g.nt; ++n) {
     double r[6];
     for (int s = 0; s < 6; ++s)
-      r[s] = dir == 1 ? st.r[g.c(n, p, k, i, j - 3 + s)] : st.r[g.c(n, p, k - 3 + s, i, j)];
+      r[s] = along<dir>(g, st.r, g.c(n, p, k, i, j), s);
     double rl = weno5(r[4], r[3], r[2], r[1], r[0]);
     double rr = weno5(r[1], r[2], r[3], r[4], r[5]);
     double m = fl[IDN];
@@ -861,6 +892,76 @@ struct StageW {
   double dfloor, sfloor;
 };
 
+// What the sources of one cell need of its geometry: the x2 / x3 face areas,
+// the volume and its reciprocal, cos theta and (ROWS) the tangents x, y.
+struct CellGeo {
+  double a2l, a2r, a3l, a3r, vol, yvol, cosine, rx, ry;
+};
+
+// GnomonicEquiangle::AddCoordTermsDivergence and the sources of one cell with
+// primitive state w, added to out[] (ROWS: the tangents come with q, else from
+// the set-up tables; without COR, the caller adds the Coriolis source).
+template <bool ROWS, int EK, bool COR = true>
+__device__ __forceinline__ void add_sources(const DGrid &g, int p, int k, int i, int j, double wght,
+                                            const CellGeo &q, const double *w, double *out) {
+  constexpr bool rows = ROWS;
+  // coordinate source terms
+  double sinc = g.T(T_SINC, p, k, j);
+  double sine2 = sinc * sinc;
+  // the shallow-water x1 velocity is zero for good (not loaded)
+  double v1 = eos_of<EK>(g) == EOS_SW ? 0. : w[IVX], v2 = w[IVY], v3 = w[IVZ], rho = w[IDN];
+  double radius = g.x1v[i], yrad = qdiv(1., radius);
+  double v_2 = v2 + v3 * q.cosine, v_3 = v3 + v2 * q.cosine;
+  double pr;
+  if (eos_of<EK>(g) == EOS_SW) {
+    pr = 0.5 * rho * rho;
+  } else {
+    pr = w[IPR];
+    double src1 = div_rn(2.0 * pr + rho * (v2 * v_2 + v3 * v_3), radius, yrad);
+    out[IVX] += wght * src1;
+  }
+  // x_ov_rD / y_ov_rC of the constructor (gnomonic_equiangle.cpp:209-218)
+  double xovrD = div_rn(q.a2l * g.T(T_SIN2, p, k, j) - q.a2r * g.T(T_SIN2, p, k, j + 1), q.vol, q.yvol);
+  double yovrC = div_rn(q.a3l * g.T(T_SIN3, p, k, j) - q.a3r * g.T(T_SIN3, p, k + 1, j), q.vol, q.yvol);
+  double src2 = -xovrD * (pr + rho * v3 * v3 * sine2) - div_rn(rho * v1 * v_2, radius, yrad);
+  out[IVY] += wght * src2;
+  double src3 = -yovrC * (pr + rho * v2 * v2 * sine2) - div_rn(rho * v1 * v_3, radius, yrad);
+  out[IVZ] += wght * src3;
+  // sources
+  if (eos_of<EK>(g) == EOS_IDEAL && g.grav != 0.0) {
+    double src = wght * rho * g.grav;
+    out[IVX] += src;
+    out[IEN] += src * v1;
+  }
+  if (COR && g.coriolis != 0) {
+    double X = rows ? q.rx : g.T(T_TANX, p, k, j), Y = rows ? q.ry : g.T(T_TANY, p, k, j);
+    double f = g.T(T_CORF, p, k, j);
+    double U, V, acc2, acc3;
+    vec_rll_from_abp(X, Y, p + 1, v2, v3, &U, &V);  // CubedSphere::GetUV
+    U = -U;
+    double llU, llV;
+    if (g.coriolis == 1) {
+      llU = f * V;
+      llV = -f * U;
+    } else {
+      double m2 = rho * U, m3 = rho * V;
+      llU = f * m3;
+      llV = -f * m2;
+    }
+    vec_abp_from_rll(X, Y, p + 1, -llU, llV, &acc2, &acc3);  // GetVyVz
+    // (with the row factors: the same C, D and quotient as the cosine given)
+    double cth = rows ? q.cosine : qdiv(-X * Y, sqrt(X * X + 1) * sqrt(Y * Y + 1));
+    double a2c = acc2 + acc3 * cth, a3c = acc3 + acc2 * cth;
+    if (g.coriolis == 1) {
+      out[IVY] += wght * rho * a2c;
+      out[IVZ] += wght * rho * a3c;
+    } else {
+      out[IVY] += wght * a2c;
+      out[IVZ] += wght * a3c;
+    }
+  }
+}
+
 // One cell (p, k, i, j) of the stage: the weighted average, AddFluxDivergence,
 // the coordinate source terms and the sources.  out[] receives the hydro
 // result: the tendency (ideal gas, whose state u is the weighted average and
@@ -923,7 +1024,7 @@ __device__ __forceinline__ void update_cell(const DGrid &g, const DState &st, in
   // from the panel's per-row tables instead, and cos theta = -x y / (C D)
   // from them with the set-up table's expression (exo_setup.cpp), which gives
   // the table's bits for one quotient.
-  const bool rows = !X2R && eos_of<EK>(g) == EOS_SW;
+  constexpr bool rows = !X2R && EK == EOS_SW;
   double rx = 0., ry = 0., rcos = 0.;
   if (rows) {
     rx = g.T1(T1_X, p, j);
@@ -997,65 +1098,14 @@ __device__ __forceinline__ void update_cell(const DGrid &g, const DState &st, in
       out[n] -= div_rn(wght * dflx, vol, yvol);
     }
   }
-  // coordinate source terms
+  double wv[5] = {0., 0., 0., 0., 0.};
+#pragma unroll
+  for (int n = 0; n < 5; ++n)
+    if (!skip_of<EK>(g, n)) wv[n] = st.w[g.c(n, p, k, i, j)];
   double cosine = rows ? rcos : g.T(T_COSC, p, k, j);
-  double sinc = g.T(T_SINC, p, k, j);
   if (cth_out) *cth_out = cosine;
-  double sine2 = sinc * sinc;
-  // the shallow-water x1 velocity is zero for good (not loaded)
-  double v1 = eos_of<EK>(g) == EOS_SW ? 0. : st.w[g.c(IVX, p, k, i, j)], v2 = st.w[g.c(IVY, p, k, i, j)];
-  double v3 = st.w[g.c(IVZ, p, k, i, j)];
-  double rho = st.w[g.c(IDN, p, k, i, j)];
-  double radius = g.x1v[i], yrad = qdiv(1., radius);
-  double v_2 = v2 + v3 * cosine, v_3 = v3 + v2 * cosine;
-  double pr;
-  if (eos_of<EK>(g) == EOS_SW) {
-    pr = 0.5 * rho * rho;
-  } else {
-    pr = st.w[g.c(IPR, p, k, i, j)];
-    double src1 = div_rn(2.0 * pr + rho * (v2 * v_2 + v3 * v_3), radius, yrad);
-    out[IVX] += wght * src1;
-  }
-  // x_ov_rD / y_ov_rC of the constructor (gnomonic_equiangle.cpp:209-218)
-  double xovrD = div_rn(a2l * g.T(T_SIN2, p, k, j) - a2r * g.T(T_SIN2, p, k, j + 1), vol, yvol);
-  double yovrC = div_rn(a3l * g.T(T_SIN3, p, k, j) - a3r * g.T(T_SIN3, p, k + 1, j), vol, yvol);
-  double src2 = -xovrD * (pr + rho * v3 * v3 * sine2) - div_rn(rho * v1 * v_2, radius, yrad);
-  out[IVY] += wght * src2;
-  double src3 = -yovrC * (pr + rho * v2 * v2 * sine2) - div_rn(rho * v1 * v_3, radius, yrad);
-  out[IVZ] += wght * src3;
-  // sources
-  if (eos_of<EK>(g) == EOS_IDEAL && g.grav != 0.0) {
-    double src = wght * rho * g.grav;
-    out[IVX] += src;
-    out[IEN] += src * v1;
-  }
-  if (g.coriolis != 0) {
-    double X = rows ? rx : g.T(T_TANX, p, k, j), Y = rows ? ry : g.T(T_TANY, p, k, j);
-    double f = g.T(T_CORF, p, k, j);
-    double U, V, acc2, acc3;
-    vec_rll_from_abp(X, Y, p + 1, v2, v3, &U, &V);  // CubedSphere::GetUV
-    U = -U;
-    double llU, llV;
-    if (g.coriolis == 1) {
-      llU = f * V;
-      llV = -f * U;
-    } else {
-      double m2 = rho * U, m3 = rho * V;
-      llU = f * m3;
-      llV = -f * m2;
-    }
-    vec_abp_from_rll(X, Y, p + 1, -llU, llV, &acc2, &acc3);  // GetVyVz
-    // (with the row factors: the same C, D and quotient as the cosine above)
-    double cth = rows ? rcos : qdiv(-X * Y, sqrt(X * X + 1) * sqrt(Y * Y + 1));
-    double a2c = acc2 + acc3 * cth, a3c = acc3 + acc2 * cth;
-    if (g.coriolis == 1) {
-      out[IVY] += wght * rho * a2c;
-      out[IVZ] += wght * rho * a3c;
-    } else {
-      out[IVY] += wght * a2c;
-      out[IVZ] += wght * a3c;
-    }
-  }
+  const CellGeo q{a2l, a2r, a3l, a3r, vol, yvol, cosine, rx, ry};
+  add_sources<rows, EK>(g, p, k, i, j, wght, q, wv, out);
   // passive scalars: weighted average and flux divergence into s (with
   // register fluxes the loop is unrolled over the largest count, so the flux
   // arrays are indexed by constants and stay in registers)
@@ -1157,10 +1207,7 @@ __device__ __forceinline__ void face_flux_mix(const DGrid &g, const DState &st, 
     if (g.skipv(n)) continue;
     float v[6];
 #pragma unroll
-    for (int s = 0; s < 6; ++s) {
-      int ks = dir == 1 ? k : k - 3 + s, js = dir == 1 ? j - 3 + s : j;
-      v[s] = st.fw[g.c(n, p, ks, i, js)];
-    }
+    for (int s = 0; s < 6; ++s) v[s] = along<dir>(g, st.fw, g.c(n, p, k, i, j), s);
     wl[n] = weno5f(v[4], v[3], v[2], v[1], v[0]);
     wr[n] = weno5f(v[1], v[2], v[3], v[4], v[5]);
   }
@@ -1253,7 +1300,7 @@ __device__ __forceinline__ void face2_update_body(const DGrid &g, const DState &
         if (n >= g.nt) break;
         float q[6];
 #pragma unroll
-        for (int s = 0; s < 6; ++s) q[s] = st.fw[g.c(g.nv + n, p, k, i, j - 3 + s)];
+        for (int s = 0; s < 6; ++s) q[s] = along<1>(g, st.fw, g.c(g.nv + n, p, k, i, j), s);
         float rl = weno5f(q[4], q[3], q[2], q[1], q[0]);
         float rr = weno5f(q[1], q[2], q[3], q[4], q[5]);
         float m = gl[IDN];
@@ -1274,7 +1321,7 @@ __device__ __forceinline__ void face2_update_body(const DGrid &g, const DState &
         if (n >= g.nt) break;
         double q[6];
 #pragma unroll
-        for (int s = 0; s < 6; ++s) q[s] = st.r[g.c(n, p, k, i, j - 3 + s)];
+        for (int s = 0; s < 6; ++s) q[s] = along<1>(g, st.r, g.c(n, p, k, i, j), s);
         double rl = weno5(q[4], q[3], q[2], q[1], q[0]);
         double rr = weno5(q[1], q[2], q[3], q[4], q[5]);
         double m = fl[IDN];
@@ -1980,19 +2027,14 @@ __global__ void __launch_bounds__(BLK) k_add_du(const Inst *__restrict__ I_, Wor
 // Hydro::NewBlockTimeStep (patches/21.new_blockdt.patch:16-37): per-cell
 // width / signal speed, block minimum, device-wide minimum on the IEEE bits
 // (positive doubles order like unsigned integers).
-// one block per instance (work list of one block each), thread 0 acts
-__global__ void k_dt_reset(const Inst *__restrict__ I_, Work w) {
-  WORK_LOOP(w) {
-    WORK_INST(w);
-    (void)g;
-    (void)lb;
-    if (threadIdx.x == 0) *st.dtbits = 0x7FF0000000000000ull;
-  }
-}
-
 constexpr int DTC = 8;  // cells per thread of the CFL minimum (fewer block atomics)
 
-__device__ __forceinline__ void dt_body(const DGrid &g, const DState &st, int lb, double *wmin) {
+constexpr unsigned long long DT_NONE = 0x7FF0000000000000ull;  // +infinity's bits
+constexpr int DT_SLOTS = 32, DT_LINE = 16;  // lines of the minimum, words of a line
+constexpr int DT_WORDS = DT_LINE * (DT_SLOTS + 1);
+
+__device__ __forceinline__ void dt_body(const DGrid &g, const DState &st, int lb, int nblk,
+                                        double *wmin) {
   int N = g.N, ni = g.nx1;
   size_t total = (size_t)6 * N * ni * N;
   double m = HUGE_VAL;
@@ -2035,34 +2077,66 @@ __device__ __forceinline__ void dt_body(const DGrid &g, const DState &st, int lb
   if (threadIdx.x == 0) {
     double b = wmin[0];
     for (int q = 1; q < (int)(blockDim.x >> 6); ++q) b = wmin[q] < b ? wmin[q] : b;
-    atomicMin((unsigned long long *)st.dtbits, (unsigned long long)__double_as_longlong(b));
+    // The instance's last block turns the minimum into dt and leaves the words
+    // as the next call finds them.  Minimum and count of blocks are kept in
+    // DT_SLOTS lines, then once more over those: 1,728 blocks on one line took
+    // 65 us on 6 x 96 x 96 x 64, 37 this way (42 with launches of their own
+    // for the reset and the result).  Only device-scope atomics touch
+    // the words, so waiting for each is order enough; a fence would write the
+    // caches back and drop them in every block (84 us).
+    unsigned long long *top = (unsigned long long *)st.dtbits;
+    int slot = lb % DT_SLOTS, slots = nblk < DT_SLOTS ? nblk : DT_SLOTS;
+    auto last = [&](unsigned long long *q, unsigned long long v, int count) {
+      atomicMin(q, v);
+      __builtin_amdgcn_s_waitcnt(0);
+      return atomicAdd(q + 1, 1ull) == (unsigned long long)(count - 1);
+    };
+    auto take = [&](unsigned long long *q) {  // the minimum; both words reset
+      unsigned long long v = atomicExch(q, DT_NONE);
+      atomicExch(q + 1, 0ull);
+      return v;
+    };
+    unsigned long long *mine = top + DT_LINE * (1 + slot);
+    if (last(mine, (unsigned long long)__double_as_longlong(b),
+             (nblk - slot + DT_SLOTS - 1) / DT_SLOTS) &&
+        last(top, take(mine), slots)) {
+      double d = __longlong_as_double((long long)take(top)) * g.cfl;
+      // dt = min(cfl * min_cells, 2 dt_prev) (Mesh::NewTimeStep growth limit)
+      double dt = 2.0 * st.dtv[1];
+      if (d < dt) dt = d;
+      st.dtv[0] = dt;
+      st.dtv[1] = dt;
+    }
   }
 }
 
-__global__ void __launch_bounds__(BLK) k_dt(const Inst *__restrict__ I_, Work w) {
+// The CFL time step of every instance in one launch, with the panel-edge states
+// of the first stage of shallow-water instances whose step is k_sw_stage's
+// (work list we): both only read the primitive state, and a launch of its own
+// for each costs a small sphere more than its work.
+// EDGE: the launch has such instances (without, half the registers).
+template <bool EDGE>
+__global__ void __launch_bounds__(BLK) k_dt(const Inst *__restrict__ I_, Work w, Work we, int ngrid) {
   __shared__ double wmin[BLK / 64];
-  WORK_LOOP(w) {
+  for (int h_ = blockIdx.x; h_ < ((int)blockIdx.x < ngrid ? w.nblk : 0); h_ += ngrid) {
     WORK_INST(w);
-    dt_body(g, st, lb, wmin);
+    dt_body(g, st, lb, w.bstart[ii_ + 1] - w.bstart[ii_], wmin);
     __syncthreads();  // wmin is reused by the next block of the loop
   }
+  if constexpr (EDGE)
+    for (int h_ = (int)blockIdx.x - ngrid; h_ >= 0 && h_ < we.nblk; h_ += gridDim.x - ngrid) {
+      WORK_INST(we);
+      edge_body(g, st, lb, glb(I_[ii_].ed), I_[ii_].ned);
+    }
 }
 
-// dt = min(cfl * min_cells, 2 dt_prev) (Mesh::NewTimeStep growth limit)
-__global__ void k_dt_finish(const Inst *__restrict__ I_, Work w, double dt_fixed) {
+// a given time step (one block per instance, thread 0 acts)
+__global__ void k_dt_fixed(const Inst *__restrict__ I_, Work w, double dt_fixed) {
   WORK_LOOP(w) {
     WORK_INST(w);
+    (void)g;
     (void)lb;
-    if (threadIdx.x != 0) continue;
-    if (dt_fixed > 0.0) {
-      st.dtv[0] = dt_fixed;
-      continue;
-    }
-    double d = __longlong_as_double((long long)*st.dtbits) * g.cfl;
-    double dt = 2.0 * st.dtv[1];
-    if (d < dt) dt = d;
-    st.dtv[0] = dt;
-    st.dtv[1] = dt;
+    if (threadIdx.x == 0) st.dtv[0] = dt_fixed;
   }
 }
 
@@ -2431,80 +2505,42 @@ __device__ __forceinline__ void sw_base_flux(double h, double v2, double v3, dou
   f[IVZ] = fz + fy * ct;
 }
 
-template <int dir, bool SW, int RK = -1>
-__device__ __forceinline__ void flux_h_mix_body(const DGrid &g, const DState &st, int lb) {
+// Mixed shallow-water flux of a face off the panel edges: WENO5 and Riemann
+// deltas in FP32 about the face's left cell, the base flux in FP64.  cell(n, q)
+// as in face_flux64.  f receives (IDN, -, IVY, IVZ).  The face arithmetic of
+// panel-edge faces too (fa = 0, N), where only f[IDN] is used, for the scalars.
+template <int dir, int RK = -1, typename C>
+__device__ __forceinline__ void face_flux_sw_mix(const DGrid &g, const DState &st, int p, int kk,
+                                                 int fa, int i, int k, int j, C &&cell, double *f) {
 #pragma clang fp contract(fast)
-  size_t t = (size_t)lb * BLK + threadIdx.x;
   int N = g.N, ni = g.nx1;
-  int na = N + 1;
-  size_t total = (size_t)6 * N * ni * na;
-  if (t >= total) return;
-  int kk, fa, i, p;
-  face_index<dir>(g, (unsigned)t, p, kk, i, fa);
-  int k = dir == 1 ? g.ks + kk : g.ks + fa;
-  int j = dir == 1 ? g.js + fa : g.js + kk;
-  if (!SW) {
-    float fl[5];
-    face_flux_mix<dir, RK>(g, st, p, kk, fa, i, k, j, fl);
-    float m = fl[IDN];
-    ADDR(1) float *F = st.fflx[dir];
-#pragma unroll
-    for (int n = 0; n < 5; ++n)
-      if (!g.skipv(n)) F[g.f(n, p, k, i, j)] = fl[n];
-    for (int n = 0; n < g.nt; ++n) {
-      float r[6];
-      int nr = g.nv + n;  // the tracer's FP32 copy
-      for (int s = 0; s < 6; ++s)
-        r[s] = dir == 1 ? st.fw[g.c(nr, p, k, i, j - 3 + s)] : st.fw[g.c(nr, p, k - 3 + s, i, j)];
-      float rl = weno5f(r[4], r[3], r[2], r[1], r[0]);
-      float rr = weno5f(r[1], r[2], r[3], r[4], r[5]);
-      st.fsflx[dir][g.f(n, p, k, i, j)] = m >= 0.f ? m * rl : m * rr;
-    }
-    return;
-  }
   float wl[5] = {0, 0, 0, 0, 0}, wr[5] = {0, 0, 0, 0, 0}, fl[5];
-  // shallow water: deltas about the face's left cell (riemann_sw_delta)
-  constexpr bool sw = SW;
+  // deltas about the face's left cell (riemann_sw_delta)
   double B[5] = {0., 0., 0., 0., 0.};
-  if (sw) {
-    int kL = dir == 1 ? k : k - 1, jL = dir == 1 ? j - 1 : j;
-    B[IDN] = st.w[g.c(IDN, p, kL, i, jL)];
-    B[IVY] = st.w[g.c(IVY, p, kL, i, jL)];
-    B[IVZ] = st.w[g.c(IVZ, p, kL, i, jL)];
-  }
+  B[IDN] = cell(IDN, 2);
+  B[IVY] = cell(IVY, 2);
+  B[IVZ] = cell(IVZ, 2);
 #pragma unroll
   for (int n = 0; n < 5; ++n) {
-    if (g.skipv(n)) continue;
+    if (skip_of<EOS_SW>(g, n)) continue;
     float v[6];
 #pragma unroll
-    for (int s = 0; s < 6; ++s) {
-      int ks = dir == 1 ? k : k - 3 + s, js = dir == 1 ? j - 3 + s : j;
-      v[s] = sw ? (float)(st.w[g.c(n, p, ks, i, js)] - B[n]) : st.fw[g.c(n, p, ks, i, js)];
-    }
+    for (int s = 0; s < 6; ++s) v[s] = (float)(cell(n, s) - B[n]);
     wl[n] = weno5f(v[4], v[3], v[2], v[1], v[0]);
     wr[n] = weno5f(v[1], v[2], v[3], v[4], v[5]);
   }
-  size_t vs = (size_t)6 * 4 * N * ni;
-  int lo_side = dir == 1 ? 0 : 2;
-  // panel edges: the neighbour's state (FP64 for shallow water, taken about B)
-  if (fa == 0) {
-    size_t b = (((size_t)p * 4 + lo_side) * N + kk) * ni + (i - g.is);
+  // panel edges: the neighbour's FP64 state, taken about B
+  if (fa == 0 || fa == N) {
+    size_t vs = (size_t)6 * 4 * N * ni;
+    int side = (dir == 1 ? 0 : 2) + (fa == 0 ? 0 : 1);
+    size_t b = (((size_t)p * 4 + side) * N + kk) * ni + (i - g.is);
 #pragma unroll
-    for (int n = 0; n < 5; ++n)
-      if (!g.skipv(n)) wl[n] = sw ? (float)(st.edge[n * vs + b] - B[n]) : st.fedge[n * vs + b];
-  } else if (fa == N) {
-    size_t b = (((size_t)p * 4 + lo_side + 1) * N + kk) * ni + (i - g.is);
-#pragma unroll
-    for (int n = 0; n < 5; ++n)
-      if (!g.skipv(n)) wr[n] = sw ? (float)(st.edge[n * vs + b] - B[n]) : st.fedge[n * vs + b];
-  }
-  // full density for the ideal gas
-  float P = 0.f;
-  if (!sw) {
-    float rref = (float)st.lref[2 * g.nc1 + i];
-    wl[IDN] += rref;
-    wr[IDN] += rref;
-    P = (float)st.lref[g.nc1 + i];
+    for (int n = 0; n < 5; ++n) {
+      if (skip_of<EOS_SW>(g, n)) continue;
+      float e = (float)(st.edge[n * vs + b] - B[n]);
+      wl[n] = fa == 0 ? e : wl[n];
+      wr[n] = fa == 0 ? wr[n] : e;
+    }
   }
   double cosd, sind, cthd;
   if (dir == 1) {
@@ -2517,29 +2553,67 @@ __device__ __forceinline__ void flux_h_mix_body(const DGrid &g, const DState &st
     cthd = g.T(T_CTH3, p, k, j);
   }
   float cosf = (float)cosd, sinf = (float)sind, cth = (float)cthd;
-  if (sw) {
-    // FP64 face flux = base flux + FP32 delta; the panel-edge faces are
-    // written by k_edge_flux in FP64
-    float bf[5] = {(float)B[IDN], 0.f, (float)B[IVY], (float)B[IVZ], 0.f}, mb;
-    riemann_sw_delta(rs_of<RK>(g), dir == 1 ? IVY : IVZ, bf, wl, wr, fl, cth, cosf, sinf, &mb);
-    double fb[4];
-    sw_base_flux<dir>(B[IDN], B[IVY], B[IVZ], cosd, sind, cthd, fb);
+  float bf[5] = {(float)B[IDN], 0.f, (float)B[IVY], (float)B[IVZ], 0.f}, mb;
+  riemann_sw_delta(rs_of<RK>(g), dir == 1 ? IVY : IVZ, bf, wl, wr, fl, cth, cosf, sinf, &mb);
+  double fb[4];
+  sw_base_flux<dir>(B[IDN], B[IVY], B[IVZ], cosd, sind, cthd, fb);
+#pragma unroll
+  for (int n = 0; n < 4; ++n) f[n] = n == IVX ? 0. : fb[n] + (double)fl[n];
+}
+
+template <int dir, bool SW, int RK = -1>
+__device__ __forceinline__ void flux_h_mix_body(const DGrid &g, const DState &st, int lb) {
+#pragma clang fp contract(fast)
+  size_t t = (size_t)lb * BLK + threadIdx.x;
+  int N = g.N, ni = g.nx1;
+  int na = N + 1;
+  size_t total = (size_t)6 * N * ni * na;
+  if (t >= total) return;
+  int kk, fa, i, p;
+  face_index<dir>(g, (unsigned)t, p, kk, i, fa);
+  int k = dir == 1 ? g.ks + kk : g.ks + fa;
+  int j = dir == 1 ? g.js + fa : g.js + kk;
+  if constexpr (!SW) {
+    float fl[5];
+    face_flux_mix<dir, RK>(g, st, p, kk, fa, i, k, j, fl);
+    float m = fl[IDN];
+    ADDR(1) float *F = st.fflx[dir];
+#pragma unroll
+    for (int n = 0; n < 5; ++n)
+      if (!g.skipv(n)) F[g.f(n, p, k, i, j)] = fl[n];
+    for (int n = 0; n < g.nt; ++n) {
+      float r[6];
+      int nr = g.nv + n;  // the tracer's FP32 copy
+      for (int s = 0; s < 6; ++s)
+        r[s] = along<dir>(g, st.fw, g.c(nr, p, k, i, j), s);
+      float rl = weno5f(r[4], r[3], r[2], r[1], r[0]);
+      float rr = weno5f(r[1], r[2], r[3], r[4], r[5]);
+      st.fsflx[dir][g.f(n, p, k, i, j)] = m >= 0.f ? m * rl : m * rr;
+    }
+  } else {
+    // the panel-edge faces are written by k_edge_flux in FP64
+    double f[4];
+    face_flux_sw_mix<dir, RK>(
+        g, st, p, kk, fa, i, k, j,
+        [&](int n, int q) -> double {
+          return along<dir>(g, st.w, g.c(n, p, k, i, j), q);
+        },
+        f);
     ADDR(1) double *F = st.flx[dir];
     if (fa != 0 && fa != N) {
 #pragma unroll
       for (int n = 0; n < 4; ++n)
-        if (!g.skipv(n)) F[g.f(n, p, k, i, j)] = fb[n] + (double)fl[n];
+        if (!skip_of<EOS_SW>(g, n)) F[g.f(n, p, k, i, j)] = f[n];
     }
-    double m = fb[IDN] + (double)fl[IDN];
+    double m = f[IDN];
     for (int n = 0; n < g.nt; ++n) {
       float r[6];
       for (int s = 0; s < 6; ++s)
-        r[s] = (float)(dir == 1 ? st.r[g.c(n, p, k, i, j - 3 + s)] : st.r[g.c(n, p, k - 3 + s, i, j)]);
+        r[s] = (float)along<dir>(g, st.r, g.c(n, p, k, i, j), s);
       float rl = weno5f(r[4], r[3], r[2], r[1], r[0]);
       float rr = weno5f(r[1], r[2], r[3], r[4], r[5]);
       st.sflx[dir][g.f(n, p, k, i, j)] = m >= 0.0 ? m * (double)rl : m * (double)rr;
     }
-    return;
   }
 }
 
@@ -2551,6 +2625,367 @@ __global__ void __launch_bounds__(BLK) k_flux_h_mix(const Inst *__restrict__ I_,
   WORK_LOOP(w) {
     WORK_INST(w);
     flux_h_mix_body<dir, SW, RK>(g, st, lb);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The step of a shallow-water instance without scalars: a stage is two
+// launches, k_sw_stage (faces, update) and k_sw_halo (ghost cells, panel-edge
+// states), where the single phases take six (edge states, two face kernels,
+// update, ghost remap, ghost conversion), and the fluxes, the primitive state
+// and the stage register stay off memory.
+//   * Small spheres are bound by the launches, 4.7 us each in a replayed graph,
+//     and by a block's latency: 6 x 48 x 48 x 3 takes 75 us a step instead of
+//     109, 6 x 24 x 24 80 instead of 115.
+//   * Large ones moved some 270 bytes a cell and stage (face fluxes out and in,
+//     u, u1 and w); here a stage reads its input (24 bytes) and, in stages 2
+//     and 3, the step's first state (24), writes 24, and reads 100 bytes of
+//     tables.  What is left is FP64 issue: 56 spheres of 24 to 182 cells a side
+//     (2.3 M cells, Roe) take 0.84 ms a step instead of 1.04, the stage kernel
+//     0.217 ms, 0.17 of it the issue of its instructions.
+// A stage reads u and converts it on the way into LDS (12 % of the cells twice
+// or more, the tiles' margins), so the primitive state is written only by the
+// last one.  No stage may write what its neighbours' tiles read: stage 1 goes
+// from u to u1, 2 from u1 to du, 3 from du back to u, which stages 2 and 3 read
+// at their own cell only, as the step's first state (SSPRK3's u1).  (du is
+// unused by shallow water otherwise; outside a step u1 is the stage register.)
+// A tile is 16 x 15 cells: its 511 faces are one for each of 512 threads or two
+// for each of 256, without a nearly empty pass after them (a 16 x 16 tile has
+// 544; it ran at 0.225 ms a stage of the batch above against 0.218, 32 x 7 cells
+// at 0.239).
+constexpr int SWTJ = 16, SWTK = 15;                  // cells along x2, x3
+constexpr int SWNF = 2 * SWTJ * SWTK + SWTJ + SWTK;  // faces
+constexpr int SWP = SWTJ + 2 * NG + 1;   // row pitch of the tile with its margins in LDS
+struct SwLds {
+  double w[3][SWTK + 2 * NG][SWP];       // primitive state of the tile and its margins
+  double f2[3][SWTK][SWTJ + 1];          // x2 faces, the right edge's included
+  double f3[3][SWTK + 1][SWTJ];          // x3 faces, the upper edge's included
+};
+__device__ __forceinline__ int sw_var(int q) { return q == 0 ? IDN : q == 1 ? IVY : IVZ; }
+
+__device__ __forceinline__ ADDR(1) double *sw_in(const DState &st, int stage) {
+  return stage == 0 ? st.u : stage == 1 ? st.u1 : st.du;
+}
+__device__ __forceinline__ ADDR(1) double *sw_out(const DState &st, int stage) {
+  return stage == 0 ? st.u1 : stage == 1 ? st.du : st.u;
+}
+
+// Flux of one face, x2 or (x3) x3, into f[] (depth, x2 and x3 momentum).  One
+// body serves both directions: the wind is taken as (normal, transverse) and
+// goes through the x2 solver.  The x3 solver's expressions are those with the
+// two components' names exchanged, up to the order of a sum's two terms, so the
+// bits are the same; one body is half the code, and a wavefront may hold faces
+// of both.
+template <bool MIX, int RK>
+__device__ __forceinline__ void sw_face(const DGrid &g, const DState &st, const SwLds &l, int p,
+                                        int i, int x, int y, int j, int k, bool x3, double *f) {
+  int N = g.N, ni = g.nx1;
+  int fa = x3 ? k - g.ks : j - g.js, kk = x3 ? j - g.js : k - g.ks;
+  constexpr int V = (SWTK + 2 * NG) * SWP;
+  const double *w0 = &l.w[0][0][0] + (x3 ? y * SWP + x + NG : (y + NG) * SWP + x);
+  const int wn = (x3 ? 2 : 1) * V, wt = (x3 ? 1 : 2) * V, s = x3 ? SWP : 1;
+  // variable v (0 depth, 1 normal, 2 transverse wind) of stencil cell q
+  auto cell = [&](int v, int q) -> double {
+    return w0[(v == 0 ? 0 : v == 1 ? wn : wt) + q * s];
+  };
+  size_t at = ((size_t)p * g.nc3 + k) * g.nc2 + j;
+  double cosf = g.tab[(x3 ? T_COS3 : T_COS2) * g.t2stride + at];
+  double sinf = g.tab[(x3 ? T_SIN3 : T_SIN2) * g.t2stride + at];
+  double cth = g.tab[(x3 ? T_CTH3 : T_CTH2) * g.t2stride + at];
+  const bool rim = fa == 0 || fa == N;
+  double fl[5];
+  if (!MIX || rim) {  // the mixed form's panel-edge faces are FP64, as both panels' are
+    double wl[5] = {0., 0., 0., 0., 0.}, wr[5] = {0., 0., 0., 0., 0.};
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+      int n = sw_var(v);
+      double m3 = cell(v, 0), m2 = cell(v, 1), m1 = cell(v, 2), c0 = cell(v, 3), p1 = cell(v, 4),
+             p2 = cell(v, 5);
+      // (branches, not selects: they keep the scheduler from working on all six
+      // values at once, 141 registers)
+      if (fa != 0) wl[n] = weno5(p1, c0, m1, m2, m3);
+      if (fa != N) wr[n] = weno5(m2, m1, c0, p1, p2);
+    }
+    if (rim) {  // the ghost side is the neighbour's state (k_edge_states)
+      size_t vs = (size_t)6 * 4 * N * ni;
+      size_t b = (((size_t)p * 4 + (x3 ? 2 : 0) + (fa == 0 ? 0 : 1)) * N + kk) * ni + (i - g.is);
+      double e[3] = {st.edge[IDN * vs + b], st.edge[(x3 ? IVZ : IVY) * vs + b],
+                     st.edge[(x3 ? IVY : IVZ) * vs + b]};
+#pragma unroll
+      for (int v = 0; v < 3; ++v) {
+        int n = sw_var(v);
+        wl[n] = fa == 0 ? e[v] : wl[n];
+        wr[n] = fa == 0 ? wr[n] : e[v];
+      }
+    }
+    riemann<double>(EOS_SW, rs_of<RK>(g), IVY, g.gamma, wl, wr, fl, cth, cosf, sinf, 0.);
+  } else {  // as face_flux_sw_mix
+    float wl[5] = {0, 0, 0, 0, 0}, wr[5] = {0, 0, 0, 0, 0}, fd[5], mb;
+    double B[3] = {cell(0, 2), cell(1, 2), cell(2, 2)};
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+      float q[6];
+#pragma unroll
+      for (int c = 0; c < 6; ++c) q[c] = (float)(cell(v, c) - B[v]);
+      wl[sw_var(v)] = weno5f(q[4], q[3], q[2], q[1], q[0]);
+      wr[sw_var(v)] = weno5f(q[1], q[2], q[3], q[4], q[5]);
+    }
+    float bf[5] = {(float)B[0], 0.f, (float)B[1], (float)B[2], 0.f};
+    riemann_sw_delta(rs_of<RK>(g), IVY, bf, wl, wr, fd, (float)cth, (float)cosf, (float)sinf, &mb);
+    // sw_base_flux, its transverse product in each direction's own order
+    double hs = B[0] * sinf, Ps = qdiv(0.5 * B[0] * B[0], sinf);
+    double fn = hs * B[1] * B[1] + Ps;
+    double ft = hs * (x3 ? B[2] : B[1]) * (x3 ? B[1] : B[2]) - cosf * Ps;
+    fl[IDN] = hs * B[1] + (double)fd[IDN];
+    fl[IVY] = (fn + ft * cth) + (double)fd[IVY];
+    fl[IVZ] = (ft + fn * cth) + (double)fd[IVZ];
+  }
+  f[0] = fl[IDN];
+  f[1] = x3 ? fl[IVZ] : fl[IVY];
+  f[2] = x3 ? fl[IVY] : fl[IVZ];
+}
+
+// The Coriolis source of one cell: add_sources' expressions with C and D from
+// the row tables and quotients that share a divisor sharing its correctly
+// rounded reciprocal, some 300 instructions fewer (no register is spared for
+// them in k_update; here the faces need more than this).
+__device__ __forceinline__ void sw_coriolis(const DGrid &g, int p, int k, int j, double wght,
+                                            double X, double Y, double C, double D, double cth,
+                                            double h, double v2, double v3, double *out) {
+  double f = g.T(T_CORF, p, k, j);
+  double delta = sqrt(1 + X * X + Y * Y);
+  bool polar = p == 0 || p == 4;
+  double U, V, r1 = 0., r2, r3 = 0., r4;
+  if (polar) {
+    double E = sqrt(X * X + Y * Y), sg = p == 0 ? -1. : 1.;
+    double DE = D * E, CE = C * E, yD = qdiv(1., DE), yC = qdiv(1., CE);
+    U = sg * (div_rn(delta * Y, DE, yD) * v2 - div_rn(delta * X, CE, yC) * v3);
+    V = sg * (div_rn(X, DE, yD) * v2 + div_rn(Y, CE, yC) * v3);
+    double dE = delta * E, yE = qdiv(1., dE), e = qdiv(1., E);
+    r1 = sg * div_rn(D * Y, dE, yE);
+    r2 = sg * div_rn(D * X, E, e);
+    r3 = -sg * div_rn(C * X, dE, yE);
+    r4 = sg * div_rn(C * Y, E, e);
+  } else {
+    double CD = C * D, yCD = qdiv(1., CD), yd = qdiv(1., delta);
+    U = div_rn(delta, CD, yCD) * v3;
+    V = -cth * v3 - v2;
+    r1 = div_rn(X * Y, delta, yd);
+    r2 = -1.;
+    r3 = div_rn(CD, delta, yd);
+    r4 = 0.;
+  }
+  U = -U;
+  double a, b, s = wght;
+  if (g.coriolis == 1) {
+    a = f * V;
+    b = -f * U;
+    s = wght * h;
+  } else {
+    a = f * (h * V);
+    b = -f * (h * U);
+  }
+  a = -a;
+  double acc2 = r1 * a + r2 * b, acc3 = polar ? r3 * a + r4 * b : r3 * a;
+  out[IVY] += s * (acc2 + acc3 * cth);
+  out[IVZ] += s * (acc3 + acc2 * cth);
+}
+
+template <bool MIX, int RK, int NT>
+__device__ __forceinline__ void sw_stage_body(const DGrid &g, const DState &st, int lb,
+                                              const StageW &sw, int stage, SwLds &l) {
+  int N = g.N, ntj = (N + SWTJ - 1) / SWTJ, ntk = (N + SWTK - 1) / SWTK, ni = g.nx1;
+  int tj = lb % ntj, r = lb / ntj;
+  int tk = r % ntk;
+  r /= ntk;
+  int i = g.is + r % ni, p = r / ni;
+  int j0 = g.js + tj * SWTJ, k0 = g.ks + tk * SWTK;
+  const int tid = threadIdx.x;
+  const ADDR(1) double *in = sw_in(st, stage);
+  ADDR(1) double *outp = sw_out(st, stage);
+  size_t vs = g.vstride;
+  // the tile and its margins into LDS, one cell a thread: the tile, then left
+  // and right, then lower and upper.  Cells past the panel's ghosts are no
+  // stencil's, nor are the corners.
+  for (int t = tid; t < SWTJ * SWTK + 2 * NG * (SWTJ + SWTK); t += NT) {
+    constexpr int M = 2 * NG;
+    int x = t % SWTJ, y = t / SWTJ;
+    if (t >= SWTJ * SWTK) {
+      int m = t - SWTJ * SWTK;
+      bool lr = m < M * SWTK;
+      int q = lr ? m % M : (m - M * SWTK) / SWTJ, a = lr ? m / M : (m - M * SWTK) % SWTJ;
+      int o = q < NG ? q - NG : (lr ? SWTJ : SWTK) + q - NG;
+      x = lr ? o : a;
+      y = lr ? a : o;
+    }
+    int j = j0 + x, k = k0 + y;
+    if (j < g.nc2 && k < g.nc3) {
+      size_t c = g.c(0, p, k, i, j);
+      double h = in[IDN * vs + c], w2, w3;
+      sw_prim(h, in[IVY * vs + c], in[IVZ * vs + c], g.T(T_COSC, p, k, j), sw.dfloor, w2, w3);
+      l.w[0][y + NG][x + NG] = h;
+      l.w[1][y + NG][x + NG] = w2;
+      l.w[2][y + NG][x + NG] = w3;
+    }
+  }
+  __syncthreads();
+  // the tile's faces: SWTJ + 1 columns of x2 faces, SWTK + 1 rows of x3 faces
+  constexpr int NF2 = (SWTJ + 1) * SWTK;
+#pragma unroll 1
+  for (int t = tid; t < SWNF; t += NT) {
+    bool x3 = t >= NF2;
+    int f = x3 ? t - NF2 : t;
+    int y = x3 ? f / SWTJ : f / (SWTJ + 1), x = x3 ? f % SWTJ : f % (SWTJ + 1);
+    int j = j0 + x, k = k0 + y;
+    if (j <= g.je + (x3 ? 0 : 1) && k <= g.ke + (x3 ? 1 : 0)) {
+      double fl[3];
+      sw_face<MIX, RK>(g, st, l, p, i, x, y, j, k, x3, fl);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        if (x3) l.f3[q][y][x] = fl[q];
+        else l.f2[q][y][x] = fl[q];
+      }
+    }
+  }
+  __syncthreads();
+  if (tid >= SWTJ * SWTK) return;
+  int x = tid % SWTJ, y = tid / SWTJ;
+  int j = j0 + x, k = k0 + y;
+  if (j > g.je || k > g.ke) return;
+  // the cell: update_cell's expressions, with the tangents from the row tables
+  double dt = st.dtv[0];
+  double wght = sw.beta * dt;
+  CellGeo geo;
+  geo.a2l = g.area2(p, k, j, i);
+  geo.a3l = g.area3(p, k, j, i);
+  geo.vol = g.volume(p, k, j, i);
+  geo.a2r = g.area2(p, k, j + 1, i);
+  geo.a3r = g.area3(p, k + 1, j, i);
+  geo.yvol = qdiv(1., geo.vol);
+  geo.rx = g.T1(T1_X, p, j);
+  geo.ry = g.T1(T1_Y, p, k);
+  double cth = geo.cosine = g.T(T_COSC, p, k, j);
+  size_t c = g.c(0, p, k, i, j);
+  double out[5] = {0., 0., 0., 0., 0.}, wv[5] = {0., 0., 0., 0., 0.};
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    int n = sw_var(q);
+    // the stage register of the step's first state is 0 + u
+    double uv = in[n * vs + c];
+    double u = sw.first ? 0. + uv : sw.g1 * uv + sw.g2 * (0. + st.u[n * vs + c]);
+    double dflx = 0.;
+    dflx += geo.a2r * l.f2[q][y][x + 1] - geo.a2l * l.f2[q][y][x];
+    dflx += geo.a3r * l.f3[q][y + 1][x] - geo.a3l * l.f3[q][y][x];
+    out[n] = u - div_rn(wght * dflx, geo.vol, geo.yvol);
+    wv[n] = l.w[q][y + NG][x + NG];
+  }
+  // (each part's loads stay with it: hoisted together they take the kernel past
+  // the registers of five wavefronts a SIMD, two blocks a CU)
+  __builtin_amdgcn_sched_barrier(0);
+  add_sources<true, EOS_SW, false>(g, p, k, i, j, wght, geo, wv, out);
+  __builtin_amdgcn_sched_barrier(0);
+  if (g.coriolis != 0)
+    sw_coriolis(g, p, k, j, wght, geo.rx, geo.ry, g.T1(T1_C, p, j), g.T1(T1_D, p, k), cth, wv[IDN],
+                wv[IVY], wv[IVZ], out);
+  double h = out[IDN], w2, w3;
+  sw_prim(h, out[IVY], out[IVZ], cth, sw.dfloor, w2, w3);
+  outp[IDN * vs + c] = h;  // with the floor, as the conversion writes it back
+  outp[IVY * vs + c] = out[IVY];
+  outp[IVZ * vs + c] = out[IVZ];
+  if (stage == 2) {
+    st.w[IDN * vs + c] = h;
+    st.w[IVY * vs + c] = w2;
+    st.w[IVZ * vs + c] = w3;
+  }
+}
+
+// RK: the Riemann solver of every instance of the launch, or -1.  NT: threads,
+// 512 for launches that leave CUs without a tile, where a block's latency is
+// what counts (6 x 48 x 48 x 3, 216 tiles: 12.0 against 13.6 us, event times),
+// else 256, four blocks a CU in different phases (6 x 192 x 192 mixed, 936
+// tiles: 21.9 against 23.4 us; the batch 0.218 against 0.298 ms).
+template <bool MIX, int RK, int NT>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
+k_sw_stage(const Inst *__restrict__ I_, Work w, StageW sw, int stage) {
+  __shared__ SwLds l;
+  WORK_LOOP(w) {
+    WORK_INST(w);
+    sw_stage_body<MIX, RK, NT>(g, st, lb, sw, stage, l);
+    __syncthreads();  // the tile is refilled by the next block of the loop
+  }
+}
+
+// The halo of a stage's result: thread (panel, side, a, i) fills the three
+// ghost cells of its row (k_ghost's remap) and, from two of them and the row's
+// first three cells, the interior-side state of the panel-edge face
+// (k_edge_states), which goes to the neighbour's slot.  The last stage writes
+// the ghost cells' primitive state instead: the next step's first states come
+// with its CFL minimum (k_dt).
+__device__ __forceinline__ void sw_halo_body(const DGrid &g, const DState &st, int lb, const Inst &I,
+                                             double dfloor, int stage) {
+  int t = lb * BLK + threadIdx.x;
+  int ni = g.nx1;
+  if (t >= I.ned * ni) return;
+  int e = t / ni, i = g.is + t % ni;
+  EdgeDesc d = *(const EdgeDesc *)(glb(I.ed) + e);
+  int p = d.src_panel, side = d.src_dir, a = side < 2 ? d.src_k - g.ks : d.src_j - g.js;
+  ADDR(1) double *arr = sw_out(st, stage);
+  size_t vs = g.vstride;
+  // the cells of the row across the edge: ghosts q = 1 (depth 1), 0, -1, ..
+  auto place = [&](int depth, int &k, int &j) {
+    int lo = g.is - 1 - depth, hi = g.je + 1 + depth;  // is = js = ks, je = ke
+    k = side == 2 ? lo : side == 3 ? hi : g.ks + a;
+    j = side == 0 ? lo : side == 1 ? hi : g.js + a;
+  };
+  double s[3][5];  // the face's WENO5 cells: two ghosts, three cells
+#pragma unroll
+  for (int depth = 0; depth < NG; ++depth) {
+    GhostDesc gd = *(const GhostDesc *)(glb(I.gd) + I.gx[((p * 4 + side) * g.N + a) * NG + depth]);
+    size_t o0, o1;
+    ghost_source(g, gd, i, o0, o1);
+    double h = qdiv(gd.A * arr[IDN * vs + o0] + gd.B * arr[IDN * vs + o1], gd.D), v2, v3;
+    ghost_vector(gd, arr[IVY * vs + o0], arr[IVZ * vs + o0], arr[IVY * vs + o1],
+                 arr[IVZ * vs + o1], v2, v3);
+    int k, j;
+    place(depth, k, j);
+    size_t c = g.c(0, p, k, i, j);
+    double w2, w3;
+    sw_prim(h, v2, v3, g.T(T_COSC, p, k, j), dfloor, w2, w3);
+    arr[IDN * vs + c] = h;
+    arr[IVY * vs + c] = v2;
+    arr[IVZ * vs + c] = v3;
+    if (stage == 2) {
+      st.w[IDN * vs + c] = h;
+      st.w[IVY * vs + c] = w2;
+      st.w[IVZ * vs + c] = w3;
+    } else if (depth < 2) {
+      s[0][1 - depth] = h;
+      s[1][1 - depth] = w2;
+      s[2][1 - depth] = w3;
+    }
+  }
+  if (stage == 2) return;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    int k, j;
+    place(-1 - q, k, j);
+    size_t c = g.c(0, p, k, i, j);
+    double h = arr[IDN * vs + c], w2, w3;
+    sw_prim(h, arr[IVY * vs + c], arr[IVZ * vs + c], g.T(T_COSC, p, k, j), dfloor, w2, w3);
+    s[0][2 + q] = h;
+    s[1][2 + q] = w2;
+    s[2][2 + q] = w3;
+  }
+  double q[5] = {0., 0., 0., 0., 0.};
+  for (int v = 0; v < 3; ++v) q[sw_var(v)] = weno5(s[v][0], s[v][1], s[v][2], s[v][3], s[v][4]);
+  edge_store(g, st, d, i, q);
+}
+
+__global__ void __launch_bounds__(BLK) k_sw_halo(const Inst *__restrict__ I_, Work w, double dfloor,
+                                                 int stage) {
+  WORK_LOOP(w) {
+    WORK_INST(w);
+    sw_halo_body(g, st, lb, I_[ii_], dfloor, stage);
   }
 }
 
@@ -2724,7 +3159,10 @@ enum {
   // within a stage, the FP64 ideal gas takes its x2 faces and update in one
   // kernel (k_face2_update, without and with scalars), FP64 shallow water its
   // separate x2 face kernel (the mixed forms have their own kinds)
-  K_FUSE2, K_FACE_NF, K_FUSE2_S, K_FUSE2_MIX, K_FUSE2_MIX_S, K_NKIND
+  K_FUSE2, K_FACE_NF, K_FUSE2_S, K_FUSE2_MIX, K_FUSE2_MIX_S,
+  // within a step, shallow water without scalars: its stages, their halos and
+  // the first stage's panel-edge states
+  K_SW, K_SW_MIX, K_SW_HALO, K_SW_EDGE, K_NKIND
 };
 
 // kernel ids of the profile (exo_profile_end)
@@ -2741,13 +3179,17 @@ struct Launcher {
   hipStream_t stream = nullptr;
   int ninst = 0;
   Inst *d_inst = nullptr;
-  int *d_bstart = nullptr;  // [K_NKIND][ninst + 1]
-  int nblk[K_NKIND] = {};
+  // two work lists: of the single phases, and (mode 1) of a whole step, where
+  // k_sw_stage takes the shallow-water instances it covers off the others
+  int mode = 0;
+  int *d_bstart = nullptr;  // [mode][K_NKIND][ninst + 1]
+  int nblk[2][K_NKIND] = {};
   int cap[K_NKIND] = {};    // workgroups of a persistent launch (0: one per block)
   int shape[K_NKIND] = {};  // tuned block shape of a kind (0: the default): the x1
                             // kinds' waves per 64-column block (2, 4 or 8)
   int eos = -1;             // equation of state of every instance (-1: they differ)
   int rs = -1;              // Riemann solver of every instance (-1: they differ)
+  int ncu = 0;              // CUs of the device
   std::vector<Inst> h_inst;     // host copies of the instances (the tuner reads them)
   size_t lds_x1 = 0;        // dynamic LDS of the x1 kernels (largest instance)
   // live per-kernel timing with HIP events on the stream
@@ -2757,10 +3199,10 @@ struct Launcher {
   std::vector<int> ev_kind;
 
   Work work(int kind) const {
-    return Work{d_bstart + (size_t)kind * (ninst + 1), ninst, nblk[kind]};
+    return Work{d_bstart + ((size_t)mode * K_NKIND + kind) * (ninst + 1), ninst, nblk[mode][kind]};
   }
   unsigned grid(int kind) const {
-    int n = nblk[kind];
+    int n = nblk[mode][kind];
     return (unsigned)(cap[kind] > 0 && cap[kind] < n ? cap[kind] : n);
   }
 };
@@ -2777,6 +3219,7 @@ struct exo_handle {
   std::vector<void *> allocs;
   GhostDesc *d_ghost = nullptr;
   EdgeDesc *d_edge = nullptr;
+  int *d_gx = nullptr;          // Inst::gx
   double *d_x1 = nullptr, *d_tab = nullptr;
   double *d_sums = nullptr;     // [5] totals of exo_conserved_sums
   double *d_stage = nullptr;    // stage_doubles(g): pieces of host transfers
@@ -2828,8 +3271,20 @@ hipEvent_t next_event(Launcher &L) {
 }
 
 // blocks of one instance in a launch of the given kind (0: not applicable)
-int kind_blocks(int kind, const Grid &g, bool mixed, int ngd, int ned) {
+bool sw_fused(const Grid &g) { return g.eos == EOS_SW && g.nt == 0; }
+
+// step: the work list of a whole step (Launcher::mode 1)
+int kind_blocks(int kind, const Grid &g, bool mixed, int ngd, int ned, bool step) {
   bool ideal = g.eos == EOS_IDEAL;
+  bool sw = step && sw_fused(g);
+  int tiles = ((g.N + SWTJ - 1) / SWTJ) * ((g.N + SWTK - 1) / SWTK);
+  switch (kind) {
+    case K_SW: return sw && !mixed ? 6 * g.nx1 * tiles : 0;
+    case K_SW_MIX: return sw && mixed ? 6 * g.nx1 * tiles : 0;
+    case K_SW_HALO:
+    case K_SW_EDGE: return sw ? (int)grid1((size_t)ned * g.nx1) : 0;
+  }
+  if (sw && kind != K_DT && kind != K_ONE && kind != K_CELLS) return 0;
   size_t cells = (size_t)6 * g.N * g.N * g.nx1;
   size_t faces = (size_t)6 * g.N * g.nx1 * (g.N + 1);
   size_t cols = (size_t)g.N * g.N;
@@ -2889,7 +3344,7 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
   int n = (int)hs.size();
   L.ninst = n;
   std::vector<Inst> inst(n);
-  std::vector<int> tab((size_t)K_NKIND * (n + 1));
+  std::vector<int> tab((size_t)2 * K_NKIND * (n + 1));
   L.lds_x1 = 0;
   for (int i = 0; i < n; ++i) {
     const exo_handle *h = hs[i];
@@ -2897,6 +3352,7 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
     inst[i].st = h->st;
     inst[i].gd = h->d_ghost;
     inst[i].ed = h->d_edge;
+    inst[i].gx = h->d_gx;
     inst[i].ngd = (int)h->setup.ghosts.size();
     inst[i].ned = (int)h->setup.edges.size();
     L.lds_x1 = std::max(L.lds_x1, (size_t)(h->g.nc1 + 1) * 64 * sizeof(double));
@@ -2908,21 +3364,24 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
     if (hs[i]->g.rs != L.rs) L.rs = -1;
   }
   L.h_inst = inst;
-  for (int kind = 0; kind < K_NKIND; ++kind) {
-    long long acc = 0;
-    for (int i = 0; i < n; ++i) {
-      tab[(size_t)kind * (n + 1) + i] = (int)acc;
-      acc += kind_blocks(kind, hs[i]->g, hs[i]->mixed, inst[i].ngd, inst[i].ned);
+  for (int m = 0; m < 2; ++m)
+    for (int kind = 0; kind < K_NKIND; ++kind) {
+      int *t = &tab[((size_t)m * K_NKIND + kind) * (n + 1)];
+      long long acc = 0;
+      for (int i = 0; i < n; ++i) {
+        t[i] = (int)acc;
+        acc += kind_blocks(kind, hs[i]->g, hs[i]->mixed, inst[i].ngd, inst[i].ned, m == 1);
+      }
+      if (acc > 0x7fffffffLL) throw std::string("work list too large for one launch");
+      t[n] = (int)acc;
+      L.nblk[m][kind] = (int)acc;
     }
-    if (acc > 0x7fffffffLL) throw std::string("work list too large for one launch");
-    tab[(size_t)kind * (n + 1) + n] = (int)acc;
-    L.nblk[kind] = (int)acc;
-  }
   {
     int dev = 0, maxlds = 0;
     HIPCHK(hipGetDevice(&dev));
+    HIPCHK(hipDeviceGetAttribute(&L.ncu, hipDeviceAttributeMultiprocessorCount, dev));
     HIPCHK(hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    bool need_x1 = L.nblk[K_X1] > 0 || L.nblk[K_X1_MIX] > 0;
+    bool need_x1 = L.nblk[0][K_X1] > 0 || L.nblk[0][K_X1_MIX] > 0;
     for (const exo_handle *h : hs)
       if ((size_t)6 * h->g.nc3 * h->g.nc2 * h->g.nc1 >= ((size_t)1 << 32))
         throw std::string("instance too large: 2^32 cells or more");
@@ -2962,7 +3421,7 @@ void set_shape(Launcher &L, int kind, int shape) {
 template <typename... P, typename... A>
 void launch(Launcher &L, int kind, int kid, void (*kern)(const Inst *, Work, P...), unsigned block,
             size_t lds, A... args) {
-  if (L.nblk[kind] == 0) return;
+  if (L.nblk[L.mode][kind] == 0) return;
   bool t = L.prof && kid >= 0;
   if (t) {
     L.ev_kind.push_back(kid);
@@ -3022,6 +3481,7 @@ size_t footprint_bytes(const Setup &s) {
   add((s.tab2.size() + s.tab1.size()) * sizeof(double));
   add(s.ghosts.size() * sizeof(GhostDesc));
   add(s.edges.size() * sizeof(EdgeDesc));
+  if (sw_fused(g)) add(s.ghosts.size() * sizeof(int));
   for (int q = 0; q < 4; ++q) add(cell * g.nv);           // u, w, u1, du
   if (g.nt)
     for (int q = 0; q < 3; ++q) add(cell * g.nt);         // s, r, s1
@@ -3044,14 +3504,14 @@ size_t footprint_bytes(const Setup &s) {
     add(g.vstride * sizeof(float) * (g.nv + g.nt));  // fw
   }
   if (mixed) add(3 * (size_t)g.nc1 * sizeof(double));
-  add(sizeof(unsigned long long));
+  add(DT_WORDS * sizeof(unsigned long long));
   add(2 * sizeof(double));
   add(sizeof(int));
   add((size_t)grid1((size_t)6 * g.N * g.N * g.nx1) * 10 * sizeof(double));
   add(5 * sizeof(double));
   add(stage_doubles(g) * sizeof(double));
   add(sizeof(Inst));
-  add(sizeof(int) * K_NKIND * 2);
+  add(sizeof(int) * 2 * K_NKIND * 2);
   return tot;
 }
 
@@ -3087,6 +3547,21 @@ void init_handle(exo_handle *h) {
   h->d_edge = (EdgeDesc *)h->dalloc(s.edges.size() * sizeof(EdgeDesc));
   HIPCHK(hipMemcpyAsync(h->d_edge, s.edges.data(), s.edges.size() * sizeof(EdgeDesc),
                         hipMemcpyHostToDevice, h->stream));
+  std::vector<int> gx;
+  if (sw_fused(g)) {
+    gx.assign(s.ghosts.size(), 0);
+    for (size_t q = 0; q < s.ghosts.size(); ++q) {
+      const GhostDesc &d = s.ghosts[q];
+      bool x2 = d.tgt_j < g.js || d.tgt_j > g.je;
+      int at = x2 ? d.tgt_j : d.tgt_k, along = x2 ? d.tgt_k - g.ks : d.tgt_j - g.js;
+      int lo = x2 ? g.js : g.ks, hi = x2 ? g.je : g.ke;
+      int side = (x2 ? 0 : 2) + (at > hi ? 1 : 0), depth = at > hi ? at - hi - 1 : lo - 1 - at;
+      gx[((size_t)(d.tgt_panel * 4 + side) * g.N + along) * NG + depth] = (int)q;
+    }
+    h->d_gx = (int *)h->dalloc(gx.size() * sizeof(int));
+    HIPCHK(hipMemcpyAsync(h->d_gx, gx.data(), gx.size() * sizeof(int), hipMemcpyHostToDevice,
+                          h->stream));
+  }
   // state
   State &st = h->st;
   std::memset(&st, 0, sizeof(st));
@@ -3129,7 +3604,11 @@ void init_handle(exo_handle *h) {
     st.fw = (float *)h->dalloc((size_t)(g.nv + g.nt) * g.vstride * sizeof(float));
   }
   if (h->mixed) st.lref = (double *)h->dalloc((size_t)3 * g.nc1 * sizeof(double));
-  st.dtbits = (unsigned long long *)h->dalloc(sizeof(unsigned long long));
+  st.dtbits = (unsigned long long *)h->dalloc(DT_WORDS * sizeof(unsigned long long));
+  std::vector<unsigned long long> bits0(DT_WORDS, 0);
+  for (int q = 0; q < DT_WORDS; q += DT_LINE) bits0[q] = DT_NONE;
+  HIPCHK(hipMemcpyAsync(st.dtbits, bits0.data(), DT_WORDS * sizeof(unsigned long long),
+                        hipMemcpyHostToDevice, h->stream));
   st.dtv = (double *)h->dalloc(2 * sizeof(double));
   st.bad = (int *)h->dalloc(sizeof(int));
   st.part = (double *)h->dalloc((size_t)grid1((size_t)6 * g.N * g.N * g.nx1) * 10 * sizeof(double));
@@ -3289,12 +3768,22 @@ void launch_implicit(Launcher &L, double beta) {
   HIPCHK(hipGetLastError());
 }
 
+// the time step (dt_fixed <= 0: from the CFL condition) and, within a step, the
+// panel-edge states of its first stage (K_SW_EDGE)
 void launch_dt(Launcher &L, double dt_fixed) {
-  if (dt_fixed <= 0.0) {
-    launch(L, K_ONE, -1, k_dt_reset, 64, 0);
-    launch(L, K_DT, KID_DT, k_dt, BLK, 0);
+  bool cfl = dt_fixed <= 0.0;
+  if (!cfl) launch(L, K_ONE, -1, k_dt_fixed, 64, 0, dt_fixed);
+  Work w = L.work(K_DT), we = L.work(K_SW_EDGE);
+  unsigned nd = cfl ? L.grid(K_DT) : 0;
+  if (nd + we.nblk == 0) return;
+  if (!cfl) w.nblk = 0;
+  if (L.prof) {
+    L.ev_kind.push_back(KID_DT);
+    HIPCHK(hipEventRecord(next_event(L), L.stream));
   }
-  launch(L, K_ONE, -1, k_dt_finish, 64, 0, dt_fixed);
+  auto kern = we.nblk ? k_dt<true> : k_dt<false>;
+  kern<<<dim3(nd + L.grid(K_SW_EDGE)), dim3(BLK), 0, L.stream>>>(L.d_inst, w, we, (int)nd);
+  if (L.prof) HIPCHK(hipEventRecord(next_event(L), L.stream));
   HIPCHK(hipGetLastError());
 }
 
@@ -3314,9 +3803,34 @@ void run_stage(Launcher &L, int stage) {
   launch_fill_ghosts_stage(L);
 }
 
+// one stage of the shallow-water instances whose step is k_sw_stage's (mode 1)
+void launch_sw(Launcher &L, int stage) {
+  int s0 = stage - 1;
+  StageW sw{SS_DELTA[s0], SS_G1[s0], SS_G2[s0], SS_BETA[s0], s0 == 0 ? 1 : 0, 1, DFLOOR, SFLOOR};
+  with_solver<EOS_SW>(L, [&](auto R) {
+    constexpr int RK = decltype(R)::value;
+    if (L.nblk[1][K_SW] <= L.ncu)
+      launch(L, K_SW, KID_UPDATE, k_sw_stage<false, RK, 512>, 512, 0, sw, s0);
+    else launch(L, K_SW, KID_UPDATE, k_sw_stage<false, RK, 256>, 256, 0, sw, s0);
+    if (L.nblk[1][K_SW_MIX] <= L.ncu)
+      launch(L, K_SW_MIX, KID_UPDATE, k_sw_stage<true, RK, 512>, 512, 0, sw, s0);
+    else launch(L, K_SW_MIX, KID_UPDATE, k_sw_stage<true, RK, 256>, 256, 0, sw, s0);
+  });
+  launch(L, K_SW_HALO, KID_GHOST, k_sw_halo, BLK, 0, DFLOOR, s0);
+  HIPCHK(hipGetLastError());
+}
+
 void run_step(Launcher &L, double dt_fixed) {
+  struct Mode {  // back to the single phases' work list also when a launch throws
+    Launcher &L;
+    explicit Mode(Launcher &l) : L(l) { L.mode = 1; }
+    ~Mode() { L.mode = 0; }
+  } mode(L);
   launch_dt(L, dt_fixed);
-  for (int stg = 1; stg <= 3; ++stg) run_stage(L, stg);
+  for (int stg = 1; stg <= 3; ++stg) {
+    run_stage(L, stg);
+    launch_sw(L, stg);
+  }
 }
 
 // compensated conserved totals of every instance into out[ninst][5] (device)
@@ -3331,9 +3845,7 @@ void launch_sums(Launcher &L, double *out) {
 // reads the conserved state (so repeating it changes nothing), time each
 // candidate width and keep the fastest.  Widths are multiples of the CU count.
 void tune_launcher(Launcher &L, int reps) {
-  int dev = 0, ncu = 0;
-  HIPCHK(hipGetDevice(&dev));
-  HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  const int ncu = L.ncu;
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
@@ -3353,10 +3865,10 @@ void tune_launcher(Launcher &L, int reps) {
     int best_cap = 0, best_shape = 0;
     for (int sh : shapes) {
       set_shape(L, kind, sh);
-      if (L.nblk[kind] == 0) break;
+      if (L.nblk[0][kind] == 0) break;
       std::vector<int> cands = {0};
       for (int m : {1, 2, 4, 8, 16})
-        if ((long long)m * ncu < L.nblk[kind]) cands.push_back(m * ncu);
+        if ((long long)m * ncu < L.nblk[0][kind]) cands.push_back(m * ncu);
       for (int c : cands) {
         L.cap[kind] = c;
         for (int r = -1; r < reps; ++r) {  // r = -1 warms up
@@ -3376,7 +3888,12 @@ void tune_launcher(Launcher &L, int reps) {
             case K_FACE: launch_face64<1>(L, K_FACE, -1); break;
             case K_FACE_MIX: launch_face_mix<1, false>(L, K_FACE_MIX, -1); break;
             case K_FACE_MIX_SW: launch_face_mix<1, true>(L, K_FACE_MIX_SW, -1); break;
-            case K_DT: launch(L, K_DT, -1, k_dt, BLK, 0); break;
+            case K_DT: {
+              Work none{nullptr, 0, 0};
+              k_dt<false><<<dim3(L.grid(K_DT)), dim3(BLK), 0, L.stream>>>(
+                  L.d_inst, L.work(K_DT), none, (int)L.grid(K_DT));
+              break;
+            }
             case K_FUSE2: launch_fuse2<false, false>(L, K_FUSE2, -1, sw); break;
             case K_FUSE2_MIX: launch_fuse2<false, true>(L, K_FUSE2_MIX, -1, sw); break;
           }
