@@ -169,6 +169,30 @@ __device__ __forceinline__ DState to_global(const State &h) {
 
 constexpr int BLK = 256;
 
+// Remap tables of an instance, made on the host from its descriptors: by ghost
+// cell [panel][side][depth][along] and by edge face [panel][side][along], each
+// entry of its own array, so that lanes along an edge read whole lines.  The
+// panel <-> lat-lon maps of a fixed point are products with constants; formed
+// here from the descriptor's tangents with the maps' own expressions
+// (vec_rll_from_abp, vec_abp_from_rll), they leave the kernels a few products
+// where each map took four square roots and four to eight divisions.
+enum { GT_A = 0, GT_B, GT_D, GT_YD, GT_STH, GT_YSTH, GT_CTH, GT_CTHT, GT_MAP, GT_N = GT_MAP + 8 };
+enum { GI_SRC0 = 0, GI_SRC1, GI_POLAR, GI_N };  // elements of variable 0, level 0
+enum { ET_MAP = 0, ET_N = 8 };
+enum { EI_SLOT = 0, EI_POLAR, EI_N };  // slot: target (panel * 4 + side) * 2^16 + along
+
+// The map of one vector from a point's panel frame to another's: m[0..3] to
+// east and north, m[4..7] from them.  Off the polar panels east takes the x3
+// component alone, and x3 the east one.
+__device__ __forceinline__ void frame_map(const double *m, int polar, double v2, double v3,
+                                          double &o2, double &o3) {
+  double U = m[1] * v3, V = m[2] * v2 + m[3] * v3;
+  if (polar & 1) U = m[0] * v2 + U;
+  o2 = m[4] * U + m[5] * V;
+  o3 = m[6] * U;
+  if (polar & 2) o3 = o3 + m[7] * V;
+}
+
 // One instance as the kernels see it, and the work list of one launch.  The
 // blocks of a launch are split over the instances by a prefix table (an
 // instance that a kernel does not apply to gets no blocks); a launch with
@@ -177,10 +201,10 @@ constexpr int BLK = 256;
 struct Inst {
   Grid g;
   State st;
-  const GhostDesc *gd;
-  const EdgeDesc *ed;
-  const int *gx;  // [6][4 sides][N][3 depths]: which of gd fills that ghost cell
-                  // (instances whose step is k_sw_stage's, else null)
+  const double *gt;  // [GT_N][ngd] and [GI_N][ngd]: the ghost remap (RemapTables)
+  const int *gi;
+  const double *et;  // [ET_N][ned] and [EI_N][ned]: the panel-edge exchange
+  const int *ei;
   int ngd, ned;
 };
 
@@ -423,57 +447,111 @@ __global__ void __launch_bounds__(BLK) k_prim_ghost(const Inst *__restrict__ I_,
 // Panel-edge ghost remap (CubedSphereUtility::PackData with InteprolateX2/X3,
 // cubed_sphere_utility.cpp:92-617): one thread per (ghost cell, i); the
 // descriptor carries the interpolation weights and vector-map points.
-__device__ __forceinline__ void ghost_source(const DGrid &g, const GhostDesc &d, int i, size_t &o0,
-                                             size_t &o1) {
-  int sp = d.src_panel;
-  if (d.along_x2) {
-    o0 = g.c(0, sp, d.src_row, i, d.src_a0);
-    o1 = g.c(0, sp, d.src_row, i, d.src_a0 + 1);
-  } else {
-    o0 = g.c(0, sp, d.src_a0, i, d.src_row);
-    o1 = g.c(0, sp, d.src_a0 + 1, i, d.src_row);
+struct GhostCell {
+  double A, B, D, yD, sth, ysth, cths, ctht, m[8];
+  unsigned o0, o1;  // an instance that fits the memory has fewer than 2^31 elements a variable
+  int polar;
+};
+
+__device__ __forceinline__ GhostCell ghost_cell(const Inst &I, int q, bool vectors) {
+  const ADDR(1) double *t = glb(I.gt) + q;
+  const ADDR(1) int *ti = glb(I.gi) + q;
+  size_t n = I.ngd;
+  GhostCell c;
+  c.A = t[GT_A * n];
+  c.B = t[GT_B * n];
+  c.D = t[GT_D * n];
+  c.yD = t[GT_YD * n];
+  c.o0 = (unsigned)ti[GI_SRC0 * n];
+  c.o1 = (unsigned)ti[GI_SRC1 * n];
+  if (vectors) {
+    c.sth = t[GT_STH * n];
+    c.ysth = t[GT_YSTH * n];
+    c.cths = t[GT_CTH * n];
+    c.ctht = t[GT_CTHT * n];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) c.m[e] = t[(GT_MAP + e) * n];
+    c.polar = ti[GI_POLAR * n];
   }
+  return c;
+}
+
+__device__ __forceinline__ double ghost_scalar(const GhostCell &c, double v1, double v2) {
+  return div_rn(c.A * v1 + c.B * v2, c.D, c.yD);
 }
 
 // the covariant x2 / x3 components of a ghost cell from the two source cells
-__device__ __forceinline__ void ghost_vector(const GhostDesc &d, double v1y, double v1z, double v2y,
+__device__ __forceinline__ void ghost_vector(const GhostCell &c, double v1y, double v1z, double v2y,
                                              double v2z, double &vy, double &vz) {
-  vy = qdiv(d.A * v1y + d.B * v2y, d.D);
-  vz = qdiv(d.A * v1z + d.B * v2z, d.D);
-  double sth = d.sth_s, cth = d.cth_s;
-  double vyt = vy, vzt = vz;
-  vy = qdiv(qdiv(vyt, sth), sth) - qdiv(qdiv(vzt * cth, sth), sth);
-  vz = qdiv(qdiv(vzt, sth), sth) - qdiv(qdiv(vyt * cth, sth), sth);
-  double U, V;
-  vec_rll_from_abp(d.src_cy, d.src_cz, d.src_block, vy, vz, &U, &V);
-  vec_abp_from_rll(d.tgt_cy, d.tgt_cz, d.tgt_block, U, V, &vy, &vz);
-  cth = d.cth_t;
-  vyt = vy;
-  vzt = vz;
-  vy = vyt + vzt * cth;
-  vz = vzt + vyt * cth;
+  double y = ghost_scalar(c, v1y, v2y), z = ghost_scalar(c, v1z, v2z);
+  auto by2 = [&](double v) { return div_rn(div_rn(v, c.sth, c.ysth), c.sth, c.ysth); };
+  double cy = by2(y) - by2(z * c.cths), cz = by2(z) - by2(y * c.cths);
+  double ty, tz;
+  frame_map(c.m, c.polar, cy, cz, ty, tz);
+  vy = ty + tz * c.ctht;
+  vz = tz + ty * c.ctht;
 }
 
-__device__ __forceinline__ void ghost_body(const DGrid &g, int lb,
-                                           const ADDR(1) GhostDesc *__restrict__ gd, int ndesc,
-                                           ADDR(1) double *arr, int nvar, int vectors) {
-  int t = lb * BLK + threadIdx.x;
-  int ni = g.nx1;
-  if (t >= ndesc * ni) return;
-  int di = t / ni, i = g.is + t % ni;
-  GhostDesc d = *(const GhostDesc *)(gd + di);
-  size_t o0, o1;
-  ghost_source(g, d, i, o0, o1);
-  size_t ot = g.c(0, d.tgt_panel, d.tgt_k, i, d.tgt_j);
-  for (int n = 0; n < nvar; ++n) {
-    if (vectors && (n == IVY || n == IVZ || g.skipv(n))) continue;
-    double v1 = arr[n * g.vstride + o0], v2 = arr[n * g.vstride + o1];
-    arr[n * g.vstride + ot] = qdiv(d.A * v1 + d.B * v2, d.D);
+// where ghost cell (p, side, depth, a) or, depth < 0, the panel's cell -1 -
+// depth from that edge, lies
+__device__ __forceinline__ void edge_cell(const DGrid &g, int side, int depth, int a, int &k,
+                                          int &j) {
+  int lo = g.js - 1 - depth, hi = g.je + 1 + depth;  // js = ks, je = ke
+  k = side == 2 ? lo : side == 3 ? hi : g.ks + a;
+  j = side == 0 ? lo : side == 1 ? hi : g.js + a;
+}
+
+// Thread t of a walk over the rows across the panel edges: row q = (panel, side,
+// along a), level i; lanes walk the edge, as the exchanged states lie.
+__device__ __forceinline__ bool edge_thread(const DGrid &g, int nrow, int lb, int &q, int &p,
+                                            int &side, int &a, int &i) {
+  unsigned t = (unsigned)lb * BLK + threadIdx.x, N = g.N, ni = g.nx1;
+  if (t >= (unsigned)nrow * ni) return false;
+  unsigned r = t / N, ps = r / ni;
+  a = (int)(t - r * N);
+  i = g.is + (int)(r - ps * ni);
+  p = (int)(ps / 4);
+  side = (int)(ps % 4);
+  q = (int)(ps * N) + a;
+  return true;
+}
+
+// Ghost remap, a thread for each ghost cell and level.  It is bound by the lines
+// it touches: on the two sides whose rows lie along x2 a row's three ghosts are
+// 24 bytes of a line, and so are their sources.  There lanes walk the levels,
+// then the three depths (a line's users at one time); on the other two they walk
+// the edge, whole lines.  6 x 96 x 96 x 64: 41 us a stage, 44 with lanes along
+// the levels everywhere and the maps' square roots and quotients in the kernel;
+// three depths or four levels a thread 54 and 45 us (fewer wavefronts).
+__device__ __forceinline__ void ghost_body(const DGrid &g, int lb, const Inst &I,
+                                           ADDR(1) double *arr, int nvar, bool vectors) {
+  unsigned t = (unsigned)lb * BLK + threadIdx.x, N = g.N, ni = g.nx1;
+  if (t >= (unsigned)I.ngd * ni) return;
+  unsigned ps = t / (NG * N * ni), r = t - ps * (NG * N * ni);
+  int p = (int)(ps / 4), side = (int)(ps % 4);
+  unsigned f = side < 2 ? ni : N, q = r / f, lo = r - q * f, hi = q / NG;
+  int d = (int)(q - hi * NG), a = (int)(side < 2 ? hi : lo), i = g.is + (int)(side < 2 ? lo : hi);
+  GhostCell c = ghost_cell(I, (int)((ps * NG + d) * N) + a, vectors);
+  int k, j;
+  edge_cell(g, side, d, a, k, j);
+  size_t ot = g.c(0, p, k, i, j), up = (size_t)i * g.jp, o0 = c.o0 + up, o1 = c.o1 + up;
+  // every value is loaded before the first is stored (the compiler must take a
+  // store for one that a later load may read)
+  double v0[5], v1[5];
+#pragma unroll
+  for (int n = 0; n < 5; ++n) {
+    if (n >= nvar || (vectors && g.skipv(n))) continue;
+    v0[n] = arr[n * g.vstride + o0];
+    v1[n] = arr[n * g.vstride + o1];
+  }
+#pragma unroll
+  for (int n = 0; n < 5; ++n) {
+    if (n >= nvar || (vectors && (n == IVY || n == IVZ || g.skipv(n)))) continue;
+    arr[n * g.vstride + ot] = ghost_scalar(c, v0[n], v1[n]);
   }
   if (vectors) {
     double vy, vz;
-    ghost_vector(d, arr[IVY * g.vstride + o0], arr[IVZ * g.vstride + o0],
-                 arr[IVY * g.vstride + o1], arr[IVZ * g.vstride + o1], vy, vz);
+    ghost_vector(c, v0[IVY], v0[IVZ], v1[IVY], v1[IVZ], vy, vz);
     arr[IVY * g.vstride + ot] = vy;
     arr[IVZ * g.vstride + ot] = vz;
   }
@@ -484,8 +562,8 @@ __global__ void __launch_bounds__(BLK) k_ghost(const Inst *__restrict__ I_, Work
   WORK_LOOP(w) {
     WORK_INST(w);
     const Inst &I = I_[ii_];
-    if (which == 0) ghost_body(g, lb, glb(I.gd), I.ngd, st.u, g.nv, 1);
-    else ghost_body(g, lb, glb(I.gd), I.ngd, st.s, g.nt, 0);
+    if (which == 0) ghost_body(g, lb, I, st.u, g.nv, true);
+    else ghost_body(g, lb, I, st.s, g.nt, false);
   }
 }
 
@@ -646,59 +724,65 @@ k_flux_x1(const Inst *__restrict__ I_, Work w) {
 // 326-576): the interior-side WENO state of each edge face, its IVY / IVZ
 // mapped through lat-lon into the neighbour's frame, stored in the
 // neighbour's ghost-side slot [n][panel][side][a][i].
-__device__ __forceinline__ void edge_store(const DGrid &g, const DState &st, const EdgeDesc &d,
-                                           int i, double *q) {
-  double U, V, vx, vy;
-  vec_rll_from_abp(d.x2s, d.x3s, d.src_block, q[IVY], q[IVZ], &U, &V);
-  vec_abp_from_rll(d.x2d, d.x3d, d.tgt_block, U, V, &vx, &vy);
-  q[IVY] = vx;
-  q[IVZ] = vy;
-  int ni = g.nx1;
-  size_t base = (((size_t)d.tgt_panel * 4 + d.tgt_dir) * g.N + d.tgt_a) * ni + (i - g.is);
-  size_t vs = (size_t)6 * 4 * g.N * ni;
+// element of the exchanged state of edge face (panel, side, along a) at level
+// index ii in [0, nx1): [panel][side][level][along], [variable] outside
+__device__ __forceinline__ size_t edge_at(const DGrid &g, int p, int side, int a, int ii) {
+  return (((size_t)p * 4 + side) * g.nx1 + ii) * g.N + a;
+}
+__device__ __forceinline__ size_t edge_stride(const DGrid &g) { return (size_t)24 * g.N * g.nx1; }
+
+// moves the state q5 of edge face q into the neighbour's frame and slot
+template <typename R>
+__device__ __forceinline__ void edge_store(const DGrid &g, const Inst &I, int q, int i,
+                                           ADDR(1) R *edge, R *q5) {
+  const ADDR(1) double *t = glb(I.et) + q;
+  size_t n = I.ned;
+  double m[8];
 #pragma unroll
-  for (int n = 0; n < 5; ++n)
-    if (!g.skipv(n)) st.edge[n * vs + base] = q[n];
+  for (int e = 0; e < 8; ++e) m[e] = t[(ET_MAP + e) * n];
+  int slot = glb(I.ei)[EI_SLOT * n + q], polar = glb(I.ei)[EI_POLAR * n + q];
+  double vy, vz;
+  frame_map(m, polar, (double)q5[IVY], (double)q5[IVZ], vy, vz);
+  q5[IVY] = (R)vy;
+  q5[IVZ] = (R)vz;
+  int ps = slot >> 16;
+  size_t at = edge_at(g, ps >> 2, ps & 3, slot & 0xffff, i - g.is), vs = edge_stride(g);
+#pragma unroll
+  for (int v = 0; v < 5; ++v)
+    if (!g.skipv(v)) edge[v * vs + at] = q5[v];
 }
 
-__device__ __forceinline__ void edge_body(const DGrid &g, const DState &st, int lb,
-                                          const ADDR(1) EdgeDesc *__restrict__ ed, int nedge) {
-  int t = lb * BLK + threadIdx.x;
-  int ni = g.nx1;
-  if (t >= nedge * ni) return;
-  int e = t / ni, i = g.is + t % ni;
-  EdgeDesc d = *(const EdgeDesc *)(ed + e);
-  int p = d.src_panel, k = d.src_k, j = d.src_j;
+// the five cells of an edge face's interior-side value: two ghosts, then three
+// cells inwards; `step` elements apart from the first of these, element c
+__device__ __forceinline__ void edge_row(const DGrid &g, int p, int side, int a, int i, size_t &c,
+                                         ptrdiff_t &step) {
+  int k, j;
+  edge_cell(g, side, -1, a, k, j);
+  c = g.c(0, p, k, i, j);
+  step = side < 2 ? 1 : (ptrdiff_t)g.plane;
+  if (side & 1) step = -step;
+}
+
+__device__ __forceinline__ void edge_body(const DGrid &g, const DState &st, int lb, const Inst &I) {
+  int e, p, side, a, i;
+  if (!edge_thread(g, I.ned, lb, e, p, side, a, i)) return;
+  size_t c;
+  ptrdiff_t d;
+  edge_row(g, p, side, a, i, c, d);
   double q[5] = {0, 0, 0, 0, 0};
 #pragma unroll
   for (int n = 0; n < 5; ++n) {
     if (g.skipv(n)) continue;
-    double v;
-    if (d.src_dir == 0)  // R state of cell js at face js
-      v = weno5(st.w[g.c(n, p, k, i, j - 2)], st.w[g.c(n, p, k, i, j - 1)],
-                st.w[g.c(n, p, k, i, j)], st.w[g.c(n, p, k, i, j + 1)],
-                st.w[g.c(n, p, k, i, j + 2)]);
-    else if (d.src_dir == 1)  // L state of cell je at face je+1
-      v = weno5(st.w[g.c(n, p, k, i, j + 1)], st.w[g.c(n, p, k, i, j)],
-                st.w[g.c(n, p, k, i, j - 1)], st.w[g.c(n, p, k, i, j - 2)],
-                st.w[g.c(n, p, k, i, j - 3)]);
-    else if (d.src_dir == 2)
-      v = weno5(st.w[g.c(n, p, k - 2, i, j)], st.w[g.c(n, p, k - 1, i, j)],
-                st.w[g.c(n, p, k, i, j)], st.w[g.c(n, p, k + 1, i, j)],
-                st.w[g.c(n, p, k + 2, i, j)]);
-    else
-      v = weno5(st.w[g.c(n, p, k + 1, i, j)], st.w[g.c(n, p, k, i, j)],
-                st.w[g.c(n, p, k - 1, i, j)], st.w[g.c(n, p, k - 2, i, j)],
-                st.w[g.c(n, p, k - 3, i, j)]);
-    q[n] = v;
+    const ADDR(1) double *w = st.w + n * g.vstride + c;
+    q[n] = weno5(w[-2 * d], w[-d], w[0], w[d], w[2 * d]);
   }
-  edge_store(g, st, d, i, q);
+  edge_store(g, I, e, i, st.edge, q);
 }
 
 __global__ void __launch_bounds__(BLK) k_edge_states(const Inst *__restrict__ I_, Work w) {
   WORK_LOOP(w) {
     WORK_INST(w);
-    edge_body(g, st, lb, glb(I_[ii_].ed), I_[ii_].ned);
+    edge_body(g, st, lb, I_[ii_]);
   }
 }
 
@@ -736,9 +820,8 @@ __device__ __forceinline__ void face_flux64(const DGrid &g, const DState &st, in
   // side is the exchanged state; the values are selected, not the array they
   // go to, which keeps wl and wr in registers
   if (fa == 0 || fa == N) {
-    size_t vs = (size_t)6 * 4 * N * ni;
-    int side = (dir == 1 ? 0 : 2) + (fa == 0 ? 0 : 1);
-    size_t b = (((size_t)p * 4 + side) * N + kk) * ni + (i - g.is);
+    size_t vs = edge_stride(g);
+    size_t b = edge_at(g, p, (dir == 1 ? 0 : 2) + (fa == 0 ? 0 : 1), kk, i - g.is);
 #pragma unroll
     for (int n = 0; n < 5; ++n) {
       if (skip_of<E>(g, n)) continue;
@@ -1214,9 +1297,8 @@ __device__ __forceinline__ void face_flux_mix(const DGrid &g, const DState &st, 
   // panel edges (fa = 0: the L state, fa = N: the R state): the neighbour's
   // state, selected by value so wl and wr stay in registers
   if (fa == 0 || fa == N) {
-    size_t vs = (size_t)6 * 4 * N * ni;
-    int side = (dir == 1 ? 0 : 2) + (fa == 0 ? 0 : 1);
-    size_t b = (((size_t)p * 4 + side) * N + kk) * ni + (i - g.is);
+    size_t vs = edge_stride(g);
+    size_t b = edge_at(g, p, (dir == 1 ? 0 : 2) + (fa == 0 ? 0 : 1), kk, i - g.is);
 #pragma unroll
     for (int n = 0; n < 5; ++n) {
       float e = st.fedge[n * vs + b];
@@ -2126,7 +2208,7 @@ __global__ void __launch_bounds__(BLK) k_dt(const Inst *__restrict__ I_, Work w,
   if constexpr (EDGE)
     for (int h_ = (int)blockIdx.x - ngrid; h_ >= 0 && h_ < we.nblk; h_ += gridDim.x - ngrid) {
       WORK_INST(we);
-      edge_body(g, st, lb, glb(I_[ii_].ed), I_[ii_].ned);
+      edge_body(g, st, lb, I_[ii_]);
     }
 }
 
@@ -2427,55 +2509,27 @@ __global__ void __launch_bounds__(64 * W) k_flux_x1_mix(const Inst *__restrict__
 // mixed ideal gas: the interior-side WENO5 state of a panel-edge face, moved
 // into the neighbour's frame and slot
 __device__ __forceinline__ void edge_mix_body(const DGrid &g, const DState &st, int lb,
-                                              const ADDR(1) EdgeDesc *__restrict__ ed, int nedge) {
+                                              const Inst &I) {
 #pragma clang fp contract(fast)
-  int t = lb * BLK + threadIdx.x;
-  int ni = g.nx1;
-  if (t >= nedge * ni) return;
-  int e = t / ni, i = g.is + t % ni;
-  EdgeDesc d = *(const EdgeDesc *)(ed + e);
-  int p = d.src_panel, k = d.src_k, j = d.src_j;
+  int e, p, side, a, i;
+  if (!edge_thread(g, I.ned, lb, e, p, side, a, i)) return;
+  size_t c;
+  ptrdiff_t d;
+  edge_row(g, p, side, a, i, c, d);
   float q[5] = {0, 0, 0, 0, 0};
   // the FP32 perturbations k_prim wrote
-  auto FW = [&](int n, int kk, int ii, int jj) -> float { return st.fw[g.c(n, p, kk, ii, jj)]; };
 #pragma unroll
   for (int n = 0; n < 5; ++n) {
-    if (g.skipv(n)) continue;
-    float v;
-    if (d.src_dir == 0)
-      v = weno5f(FW(n, k, i, j - 2), FW(n, k, i, j - 1),
-                 FW(n, k, i, j), FW(n, k, i, j + 1),
-                 FW(n, k, i, j + 2));
-    else if (d.src_dir == 1)
-      v = weno5f(FW(n, k, i, j + 1), FW(n, k, i, j),
-                 FW(n, k, i, j - 1), FW(n, k, i, j - 2),
-                 FW(n, k, i, j - 3));
-    else if (d.src_dir == 2)
-      v = weno5f(FW(n, k - 2, i, j), FW(n, k - 1, i, j),
-                 FW(n, k, i, j), FW(n, k + 1, i, j),
-                 FW(n, k + 2, i, j));
-    else
-      v = weno5f(FW(n, k + 1, i, j), FW(n, k, i, j),
-                 FW(n, k - 1, i, j), FW(n, k - 2, i, j),
-                 FW(n, k - 3, i, j));
-    q[n] = v;
+    const ADDR(1) float *w = st.fw + n * g.vstride + c;
+    q[n] = weno5f(w[-2 * d], w[-d], w[0], w[d], w[2 * d]);
   }
-  double U, V, vx, vy;
-  vec_rll_from_abp(d.x2s, d.x3s, d.src_block, (double)q[IVY], (double)q[IVZ], &U, &V);
-  vec_abp_from_rll(d.x2d, d.x3d, d.tgt_block, U, V, &vx, &vy);
-  q[IVY] = (float)vx;
-  q[IVZ] = (float)vy;
-  size_t base = (((size_t)d.tgt_panel * 4 + d.tgt_dir) * g.N + d.tgt_a) * ni + (i - g.is);
-  size_t vs = (size_t)6 * 4 * g.N * ni;
-#pragma unroll
-  for (int n = 0; n < 5; ++n)
-    if (!g.skipv(n)) st.fedge[n * vs + base] = q[n];
+  edge_store(g, I, e, i, st.fedge, q);
 }
 
 __global__ void __launch_bounds__(BLK) k_edge_states_mix(const Inst *__restrict__ I_, Work w) {
   WORK_LOOP(w) {
     WORK_INST(w);
-    edge_mix_body(g, st, lb, glb(I_[ii_].ed), I_[ii_].ned);
+    edge_mix_body(g, st, lb, I_[ii_]);
   }
 }
 
@@ -2531,9 +2585,8 @@ __device__ __forceinline__ void face_flux_sw_mix(const DGrid &g, const DState &s
   }
   // panel edges: the neighbour's FP64 state, taken about B
   if (fa == 0 || fa == N) {
-    size_t vs = (size_t)6 * 4 * N * ni;
-    int side = (dir == 1 ? 0 : 2) + (fa == 0 ? 0 : 1);
-    size_t b = (((size_t)p * 4 + side) * N + kk) * ni + (i - g.is);
+    size_t vs = edge_stride(g);
+    size_t b = edge_at(g, p, (dir == 1 ? 0 : 2) + (fa == 0 ? 0 : 1), kk, i - g.is);
 #pragma unroll
     for (int n = 0; n < 5; ++n) {
       if (skip_of<EOS_SW>(g, n)) continue;
@@ -2707,8 +2760,8 @@ __device__ __forceinline__ void sw_face(const DGrid &g, const DState &st, const 
       if (fa != N) wr[n] = weno5(m2, m1, c0, p1, p2);
     }
     if (rim) {  // the ghost side is the neighbour's state (k_edge_states)
-      size_t vs = (size_t)6 * 4 * N * ni;
-      size_t b = (((size_t)p * 4 + (x3 ? 2 : 0) + (fa == 0 ? 0 : 1)) * N + kk) * ni + (i - g.is);
+      size_t vs = edge_stride(g);
+      size_t b = edge_at(g, p, (x3 ? 2 : 0) + (fa == 0 ? 0 : 1), kk, i - g.is);
       double e[3] = {st.edge[IDN * vs + b], st.edge[(x3 ? IVZ : IVY) * vs + b],
                      st.edge[(x3 ? IVY : IVZ) * vs + b]};
 #pragma unroll
@@ -2923,34 +2976,44 @@ k_sw_stage(const Inst *__restrict__ I_, Work w, StageW sw, int stage) {
 // with its CFL minimum (k_dt).
 __device__ __forceinline__ void sw_halo_body(const DGrid &g, const DState &st, int lb, const Inst &I,
                                              double dfloor, int stage) {
-  int t = lb * BLK + threadIdx.x;
-  int ni = g.nx1;
-  if (t >= I.ned * ni) return;
-  int e = t / ni, i = g.is + t % ni;
-  EdgeDesc d = *(const EdgeDesc *)(glb(I.ed) + e);
-  int p = d.src_panel, side = d.src_dir, a = side < 2 ? d.src_k - g.ks : d.src_j - g.js;
+  int e, p, side, a, i;
+  if (!edge_thread(g, I.ned, lb, e, p, side, a, i)) return;
   ADDR(1) double *arr = sw_out(st, stage);
   size_t vs = g.vstride;
-  // the cells of the row across the edge: ghosts q = 1 (depth 1), 0, -1, ..
-  auto place = [&](int depth, int &k, int &j) {
-    int lo = g.is - 1 - depth, hi = g.je + 1 + depth;  // is = js = ks, je = ke
-    k = side == 2 ? lo : side == 3 ? hi : g.ks + a;
-    j = side == 0 ? lo : side == 1 ? hi : g.js + a;
-  };
+  // every value is loaded before the first is stored (the compiler must take a
+  // store for one that a later load may read, and each would wait its turn)
+  GhostCell gc[NG];
+  double v0[NG][3], v1[NG][3], cg[NG], in[NG][3], ci[NG];
+#pragma unroll
+  for (int depth = 0; depth < NG; ++depth) {
+    gc[depth] = ghost_cell(I, ((p * 4 + side) * NG + depth) * g.N + a, true);
+    size_t o0 = (size_t)gc[depth].o0 + (size_t)i * g.jp;
+    size_t o1 = (size_t)gc[depth].o1 + (size_t)i * g.jp;
+    int k, j;
+    edge_cell(g, side, depth, a, k, j);
+    cg[depth] = g.T(T_COSC, p, k, j);
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+      v0[depth][v] = arr[sw_var(v) * vs + o0];
+      v1[depth][v] = arr[sw_var(v) * vs + o1];
+    }
+    if (stage < 2) {
+      edge_cell(g, side, -1 - depth, a, k, j);
+      ci[depth] = g.T(T_COSC, p, k, j);
+#pragma unroll
+      for (int v = 0; v < 3; ++v) in[depth][v] = arr[sw_var(v) * vs + g.c(0, p, k, i, j)];
+    }
+  }
   double s[3][5];  // the face's WENO5 cells: two ghosts, three cells
 #pragma unroll
   for (int depth = 0; depth < NG; ++depth) {
-    GhostDesc gd = *(const GhostDesc *)(glb(I.gd) + I.gx[((p * 4 + side) * g.N + a) * NG + depth]);
-    size_t o0, o1;
-    ghost_source(g, gd, i, o0, o1);
-    double h = qdiv(gd.A * arr[IDN * vs + o0] + gd.B * arr[IDN * vs + o1], gd.D), v2, v3;
-    ghost_vector(gd, arr[IVY * vs + o0], arr[IVZ * vs + o0], arr[IVY * vs + o1],
-                 arr[IVZ * vs + o1], v2, v3);
+    double h = ghost_scalar(gc[depth], v0[depth][0], v1[depth][0]), v2, v3;
+    ghost_vector(gc[depth], v0[depth][1], v0[depth][2], v1[depth][1], v1[depth][2], v2, v3);
     int k, j;
-    place(depth, k, j);
+    edge_cell(g, side, depth, a, k, j);
     size_t c = g.c(0, p, k, i, j);
     double w2, w3;
-    sw_prim(h, v2, v3, g.T(T_COSC, p, k, j), dfloor, w2, w3);
+    sw_prim(h, v2, v3, cg[depth], dfloor, w2, w3);
     arr[IDN * vs + c] = h;
     arr[IVY * vs + c] = v2;
     arr[IVZ * vs + c] = v3;
@@ -2967,18 +3030,15 @@ __device__ __forceinline__ void sw_halo_body(const DGrid &g, const DState &st, i
   if (stage == 2) return;
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    int k, j;
-    place(-1 - q, k, j);
-    size_t c = g.c(0, p, k, i, j);
-    double h = arr[IDN * vs + c], w2, w3;
-    sw_prim(h, arr[IVY * vs + c], arr[IVZ * vs + c], g.T(T_COSC, p, k, j), dfloor, w2, w3);
+    double h = in[q][0], w2, w3;
+    sw_prim(h, in[q][1], in[q][2], ci[q], dfloor, w2, w3);
     s[0][2 + q] = h;
     s[1][2 + q] = w2;
     s[2][2 + q] = w3;
   }
   double q[5] = {0., 0., 0., 0., 0.};
   for (int v = 0; v < 3; ++v) q[sw_var(v)] = weno5(s[v][0], s[v][1], s[v][2], s[v][3], s[v][4]);
-  edge_store(g, st, d, i, q);
+  edge_store(g, I, e, i, st.edge, q);
 }
 
 __global__ void __launch_bounds__(BLK) k_sw_halo(const Inst *__restrict__ I_, Work w, double dfloor,
@@ -3217,9 +3277,8 @@ struct exo_handle {
   hipStream_t stream = nullptr; // == L.stream
   std::string err;
   std::vector<void *> allocs;
-  GhostDesc *d_ghost = nullptr;
-  EdgeDesc *d_edge = nullptr;
-  int *d_gx = nullptr;          // Inst::gx
+  double *d_gt = nullptr, *d_et = nullptr;  // remap tables (Inst)
+  int *d_gi = nullptr, *d_ei = nullptr;
   double *d_x1 = nullptr, *d_tab = nullptr;
   double *d_sums = nullptr;     // [5] totals of exo_conserved_sums
   double *d_stage = nullptr;    // stage_doubles(g): pieces of host transfers
@@ -3350,9 +3409,10 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
     const exo_handle *h = hs[i];
     inst[i].g = h->g;
     inst[i].st = h->st;
-    inst[i].gd = h->d_ghost;
-    inst[i].ed = h->d_edge;
-    inst[i].gx = h->d_gx;
+    inst[i].gt = h->d_gt;
+    inst[i].gi = h->d_gi;
+    inst[i].et = h->d_et;
+    inst[i].ei = h->d_ei;
     inst[i].ngd = (int)h->setup.ghosts.size();
     inst[i].ned = (int)h->setup.edges.size();
     L.lds_x1 = std::max(L.lds_x1, (size_t)(h->g.nc1 + 1) * 64 * sizeof(double));
@@ -3479,9 +3539,10 @@ size_t footprint_bytes(const Setup &s) {
   size_t edge = (size_t)6 * 4 * g.N * g.nx1;
   add(3 * (s.nc1 + 1) * sizeof(double));
   add((s.tab2.size() + s.tab1.size()) * sizeof(double));
-  add(s.ghosts.size() * sizeof(GhostDesc));
-  add(s.edges.size() * sizeof(EdgeDesc));
-  if (sw_fused(g)) add(s.ghosts.size() * sizeof(int));
+  add(s.ghosts.size() * GT_N * sizeof(double));
+  add(s.ghosts.size() * GI_N * sizeof(int));
+  add(s.edges.size() * ET_N * sizeof(double));
+  add(s.edges.size() * EI_N * sizeof(int));
   for (int q = 0; q < 4; ++q) add(cell * g.nv);           // u, w, u1, du
   if (g.nt)
     for (int q = 0; q < 3; ++q) add(cell * g.nt);         // s, r, s1
@@ -3515,6 +3576,83 @@ size_t footprint_bytes(const Setup &s) {
   return tot;
 }
 
+// The constants of frame_map: from the frame of block bs at tangents (x, y) to
+// east and north (vec_rll_from_abp), and from these to block bt's frame at (X,
+// Y) (vec_abp_from_rll).  Returns the polar bits.
+int map_factors(double x, double y, int bs, double X, double Y, int bt, double *m) {
+  double C = std::sqrt(1 + x * x), D = std::sqrt(1 + y * y);
+  double E = std::sqrt(x * x + y * y), delta = std::sqrt(1 + x * x + y * y);
+  bool ps = bs == 1 || bs == 5, pt = bt == 1 || bt == 5;
+  if (!ps) {
+    m[0] = 0.;
+    m[1] = delta / (C * D);
+    m[2] = -1.;
+    m[3] = x * y / (C * D);
+  } else {
+    double sg = bs == 1 ? -1. : 1.;
+    m[0] = sg * (delta * y / (D * E));
+    m[1] = -sg * (delta * x / (C * E));
+    m[2] = sg * (x / (D * E));
+    m[3] = sg * (y / (C * E));
+  }
+  C = std::sqrt(1 + X * X);
+  D = std::sqrt(1 + Y * Y);
+  E = std::sqrt(X * X + Y * Y);
+  delta = std::sqrt(1 + X * X + Y * Y);
+  if (!pt) {
+    m[4] = X * Y / delta;
+    m[5] = -1.;
+    m[6] = C * D / delta;
+    m[7] = 0.;
+  } else {
+    double sg = bt == 1 ? -1. : 1.;
+    m[4] = sg * (D * Y / (delta * E));
+    m[5] = sg * (D * X / E);
+    m[6] = -sg * (C * X / (delta * E));
+    m[7] = sg * (C * Y / E);
+  }
+  return (ps ? 1 : 0) | (pt ? 2 : 0);
+}
+
+struct RemapTables {
+  std::vector<double> gt, et;
+  std::vector<int> gi, ei;
+};
+
+RemapTables remap_tables(const Setup &s, const Grid &g) {
+  RemapTables r;
+  size_t ng = s.ghosts.size(), ne = s.edges.size();
+  r.gt.assign(GT_N * ng, 0.);
+  r.gi.assign(GI_N * ng, 0);
+  r.et.assign(ET_N * ne, 0.);
+  r.ei.assign(EI_N * ne, 0);
+  double m[8];
+  for (const GhostDesc &d : s.ghosts) {
+    bool x2 = d.tgt_j < g.js || d.tgt_j > g.je;
+    int at = x2 ? d.tgt_j : d.tgt_k, along = x2 ? d.tgt_k - g.ks : d.tgt_j - g.js;
+    int lo = x2 ? g.js : g.ks, hi = x2 ? g.je : g.ke;
+    int side = (x2 ? 0 : 2) + (at > hi ? 1 : 0), depth = at > hi ? at - hi - 1 : lo - 1 - at;
+    size_t q = ((size_t)(d.tgt_panel * 4 + side) * NG + depth) * g.N + along;
+    const double v[8] = {d.A, d.B, d.D, 1.0 / d.D, d.sth_s, 1.0 / d.sth_s, d.cth_s, d.cth_t};
+    for (int e = 0; e < 8; ++e) r.gt[(GT_A + e) * ng + q] = v[e];
+    r.gi[GI_POLAR * ng + q] =
+        map_factors(d.src_cy, d.src_cz, d.src_block, d.tgt_cy, d.tgt_cz, d.tgt_block, m);
+    for (int e = 0; e < 8; ++e) r.gt[(GT_MAP + e) * ng + q] = m[e];
+    int k0 = d.along_x2 ? d.src_row : d.src_a0, j0 = d.along_x2 ? d.src_a0 : d.src_row;
+    size_t o0 = g.c(0, d.src_panel, k0, 0, j0);
+    r.gi[GI_SRC0 * ng + q] = (int)o0;
+    r.gi[GI_SRC1 * ng + q] = (int)(o0 + (d.along_x2 ? 1 : g.plane));
+  }
+  for (const EdgeDesc &d : s.edges) {
+    int a = d.src_dir < 2 ? d.src_k - g.ks : d.src_j - g.js;
+    size_t q = (size_t)(d.src_panel * 4 + d.src_dir) * g.N + a;
+    r.ei[EI_POLAR * ne + q] = map_factors(d.x2s, d.x3s, d.src_block, d.x2d, d.x3d, d.tgt_block, m);
+    for (int e = 0; e < 8; ++e) r.et[(ET_MAP + e) * ne + q] = m[e];
+    r.ei[EI_SLOT * ne + q] = (d.tgt_panel * 4 + d.tgt_dir) << 16 | d.tgt_a;
+  }
+  return r;
+}
+
 void init_handle(exo_handle *h) {
   Setup &s = h->setup;
   Grid &g = h->g;
@@ -3541,27 +3679,16 @@ void init_handle(exo_handle *h) {
                         hipMemcpyHostToDevice, h->stream));
   g.tab = h->d_tab;
   g.tab1 = h->d_tab + s.tab2.size();
-  h->d_ghost = (GhostDesc *)h->dalloc(s.ghosts.size() * sizeof(GhostDesc));
-  HIPCHK(hipMemcpyAsync(h->d_ghost, s.ghosts.data(), s.ghosts.size() * sizeof(GhostDesc),
-                        hipMemcpyHostToDevice, h->stream));
-  h->d_edge = (EdgeDesc *)h->dalloc(s.edges.size() * sizeof(EdgeDesc));
-  HIPCHK(hipMemcpyAsync(h->d_edge, s.edges.data(), s.edges.size() * sizeof(EdgeDesc),
-                        hipMemcpyHostToDevice, h->stream));
-  std::vector<int> gx;
-  if (sw_fused(g)) {
-    gx.assign(s.ghosts.size(), 0);
-    for (size_t q = 0; q < s.ghosts.size(); ++q) {
-      const GhostDesc &d = s.ghosts[q];
-      bool x2 = d.tgt_j < g.js || d.tgt_j > g.je;
-      int at = x2 ? d.tgt_j : d.tgt_k, along = x2 ? d.tgt_k - g.ks : d.tgt_j - g.js;
-      int lo = x2 ? g.js : g.ks, hi = x2 ? g.je : g.ke;
-      int side = (x2 ? 0 : 2) + (at > hi ? 1 : 0), depth = at > hi ? at - hi - 1 : lo - 1 - at;
-      gx[((size_t)(d.tgt_panel * 4 + side) * g.N + along) * NG + depth] = (int)q;
-    }
-    h->d_gx = (int *)h->dalloc(gx.size() * sizeof(int));
-    HIPCHK(hipMemcpyAsync(h->d_gx, gx.data(), gx.size() * sizeof(int), hipMemcpyHostToDevice,
-                          h->stream));
-  }
+  const RemapTables rt = remap_tables(s, g);
+  auto table = [&](auto &d, const auto &v) {
+    using T = std::remove_pointer_t<std::remove_reference_t<decltype(d)>>;
+    d = (T *)h->dalloc(v.size() * sizeof(T));
+    HIPCHK(hipMemcpyAsync(d, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, h->stream));
+  };
+  table(h->d_gt, rt.gt);
+  table(h->d_gi, rt.gi);
+  table(h->d_et, rt.et);
+  table(h->d_ei, rt.ei);
   // state
   State &st = h->st;
   std::memset(&st, 0, sizeof(st));
