@@ -573,10 +573,10 @@ __global__ void __launch_bounds__(BLK) k_ghost(const Inst *__restrict__ I_, Work
 // (change_to_perturbation.cpp:39-190) around Weno5X1, then the x1 Riemann
 // solve (patches/19.calculate_fluxes.patch:77-106).  The face pressure psf
 // lives in LDS, [face][lane].
-// The block holds 64 columns and X1W waves: wave 0 integrates the face
-// pressure of every column into LDS, then each wave takes a contiguous share
-// of the faces with its own WENO window, so a column's faces are worked on by
-// X1W lanes at once.  Per-face arithmetic is independent of the split.
+// The mixed form's block holds 64 columns and X1W waves: wave 0 integrates the
+// face pressure of every column into LDS, then each wave takes a contiguous
+// share of the faces with its own WENO window, so a column's faces are worked on
+// by X1W lanes at once.  Per-face arithmetic is independent of the split.
 constexpr int X1W = 4;  // the default; the autotuner may pick 2 or 8 (x1_waves)
 
 __device__ __forceinline__ void psf_scan(const DGrid &g, const DState &st, int p, int k, int j,
@@ -605,60 +605,111 @@ __device__ __forceinline__ void psf_scan(const DGrid &g, const DState &st, int p
 #undef PSF
 }
 
-template <int W, int RK = -1>
+// The FP64 sweep.  A block holds C columns; its threads are numbered level by
+// level, C columns to a level, so a wave works on 64 / C neighbouring levels of
+// the columns at once.  Density and pressure go into LDS first: the downward sum
+// of the face pressure is then one add a level, every cell is decomposed once
+// (two logarithms and an exponential) by whichever wave it falls to, and a face
+// reads its six cells by itself.  A window of six cells sliding up a column, 64
+// columns and four shares of the levels to a block, decomposed up to half of the
+// cells twice, waited for memory in the sum, and held 166 VGPRs: three waves a
+// SIMD, 864 blocks of 6 x 96 x 96 columns on 768 places.  Now four waves (127
+// VGPRs).  Bound by FP64 issue: 1390 VALU instructions a face, 0.13 of the
+// 0.19 ms.  Measured, window -> this: 6 x 96 x 96 x 64 234 -> 194 us, 6 x 64 x
+// 64 x 47 98 -> 67, 6 x 26 x 26 x 19 with a tracer 38 -> 14.  (Three or five
+// waves a SIMD, 32 columns, eight waves a block: 197 to 217 us.)
+// doubles of LDS: psf of nc1 + 1 faces, the perturbations of density and
+// pressure of nc1 cells, and e1, a column
+size_t x1_lds(int nc1, int C) { return ((size_t)3 * nc1 + 2) * C; }
+// A launch that has fewer than X1C_CU blocks of X1C columns a CU leaves places
+// empty, and blocks of half as many columns fill them and take half the time
+// each; above, they read half a line of every row: 16 -> 8 columns, 6 x 32 x 32 x
+// 48 31 -> 26 us, 6 x 48 x 48 x 48 (3.4 blocks a CU) 51.6 -> 51.9, 6 x 64 x 64 x
+// 64 (6 a CU) 98 -> 107.
+constexpr int X1C = 16, X1C_FEW = 8, X1C_CU = 4;
+
+template <int W, int RK, int C>
 __device__ __forceinline__ void flux_x1_body(const DGrid &g, const DState &st, int lb, double *lds) {
-  int lane = threadIdx.x & 63, seg = threadIdx.x >> 6;
-  int N = g.N;
-  int nbx = (N * N + 63) / 64;
-  int col = (lb % nbx) * 64 + lane;
+  constexpr int SLOTS = 64 * W / C;  // levels in work at a time
+  int c = threadIdx.x % C, slot = threadIdx.x / C;
+  int N = g.N, nc1 = g.nc1;
+  int nbx = (N * N + C - 1) / C;
+  int col = (lb % nbx) * C + c;
   int p = lb / nbx;
   bool act = col < N * N;
   int k = g.ks + (act ? col / N : 0), j = g.js + (act ? col % N : 0);
-  double *psf = lds;  // (nc1 + 1) x 64
-#define PSF(ii) psf[(ii) * 64 + lane]
-  int is = g.is, ie = g.ie, nv = g.nv;
+  double *psf = lds + c;
+  double *rho = psf + (nc1 + 1) * C, *prs = rho + nc1 * C, *le1 = prs + nc1 * C;
+  int is = g.is, ie = g.ie;
   bool decomp = g.grav != 0.;
-  double e1 = 1., ig = 1.;
-  if (seg == 0 && act && decomp) psf_scan(g, st, p, k, j, psf, lane);
-  __syncthreads();
-  if (!act) return;
-  if (decomp) {
-    double ent0 = g.gamma;
-    double ent1 = dlog(st.w[g.c(IPR, p, k, is, j)]) - ent0 * dlog(st.w[g.c(IDN, p, k, is, j)]);
-    ig = qdiv(1., ent0);
-    e1 = dexp(qdiv(-ent1, ent0));
-  }
-  // this wave's faces [f0, f1)
-  int nf = ie + 2 - is;
-  int f0 = is + (nf * seg) / W, f1 = is + (nf * (seg + 1)) / W;
-  // window of 6 cells (f-3 .. f+2) for face f, perturbed IDN / IPR
-  double q[6][5];
-  auto load = [&](int slot, int i) {
-#pragma unroll
-    for (int n = 0; n < 5; ++n) q[slot][n] = n < nv ? st.w[g.c(n, p, k, i, j)] : 0.;
-    if (decomp) {
-      double a = PSF(i), b = PSF(i + 1), psv;
-      if (fabs(a - b) < 1.E-6) psv = (a + b) / 2.;
-      else psv = qdiv(a - b, dlog(qdiv(a, b)));
-      double dsv = dpow(psv, ig) * e1;
-      q[slot][IPR] -= psv;
-      q[slot][IDN] -= dsv;
+  double grav = -g.grav;
+  const ADDR(1) double *w = st.w + g.c(0, p, k, 0, j);
+  size_t vs = g.vstride;
+  unsigned jp = g.jp;
+  if (act)
+    for (int i = slot; i < nc1; i += SLOTS) {
+      double d = w[IDN * vs + i * jp];
+      rho[i * C] = d;
+      prs[i * C] = w[IPR * vs + i * jp];
+      // the terms of the downward sum
+      if (decomp && i >= is && i <= ie) psf[i * C] = grav * d * g.dx1f[i];
     }
-  };
-#pragma unroll
-  for (int s = 0; s < 6; ++s) load(s, f0 - 3 + s);
+  __syncthreads();
+  double ig = 1., e1 = 1.;
+  if (decomp) {
+    ig = qdiv(1., g.gamma);
+    if (act && slot == 0) {
+      double acc = prs[ie * C] *
+                   dexp(qdiv(-grav * g.dx1f[ie], 2 * qdiv(prs[ie * C], rho[ie * C])));
+      psf[(ie + 1) * C] = acc;
+#pragma unroll 8
+      for (int i = ie; i >= is; --i) {
+        acc = acc + psf[i * C];
+        psf[i * C] = acc;
+      }
+      for (int q = 1; q <= NG; ++q) psf[(is - q) * C] = psf[(is + q) * C];
+      for (int q = 1; q <= NG; ++q) psf[(ie + q + 1) * C] = psf[(ie + 1 - q) * C];
+    } else if (act && slot == 64 / C) {  // meanwhile, in the second wave
+      double ent0 = g.gamma;
+      double ent1 = dlog(prs[is * C]) - ent0 * dlog(rho[is * C]);
+      *le1 = dexp(qdiv(-ent1, ent0));
+    }
+    __syncthreads();
+    e1 = *le1;
+    if (act)
+      for (int i = slot; i < nc1; i += SLOTS) {
+        double a = psf[i * C], b = psf[(i + 1) * C], psv;
+        if (fabs(a - b) < 1.E-6) psv = (a + b) / 2.;
+        else psv = qdiv(a - b, dlog(qdiv(a, b)));
+        double dsv = dpow(psv, ig) * e1;
+        prs[i * C] -= psv;
+        rho[i * C] -= dsv;
+      }
+    __syncthreads();
+  }
+  if (!act) return;
   double cth = g.T(T_CTH1, p, k, j), cosc = g.T(T_COSC, p, k, j);
-  for (int fi = f0; fi < f1; ++fi) {
+  unsigned fjp = g.jp;
+  size_t fbase = g.f(0, p, k, 0, j), fvs = g.fvstride;
+  for (int fi = is + slot; fi <= ie + 1; fi += SLOTS) {
     double wl[5], wr[5], fl[5];
 #pragma unroll
     for (int n = 0; n < 5; ++n) {
-      if (n < nv) {
-        wl[n] = weno5(q[4][n], q[3][n], q[2][n], q[1][n], q[0][n]);
-        wr[n] = weno5(q[1][n], q[2][n], q[3][n], q[4][n], q[5][n]);
+      double q[6];
+      if (n == IDN || n == IPR) {
+        const double *a = (n == IDN ? rho : prs) + (fi - 3) * C;
+#pragma unroll
+        for (int s = 0; s < 6; ++s) q[s] = a[s * C];
+      } else {
+        const ADDR(1) double *a = w + n * vs + (fi - 3) * jp;
+#pragma unroll
+        for (int s = 0; s < 6; ++s) q[s] = a[s * jp];
       }
+      wl[n] = weno5(q[4], q[3], q[2], q[1], q[0]);
+      wr[n] = weno5(q[1], q[2], q[3], q[4], q[5]);
     }
     if (decomp) {
-      double pf = PSF(fi);
+      double pf = psf[fi * C];
       wr[IPR] += pf;
       if (wr[IPR] < 0.) wr[IPR] = pf;
       wl[IPR] += pf;
@@ -670,52 +721,43 @@ __device__ __forceinline__ void flux_x1_body(const DGrid &g, const DState &st, i
       if (wl[IDN] < 0.) wl[IDN] = dsf;
     }
     riemann<double>(EOS_IDEAL, rs_of<RK>(g), IVX, g.gamma, wl, wr, fl, cth, 0., 1., cosc);
+    size_t f = fbase + fi * fjp;
 #pragma unroll
-    for (int n = 0; n < 5; ++n)
-      if (n < nv) st.flx[0][g.f(n, p, k, fi, j)] = fl[n];
-    if (fi + 1 < f1) {
+    for (int n = 0; n < 5; ++n) st.flx[0][f + n * fvs] = fl[n];
+    // passive scalars: WENO of r along x1, upwinded by the mass flux
+    for (int n = 0; n < g.nt; ++n) {
+      const ADDR(1) double *r = st.r + g.c(n, p, k, fi - 3, j);
+      double q[6];
 #pragma unroll
-      for (int s = 0; s < 5; ++s)
-#pragma unroll
-        for (int n = 0; n < 5; ++n) q[s][n] = q[s + 1][n];
-      load(5, fi + 3);
+      for (int s = 0; s < 6; ++s) q[s] = r[s * jp];
+      double m = fl[IDN];
+      double rl = weno5(q[4], q[3], q[2], q[1], q[0]);
+      double rr = weno5(q[1], q[2], q[3], q[4], q[5]);
+      st.sflx[0][f + n * fvs] = m >= 0.0 ? m * rl : m * rr;
     }
   }
-  // passive scalars: WENO of r along x1, upwinded by the mass flux; a window
-  // of 6 levels (fi - 3 .. fi + 2) slides up the column, the next level and
-  // mass flux loaded before the face's arithmetic
-  for (int n = 0; n < g.nt; ++n) {
-    double r[6];
-#pragma unroll
-    for (int s = 0; s < 6; ++s) r[s] = st.r[g.c(n, p, k, f0 - 3 + s, j)];
-    double m = f0 < f1 ? st.flx[0][g.f(IDN, p, k, f0, j)] : 0.;
-    for (int fi = f0; fi < f1; ++fi) {
-      bool more = fi + 1 < f1;
-      double rn = more ? st.r[g.c(n, p, k, fi + 3, j)] : 0.;
-      double mn = more ? st.flx[0][g.f(IDN, p, k, fi + 1, j)] : 0.;
-      double rl = weno5(r[4], r[3], r[2], r[1], r[0]);
-      double rr = weno5(r[1], r[2], r[3], r[4], r[5]);
-      st.sflx[0][g.f(n, p, k, fi, j)] = m >= 0.0 ? m * rl : m * rr;
-#pragma unroll
-      for (int s = 0; s < 5; ++s) r[s] = r[s + 1];
-      r[5] = rn;
-      m = mn;
-    }
-  }
-#undef PSF
 }
 
-// three wavefronts per SIMD (168 VGPRs, no spills): with 4 wavefronts per
-// 64-column block the LDS of the face pressures allows four blocks per CU, and
-// the sweep is 6 % faster than at the compiler's two wavefronts per SIMD
 template <int W, int RK = -1>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4)))
 k_flux_x1(const Inst *__restrict__ I_, Work w) {
   extern __shared__ double lds[];
   WORK_LOOP(w) {
     WORK_INST(w);
-    flux_x1_body<W, RK>(g, st, lb, lds);
-    __syncthreads();  // psf is rebuilt by the next block of the loop
+    flux_x1_body<W, RK, X1C>(g, st, lb, lds);
+    __syncthreads();  // the next block of the loop fills the LDS again
+  }
+}
+
+// the same for a launch of few columns
+template <int W, int RK = -1>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4)))
+k_flux_x1_few(const Inst *__restrict__ I_, Work w) {
+  extern __shared__ double lds[];
+  WORK_LOOP(w) {
+    WORK_INST(w);
+    flux_x1_body<W, RK, X1C_FEW>(g, st, lb, lds);
+    __syncthreads();  // the next block of the loop fills the LDS again
   }
 }
 
@@ -3251,7 +3293,10 @@ struct Launcher {
   int rs = -1;              // Riemann solver of every instance (-1: they differ)
   int ncu = 0;              // CUs of the device
   std::vector<Inst> h_inst;     // host copies of the instances (the tuner reads them)
-  size_t lds_x1 = 0;        // dynamic LDS of the x1 kernels (largest instance)
+  // dynamic LDS of the x1 kernels (largest instance): the mixed form's face
+  // pressures of 64 columns, which the size limit is stated for, and x1_lds
+  size_t lds_x1 = 0, lds_x1_fp64 = 0;
+  int x1c = X1C;            // columns of a block of the FP64 x1 sweep
   // live per-kernel timing with HIP events on the stream
   bool prof = false;
   std::vector<hipEvent_t> ev_pool;
@@ -3333,7 +3378,7 @@ hipEvent_t next_event(Launcher &L) {
 bool sw_fused(const Grid &g) { return g.eos == EOS_SW && g.nt == 0; }
 
 // step: the work list of a whole step (Launcher::mode 1)
-int kind_blocks(int kind, const Grid &g, bool mixed, int ngd, int ned, bool step) {
+int kind_blocks(int kind, const Grid &g, bool mixed, int ngd, int ned, bool step, int x1c) {
   bool ideal = g.eos == EOS_IDEAL;
   bool sw = step && sw_fused(g);
   int tiles = ((g.N + SWTJ - 1) / SWTJ) * ((g.N + SWTK - 1) / SWTK);
@@ -3355,7 +3400,7 @@ int kind_blocks(int kind, const Grid &g, bool mixed, int ngd, int ned, bool step
     case K_PRIM_GHOST: return !ideal ? (int)grid1((size_t)6 * 4 * NG * g.N * g.nx1) : 0;
     case K_GHOST_U: return (int)grid1((size_t)ngd * g.nx1);
     case K_GHOST_S: return g.nt ? (int)grid1((size_t)ngd * g.nx1) : 0;
-    case K_X1: return ideal && !mixed ? (int)grid1(cols, 64) * 6 : 0;
+    case K_X1: return ideal && !mixed ? (int)grid1(cols, x1c) * 6 : 0;
     case K_X1_MIX: return ideal && mixed ? (int)grid1(cols, 64) * 6 : 0;
     // mixed shallow water takes FP64 edge states (its faces are taken about an
     // FP64 base state)
@@ -3404,7 +3449,9 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
   L.ninst = n;
   std::vector<Inst> inst(n);
   std::vector<int> tab((size_t)2 * K_NKIND * (n + 1));
-  L.lds_x1 = 0;
+  L.lds_x1 = L.lds_x1_fp64 = 0;
+  int dev = 0;
+  size_t cols = 0;  // of the FP64 x1 sweep
   for (int i = 0; i < n; ++i) {
     const exo_handle *h = hs[i];
     inst[i].g = h->g;
@@ -3416,7 +3463,13 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
     inst[i].ngd = (int)h->setup.ghosts.size();
     inst[i].ned = (int)h->setup.edges.size();
     L.lds_x1 = std::max(L.lds_x1, (size_t)(h->g.nc1 + 1) * 64 * sizeof(double));
+    if (!h->mixed) cols += (size_t)6 * h->g.N * h->g.N;
   }
+  HIPCHK(hipGetDevice(&dev));
+  HIPCHK(hipDeviceGetAttribute(&L.ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  L.x1c = cols < (size_t)X1C * X1C_CU * L.ncu ? X1C_FEW : X1C;
+  for (const exo_handle *h : hs)
+    L.lds_x1_fp64 = std::max(L.lds_x1_fp64, x1_lds(h->g.nc1, L.x1c) * sizeof(double));
   L.eos = n > 0 ? hs[0]->g.eos : -1;
   L.rs = n > 0 ? hs[0]->g.rs : -1;
   for (int i = 1; i < n; ++i) {
@@ -3430,16 +3483,14 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
       long long acc = 0;
       for (int i = 0; i < n; ++i) {
         t[i] = (int)acc;
-        acc += kind_blocks(kind, hs[i]->g, hs[i]->mixed, inst[i].ngd, inst[i].ned, m == 1);
+        acc += kind_blocks(kind, hs[i]->g, hs[i]->mixed, inst[i].ngd, inst[i].ned, m == 1, L.x1c);
       }
       if (acc > 0x7fffffffLL) throw std::string("work list too large for one launch");
       t[n] = (int)acc;
       L.nblk[m][kind] = (int)acc;
     }
   {
-    int dev = 0, maxlds = 0;
-    HIPCHK(hipGetDevice(&dev));
-    HIPCHK(hipDeviceGetAttribute(&L.ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    int maxlds = 0;
     HIPCHK(hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     bool need_x1 = L.nblk[0][K_X1] > 0 || L.nblk[0][K_X1_MIX] > 0;
     for (const exo_handle *h : hs)
@@ -3782,7 +3833,8 @@ void launch_x1_w(Launcher &L, int kind, int kid) {
     with_solver<EOS_IDEAL>(L, [&](auto R) {
       launch(L, kind, kid, k_flux_x1_mix<W, decltype(R)::value>, 64 * W, L.lds_x1);
     });
-  else launch(L, kind, kid, k_flux_x1<W>, 64 * W, L.lds_x1);
+  else if (L.x1c == X1C) launch(L, kind, kid, k_flux_x1<W>, 64 * W, L.lds_x1_fp64);
+  else launch(L, kind, kid, k_flux_x1_few<W>, 64 * W, L.lds_x1_fp64);
 }
 
 void launch_x1(Launcher &L, int kind, int kid) {
