@@ -1499,9 +1499,6 @@ __device__ __forceinline__ M5 jac_e(double gm1, const double *w, double e) {
 
 constexpr int IMPL_MAXNC1 = 512;  // radial cells incl. ghosts the column solve supports
 
-// geo: LDS for the instance's x1f | x1v | dx1f, so the per-level geometry is
-// read without waiting on the vector-memory counter (which also counts the
-// coefficient stores and the prefetches in flight)
 // AVG (within a stage): the update kernel formed only the tendency, and the
 // stage's weighted average of u (with the stage register u1) is formed here,
 // as update_cell forms it, before u += delta: u is read and written once per
@@ -1513,50 +1510,65 @@ typedef double dpair __attribute__((ext_vector_type(2)));
 // the x1 face areas and volume of each level, and the end of the backward
 // substitution: u (or, with AVG, the stage's weighted average of u and u1)
 // plus the correction.
-template <bool AVG>
+template <bool AVG, typename GP>
 struct ColIOGrid {
   const ADDR(1) double *__restrict__ W;
   const ADDR(1) double *__restrict__ DU;
   ADDR(1) double *__restrict__ U;
   ADDR(1) double *__restrict__ U1;
-  size_t vs, jp, c0;
+  size_t vs, jp;
+  unsigned off;  // bytes from the panel's element (variable 0, level 0) to the column
   double cth, sth, a23, dx2a, dx3a;
-  const double *x1f, *x1v, *dx1f;
+  GP x1f, x1v, dx1f;  // in LDS or in global memory
   StageW sw;
-  bool first;
+  bool first, act;
+  // the lane's element of variable n, level i: a base that is the same for the
+  // block and the lane's 32-bit offset, so the lanes hold no addresses
+  template <typename T>
+  __device__ __forceinline__ ADDR(1) T *at(ADDR(1) T *a, int n, int i) const {
+    return (ADDR(1) T *)((ADDR(1) const char *)(a + (n * vs + (size_t)i * jp)) + off);
+  }
   __device__ __forceinline__ void wraw(int i, double *w) const {
 #pragma unroll
-    for (int n = 0; n < 5; ++n) w[n] = W[n * vs + c0 + (size_t)i * jp];
+    for (int n = 0; n < 5; ++n) w[n] = *at(W, n, i);
   }
   __device__ __forceinline__ void project(double *w) const {
     w[IVY] += w[IVZ] * cth;
     w[IVZ] *= sth;
   }
   __device__ __forceinline__ double du(int i, int n) const {
-    return DU[n * vs + c0 + (size_t)i * jp];
+    return *at(DU, n, i);
+  }
+  // what geom takes of level i, loaded ahead
+  __device__ __forceinline__ void graw(int i, double *r) const {
+    r[0] = x1f[i];
+    r[1] = x1f[i + 1];
+    r[2] = x1v[i];
+    r[3] = dx1f[i];
   }
   // Grid::area1 = ((DX2A DX3A) x1f) x1f SINC and Grid::volume =
   // ((((dx1f DX2A) DX3A) x1v) x1v) SINC with the same roundings
-  __device__ __forceinline__ void geom(int i, double &aleft, double &aright, double &v) const {
-    aleft = ((a23 * x1f[i]) * x1f[i]) * sth;
-    aright = ((a23 * x1f[i + 1]) * x1f[i + 1]) * sth;
-    v = ((((dx1f[i] * dx2a) * dx3a) * x1v[i]) * x1v[i]) * sth;
+  __device__ __forceinline__ void geom(const double *r, double &aleft, double &aright,
+                                       double &v) const {
+    aleft = ((a23 * r[0]) * r[0]) * sth;
+    aright = ((a23 * r[1]) * r[1]) * sth;
+    v = ((((r[3] * dx2a) * dx3a) * r[2]) * r[2]) * sth;
   }
   __device__ __forceinline__ void uload(int l, V5 &u, V5 &u1) const {
 #pragma unroll
-    for (int n = 0; n < 5; ++n) u.a[n] = U[n * vs + c0 + (size_t)l * jp];
+    for (int n = 0; n < 5; ++n) u.a[n] = *at(U, n, l);
     if (AVG && !first) {
 #pragma unroll
-      for (int n = 0; n < 5; ++n) u1.a[n] = U1[n * vs + c0 + (size_t)l * jp];
+      for (int n = 0; n < 5; ++n) u1.a[n] = *at(U1, n, l);
     }
   }
   // only u += delta is stored: nothing reads the correction itself afterwards
   __device__ __forceinline__ void finish(int l, const V5 &uo, const V5 &u1o, const V5 &d) const {
+    if (!act) return;
 #pragma unroll
     for (int n = 0; n < 5; ++n) {
-      size_t c = n * vs + c0 + (size_t)l * jp;
-      double ub = AVG ? stage_avg(sw, uo.a[n], first ? 0. : u1o.a[n], U1 + c) : uo.a[n];
-      U[c] = ub + d.a[n];
+      double ub = AVG ? stage_avg(sw, uo.a[n], first ? 0. : u1o.a[n], at(U1, n, l)) : uo.a[n];
+      *at(U, n, l) = ub + d.a[n];
     }
   }
 };
@@ -1570,19 +1582,27 @@ struct ColIOShim {
   double *dun;
   const double *area, *vol;
   int nc1, is;
+  bool act;
   __device__ __forceinline__ void wraw(int i, double *wv) const {
 #pragma unroll
     for (int n = 0; n < 5; ++n) wv[n] = w[n * nc1 + i];
   }
   __device__ __forceinline__ void project(double *) const {}
   __device__ __forceinline__ double du(int i, int n) const { return dun[n * nc1 + i]; }
-  __device__ __forceinline__ void geom(int i, double &aleft, double &aright, double &v) const {
-    aleft = area[i - is];
-    aright = area[i - is + 1];
-    v = vol[i - is];
+  __device__ __forceinline__ void graw(int i, double *r) const {
+    r[0] = area[i - is];
+    r[1] = area[i - is + 1];
+    r[2] = vol[i - is];
+  }
+  __device__ __forceinline__ void geom(const double *r, double &aleft, double &aright,
+                                       double &v) const {
+    aleft = r[0];
+    aright = r[1];
+    v = r[2];
   }
   __device__ __forceinline__ void uload(int, V5 &, V5 &) const {}
   __device__ __forceinline__ void finish(int l, const V5 &, const V5 &, const V5 &d) const {
+    if (!act) return;
 #pragma unroll
     for (int n = 0; n < 5; ++n) dun[n * nc1 + l] = d.a[n];
   }
@@ -1597,7 +1617,7 @@ struct ColIOShim {
 // once a whole sweep later, and streaming it past the caches leaves them to
 // the state (the solve 0.61 -> 0.56 ms on 6 x 96 x 96 x 64).
 template <bool AVG, typename IO>
-__device__ __forceinline__ void col5_solve(const IO &io, int is, int ie, double dt, double gamma,
+__device__ __forceinline__ void col5_solve_one(const IO &io, int is, int ie, double dt, double gamma,
                                            double grav, ADDR(1) dpair *__restrict__ CFP) {
   auto cfp = [&](int i, int q2) -> ADDR(1) dpair * {
     return CFP + ((size_t)(i - is) * 15 + q2) * 64;
@@ -1649,8 +1669,9 @@ __device__ __forceinline__ void col5_solve(const IO &io, int is, int ie, double 
 #pragma unroll
       for (int n = 0; n < 5; ++n) dun[n] = io.du(i + 1, n);
     }
-    double aleft, aright, v;
-    io.geom(i, aleft, aright, v);
+    double aleft, aright, v, gr[4];
+    io.graw(i, gr);
+    io.geom(gr, aleft, aright, v);
     double v2 = 2. * v, yv2 = qdiv(1., v2);
     // b, then b Aprev and b dprev, so b dies early (the first level keeps it
     // for the bottom fold)
@@ -1796,52 +1817,352 @@ __device__ __forceinline__ void col5_solve(const IO &io, int is, int ie, double 
   }
 }
 
-template <bool AVG>
-__device__ __forceinline__ void implicit_body(const DGrid &g, const DState &st, int lb,
-                                              const StageW &sw, double *geo) {
-  for (int q = threadIdx.x; q <= g.nc1; q += blockDim.x) {
-    geo[q] = g.x1f[q];
-    if (q < g.nc1) {
-      geo[IMPL_MAXNC1 + 1 + q] = g.x1v[q];
-      geo[2 * (IMPL_MAXNC1 + 1) + q] = g.dx1f[q];
+// The same solve by two waves: wave 1 assembles a level's rows (b, a, c and the
+// right-hand side: 80 doubles a lane, through LDS) and wave 0 eliminates (T = a -
+// b Aprev, its inverse, a^-1 c and delta).  The assembly has no recurrence, so it
+// runs a level ahead: |A| of the next face while wave 0 takes a level from LDS
+// and forms T, the rows while wave 0 inverts.  In the backward sweep wave 0
+// substitutes and wave 1 ends each level's state.  A column alone on its SIMD is
+// bound by latency, 11000 cycles a level by one wave, 7500 by two (assembly
+// 6100, elimination 5100, substitution 1300).  At 312 registers (no spills) a
+// SIMD takes one wave, a CU two blocks (COL5_CU), and a launch of more blocks
+// than that is faster by one wave a block, all 1024 places taken at once.  One
+// wave -> two: 6 x 16 x 16 x 16 82 -> 55 us, 6 x 48 x 48 x 48 254 -> 182, 6 x 64 x
+// 64 x 64 (384 blocks on 256 CUs) 398 -> 314; 6 x 80 x 80 x 32 (600 blocks) 253 ->
+// 296, 6 x 96 x 96 x 64 (864) 562 -> 607; 256 columns of 64 levels alone 298 ->
+// 193.  (Held to 256 registers for two waves a SIMD the assembly spills, and each
+// reload waits for the loads ahead: 6 x 96 x 96 x 64 750 us.)
+constexpr int COL5_CU = 2;
+constexpr int COL5_PAIRS = 40;
+constexpr int COL5_LDS = COL5_PAIRS * 64;  // dpairs: a level's rows, [pair][lane]
+constexpr int COL5_BK = 3;                 // levels of the backward sweep handed over at once
+
+template <typename IO>
+__device__ __forceinline__ void col5_assemble(const IO &io, int is, int ie, double dt,
+                                              double gamma, double grav, dpair *lds, int lane) {
+  double gm1c = (gamma - 1.) * 1. / 1.;
+  double gm1 = 0.5 * (gm1c + gm1c);
+  double k1 = qdiv(gm1c + 1, gm1c);
+  auto erow = [&](const double *w) { return qdiv(k1 * w[IPR], w[IDN]); };
+  // |A| at face is-1/2: the reference's row is-1 (full_correction.cpp:272-325)
+  // leaves Am = R|L|R^-1 of the Roe state of (w(is-1), w(is))
+  double wm[5], w0[5], prim[5];
+  io.wraw(is - 1, wm);
+  io.project(wm);
+  io.wraw(is, w0);
+  io.project(w0);
+  roe_average(prim, gm1, wm, w0);
+  double cs = sqrt(qdiv((1. + (gamma - 1) * 1. / 1.) * prim[IPR], prim[IDN]));
+  M5 Am = abs_a(prim, cs, gm1);
+  double em = erow(wm), e0 = erow(w0);
+  // divisions by dt and by 2 vol share one correctly rounded reciprocal each
+  double ydt = qdiv(1., dt);
+  // the next level's state, tendency and geometry are loaded a level ahead
+  double wnx[5], dun[5], gr[4];
+  io.wraw(is + 1, wnx);
+#pragma unroll
+  for (int n = 0; n < 5; ++n) dun[n] = io.du(is, n);
+  io.graw(is, gr);
+  for (int i = is; i <= ie; ++i) {
+    // |A| at the upper face, while wave 0 takes level i - 1 from LDS
+    double wp[5], rhs[5];
+#pragma unroll
+    for (int n = 0; n < 5; ++n) {
+      wp[n] = wnx[n];
+      rhs[n] = div_rn(dun[n], dt, ydt);
+    }
+    io.project(wp);
+    double aleft, aright, vol;
+    io.geom(gr, aleft, aright, vol);
+    {  // (past the top, the last level again: a load under a condition is waited for)
+      int nx = i < ie ? i + 1 : ie;
+      io.wraw(nx + 1, wnx);
+#pragma unroll
+      for (int n = 0; n < 5; ++n) dun[n] = io.du(nx, n);
+      io.graw(nx, gr);
+    }
+    double ep = erow(wp);
+    double v2 = 2. * vol, yv2 = qdiv(1., v2);
+    roe_average(prim, gm1, w0, wp);
+    cs = sqrt(qdiv((1. + (gamma - 1) * 1. / 1.) * prim[IPR], prim[IDN]));
+    M5 Ap = abs_a(prim, cs, gm1);
+    __syncthreads();
+    // the rows, each stored as it is formed, while wave 0 inverts level i - 1
+    {
+      M5 Jm = jac_e(gm1c, wm, em), J0 = jac_e(gm1c, w0, e0), Jp = jac_e(gm1c, wp, ep);
+#pragma unroll
+      for (int r = 0; r < 5; ++r) {
+        double v[16];  // rows r of b, a and c, and the right-hand side
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+          v[q] = div_rn(-(Am.a[r][q] + Jm.a[r][q]) * aleft, v2, yv2);
+          v[10 + q] = div_rn(-(Ap.a[r][q] - Jp.a[r][q]) * aright, v2, yv2);
+          double a = div_rn(Am.a[r][q] * aleft + Ap.a[r][q] * aright +
+                                (aright - aleft) * J0.a[r][q],
+                            v2, yv2);
+          if (r == q) a += ydt;
+          if ((r == IVX && q == IDN) || (r == IEN && q == IVX)) a -= grav;
+          v[5 + q] = a;
+        }
+        v[15] = rhs[r];
+        // (the empty statements keep these two a branch, not 100 selects)
+        if (i == is) {  // reflecting bottom
+          asm volatile("");
+#pragma unroll
+          for (int q = 0; q < 5; ++q) v[5 + q] += v[q] * (q == IVX ? -1. : 1.);
+        }
+        if (i == ie) {  // reflecting top
+          asm volatile("");
+#pragma unroll
+          for (int q = 0; q < 5; ++q) v[5 + q] += v[10 + q] * (q == IVX ? -1. : 1.);
+        }
+#pragma unroll
+        for (int q2 = 0; q2 < 8; ++q2)
+          lds[(8 * r + q2) * 64 + lane] = dpair{v[2 * q2], v[2 * q2 + 1]};
+        __builtin_amdgcn_sched_barrier(0);  // a row's registers are free for the next
+      }
+    }
+    __syncthreads();
+    Am = Ap;
+    em = e0;
+    e0 = ep;
+#pragma unroll
+    for (int n = 0; n < 5; ++n) {
+      wm[n] = w0[n];
+      w0[n] = wp[n];
     }
   }
+}
+
+// Wave 0.  CFP is the lane's base of the coefficient scratch, [level][pair][64
+// lanes]: the 30 doubles of a level (a^-1 c row-major, then delta) as 15 pairs,
+// each pair 64 lanes x 16 B contiguous, so a level is 15 coalesced 16-byte
+// stores, and 15 loads back.  Both are non-temporal: each coefficient is written
+// once and read once a whole sweep later, and streaming it past the caches
+// leaves them to the state.
+__device__ __forceinline__ void col5_eliminate(int is, int ie, ADDR(1) dpair *__restrict__ CFP,
+                                               dpair *lds, int lane) {
+  auto cfp = [&](int i, int q2) -> ADDR(1) dpair * {
+    return CFP + ((size_t)(i - is) * 15 + q2) * 64;
+  };
+  M5 Aprev;
+  V5 dprev;
   __syncthreads();
+  for (int i = is; i <= ie; ++i) {
+    M5 T, c;
+    V5 tv;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 5; ++r) {
+      double v[16];
+#pragma unroll
+      for (int q2 = 0; q2 < 8; ++q2) {
+        dpair t = lds[(8 * r + q2) * 64 + lane];
+        v[2 * q2] = t.x;
+        v[2 * q2 + 1] = t.y;
+      }
+#pragma unroll
+      for (int q = 0; q < 5; ++q) c.a[r][q] = v[10 + q];
+      if (i > is) {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+          double t = v[0] * Aprev.a[0][q];
+#pragma unroll
+          for (int k = 1; k < 5; ++k) t = fma(v[k], Aprev.a[k][q], t);
+          T.a[r][q] = v[5 + q] - t;
+        }
+        double t = v[0] * dprev.a[0];
+#pragma unroll
+        for (int k = 1; k < 5; ++k) t = fma(v[k], dprev.a[k], t);
+        tv.a[r] = v[15] - t;
+      } else {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) T.a[r][q] = v[5 + q];
+        tv.a[r] = v[15];
+      }
+    }
+    if (i < ie) __syncthreads();
+    M5 ainv = m5_inv(T);
+    dprev = m5_mulv(ainv, tv);
+    Aprev = m5_mul(ainv, c);
+    double cv[30];
+#pragma unroll
+    for (int e = 0; e < 25; ++e) cv[e] = Aprev.a[e / 5][e % 5];
+#pragma unroll
+    for (int n = 0; n < 5; ++n) cv[25 + n] = dprev.a[n];
+#pragma unroll
+    for (int q2 = 0; q2 < 15; ++q2)
+      __builtin_nontemporal_store(dpair{cv[2 * q2], cv[2 * q2 + 1]}, cfp(i, q2));
+  }
+  // backward substitution, level ie - t for t = 0, 1, ..; delta(ie) is final.
+  // COL5_BK levels are loaded ahead, 45 of the 63 loads the vector-memory
+  // counter tracks; past the bottom the last level is loaded again and its
+  // results are not taken, as a load under a condition would be waited for.
+  constexpr int PD = COL5_BK;
+  int nl = ie - is + 1;
+  M5 Aq[PD];
+  V5 dq[PD];
+  auto bload = [&](int t, M5 &A, V5 &d) {
+    int i = ie - t < is ? is : ie - t;
+    double cv[30];
+#pragma unroll
+    for (int q2 = 0; q2 < 15; ++q2) {
+      dpair x = __builtin_nontemporal_load(cfp(i, q2));
+      cv[2 * q2] = x.x;
+      cv[2 * q2 + 1] = x.y;
+    }
+#pragma unroll
+    for (int e = 0; e < 25; ++e) A.a[e / 5][e % 5] = cv[e];
+#pragma unroll
+    for (int n = 0; n < 5; ++n) d.a[n] = cv[25 + n];
+  };
+  // out: [parity of the piece][level][variable][lane], and delta(ie)
+  double *out = (double *)lds + lane;
+  V5 dnext = dprev;
+#pragma unroll
+  for (int n = 0; n < 5; ++n) out[(2 * PD * 5 + n) * 64] = dnext.a[n];
+#pragma unroll
+  for (int q = 0; q < PD; ++q) bload(1 + q, Aq[q], dq[q]);
+  for (int t0 = 1, par = 0; t0 < nl || par + t0 == 1; t0 += PD, par ^= 1) {
+#pragma unroll
+    for (int q = 0; q < PD; ++q) {
+      V5 ad = m5_mulv(Aq[q], dnext);
+#pragma unroll
+      for (int n = 0; n < 5; ++n) dnext.a[n] = dq[q].a[n] - ad.a[n];
+      bload(t0 + q + PD, Aq[q], dq[q]);
+#pragma unroll
+      for (int n = 0; n < 5; ++n) out[((par * PD + q) * 5 + n) * 64] = dnext.a[n];
+    }
+    __syncthreads();
+  }
+}
+
+// Wave 1 in the backward sweep: ends each level's correction, its state loaded
+// a piece ahead.
+template <typename IO>
+__device__ __forceinline__ void col5_finish(const IO &io, int is, int ie, const dpair *lds,
+                                            int lane) {
+  constexpr int PD = COL5_BK;
+  int nl = ie - is + 1;
+  const double *in = (const double *)lds + lane;
+  V5 u[PD], u1[PD], ue, u1e;
+  auto load = [&](int t, V5 &u, V5 &u1) { io.uload(ie - t < is ? is : ie - t, u, u1); };
+  auto take = [&](int e) {
+    V5 d;
+#pragma unroll
+    for (int n = 0; n < 5; ++n) d.a[n] = in[(e * 5 + n) * 64];
+    return d;
+  };
+  load(0, ue, u1e);
+#pragma unroll
+  for (int q = 0; q < PD; ++q) load(1 + q, u[q], u1[q]);
+  __syncthreads();
+  io.finish(ie, ue, u1e, take(2 * PD));
+  int t0 = 1, par = 0;
+  for (; t0 + PD <= nl; t0 += PD, par ^= 1) {
+    if (t0 > 1) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PD; ++q) {
+      V5 uo = u[q], u1o = u1[q];
+      load(t0 + q + PD, u[q], u1[q]);
+      io.finish(ie - t0 - q, uo, u1o, take(par * PD + q));
+    }
+  }
+  if (t0 < nl) {
+    if (t0 > 1) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PD; ++q)
+      if (t0 + q < nl) io.finish(ie - t0 - q, u[q], u1[q], take(par * PD + q));
+  }
+}
+
+template <typename IO>
+__device__ __forceinline__ void col5_solve_two(const IO &io, int is, int ie, double dt,
+                                               double gamma, double grav, ADDR(1) dpair *CFP,
+                                               dpair *lds) {
+  int lane = threadIdx.x & 63;
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0) {
+    col5_eliminate(is, ie, CFP, lds, lane);
+  } else {
+    col5_assemble(io, is, ie, dt, gamma, grav, lds, lane);
+    col5_finish(io, is, ie, lds, lane);
+  }
+}
+
+// the column of this lane, in block lb of 64 columns; a lane past the panel's
+// last column runs along with it and stores nothing
+template <bool AVG, typename GP>
+__device__ __forceinline__ ColIOGrid<AVG, GP> col_io(const DGrid &g, const DState &st, int lb,
+                                                     const StageW &sw) {
   int N = g.N;
   int nbx = (N * N + 63) / 64;
-  int col = (lb % nbx) * 64 + threadIdx.x;
+  int col = (lb % nbx) * 64 + (threadIdx.x & 63);
   int p = lb / nbx;
-  if (col >= N * N) return;
+  ColIOGrid<AVG, GP> io;
+  io.act = col < N * N;
+  if (!io.act) col = N * N - 1;
   int k = g.ks + col / N, j = g.js + col % N;
-  ColIOGrid<AVG> io;
-  io.W = st.w;
-  io.DU = st.du;
-  io.U = st.u;
-  io.U1 = st.u1;
+  size_t panel = p * g.pstride;
+  io.W = st.w + panel;
+  io.DU = st.du + panel;
+  io.U = st.u + panel;
+  io.U1 = st.u1 + panel;
   io.vs = g.vstride;
   io.jp = g.jp;
-  io.c0 = g.c(0, p, k, 0, j);  // column base (variable 0, i = 0)
+  io.off = (unsigned)((k * g.plane + j) * sizeof(double));
   io.cth = g.T(T_COSC, p, k, j);
   io.sth = g.T(T_SINC, p, k, j);
   io.dx2a = g.T(T_DX2A, p, k, j);
   io.dx3a = g.T(T_DX3A, p, k, j);
   io.a23 = io.dx2a * io.dx3a;
-  io.x1f = geo;
-  io.x1v = geo + IMPL_MAXNC1 + 1;
-  io.dx1f = geo + 2 * (IMPL_MAXNC1 + 1);
   io.sw = sw;
   io.first = sw.first;
-  ADDR(1) dpair *CFP = (ADDR(1) dpair *)st.coef + (size_t)lb * g.nx1 * 15 * 64 + threadIdx.x;
-  col5_solve<AVG>(io, g.is, g.ie, sw.beta * st.dtv[0], g.gamma, g.grav, CFP);
+  return io;
+}
+__device__ __forceinline__ ADDR(1) dpair *col5_coef(const DGrid &g, const DState &st, int lb) {
+  return (ADDR(1) dpair *)st.coef + (size_t)lb * g.nx1 * 15 * 64 + (threadIdx.x & 63);
 }
 
+// geo: LDS for the instance's x1f | x1v | dx1f, so the per-level geometry is
+// read without waiting on the vector-memory counter (which also counts the
+// coefficient stores and the prefetches in flight)
 template <bool AVG>
 __global__ void __launch_bounds__(64) k_implicit(const Inst *__restrict__ I_, Work w, StageW sw) {
   __shared__ double geo[3 * (IMPL_MAXNC1 + 1)];
   WORK_LOOP(w) {
     WORK_INST(w);
-    implicit_body<AVG>(g, st, lb, sw, geo);
+    for (int q = threadIdx.x; q <= g.nc1; q += blockDim.x) {
+      geo[q] = g.x1f[q];
+      if (q < g.nc1) {
+        geo[IMPL_MAXNC1 + 1 + q] = g.x1v[q];
+        geo[2 * (IMPL_MAXNC1 + 1) + q] = g.dx1f[q];
+      }
+    }
+    __syncthreads();
+    auto io = col_io<AVG, const double *>(g, st, lb, sw);
+    io.x1f = geo;
+    io.x1v = geo + IMPL_MAXNC1 + 1;
+    io.dx1f = geo + 2 * (IMPL_MAXNC1 + 1);
+    if (io.act)
+      col5_solve_one<AVG>(io, g.is, g.ie, sw.beta * st.dtv[0], g.gamma, g.grav,
+                          col5_coef(g, st, lb));
     __syncthreads();  // geo is refilled by the next block of the loop
+  }
+}
+
+template <bool AVG>
+__global__ void __launch_bounds__(128) k_implicit_two(const Inst *__restrict__ I_, Work w,
+                                                      StageW sw) {
+  __shared__ dpair lds[COL5_LDS];
+  WORK_LOOP(w) {
+    WORK_INST(w);
+    auto io = col_io<AVG, const ADDR(1) double *>(g, st, lb, sw);
+    io.x1f = g.x1f;
+    io.x1v = g.x1v;
+    io.dx1f = g.dx1f;
+    col5_solve_two(io, g.is, g.ie, sw.beta * st.dtv[0], g.gamma, g.grav, col5_coef(g, st, lb),
+                   lds);
+    __syncthreads();
   }
 }
 
@@ -1849,20 +2170,23 @@ __global__ void __launch_bounds__(64) k_implicit(const Inst *__restrict__ I_, Wo
 // column: column c's arrays follow column c - 1's (w and du nc1 levels of 5
 // variables, nx1 + 1 face areas, nx1 volumes); coef holds the coefficient
 // scratch, [64-column block][level][pair][64 lanes], written by each column's
-// forward sweep before its backward substitution reads it.
-__global__ void __launch_bounds__(64) k_implicit_columns(ColIOShim io, int ncol, int nx1,
-                                                         double dt, double gamma, double grav,
-                                                         double *coef) {
-  int c = blockIdx.x * 64 + threadIdx.x;
-  if (c >= ncol) return;
+// forward sweep before its backward substitution reads it.  The fixed scratch
+// bounds them to 273 blocks: two waves each.
+__global__ void __launch_bounds__(128)
+k_implicit_columns(ColIOShim io, int ncol, int nx1, double dt, double gamma, double grav,
+                   double *coef) {
+  __shared__ dpair lds[COL5_LDS];
+  int lane = threadIdx.x & 63;
+  int c = blockIdx.x * 64 + lane;
   ColIOShim cio = io;
+  cio.act = c < ncol;
+  if (!cio.act) c = ncol - 1;  // the lane runs along and stores nothing
   cio.w += (size_t)c * 5 * io.nc1;
   cio.dun += (size_t)c * 5 * io.nc1;
   cio.area += (size_t)c * (nx1 + 1);
   cio.vol += (size_t)c * nx1;
-  ADDR(1) dpair *CFP =
-      (ADDR(1) dpair *)glb(coef) + (size_t)blockIdx.x * nx1 * 15 * 64 + threadIdx.x;
-  col5_solve<false>(cio, NG, NG + nx1 - 1, dt, gamma, grav, CFP);
+  ADDR(1) dpair *CFP = (ADDR(1) dpair *)glb(coef) + (size_t)blockIdx.x * nx1 * 15 * 64 + lane;
+  col5_solve_two(cio, NG, NG + nx1 - 1, dt, gamma, grav, CFP, lds);
 }
 
 // ImplicitSolver::PartialCorrection on an x1 column (partial_correction.cpp:
@@ -3919,6 +4243,17 @@ void launch_update(Launcher &L, int stage, int prim) {
   HIPCHK(hipGetLastError());
 }
 
+// The 5x5 column solve: by two waves a block of 64 columns while the device has
+// a place for every block at once (two of them a CU), else by one.
+bool col5_two(int nblk, int ncu) { return nblk <= COL5_CU * ncu; }
+template <bool AVG>
+void launch_col5(Launcher &L, int kind, const StageW &sw) {
+  if (col5_two((int)L.grid(kind), L.ncu))
+    launch(L, kind, KID_IMPLICIT, k_implicit_two<AVG>, 128, 0, sw);
+  else
+    launch(L, kind, KID_IMPLICIT, k_implicit<AVG>, 64, 0, sw);
+}
+
 // the stage's update and column correction after launch_fluxes(L, true): the
 // ideal gas's x2 faces and tendency in one kernel (k_face2_update), whose
 // column step then forms the stage's weighted average of u; shallow water's
@@ -3932,7 +4267,7 @@ void launch_update_implicit(Launcher &L, int stage) {
   launch_fuse2<true, false>(L, K_FUSE2_S, KID_UPDATE, sw);
   launch_fuse2<false, true>(L, K_FUSE2_MIX, KID_UPDATE, sw);
   launch_fuse2<true, true>(L, K_FUSE2_MIX_S, KID_UPDATE, sw);
-  launch(L, K_IMPL_AVG, KID_IMPLICIT, k_implicit<true>, 64, 0, sw);
+  launch_col5<true>(L, K_IMPL_AVG, sw);
   launch(L, K_IMPL3_AVG, KID_IMPLICIT, k_implicit3<true>, 64, 0, sw);
   launch(L, K_ADD_DU_AVG, KID_IMPLICIT, k_add_du<true>, BLK, 0, sw);
   HIPCHK(hipGetLastError());
@@ -3941,7 +4276,7 @@ void launch_update_implicit(Launcher &L, int stage) {
 void launch_implicit(Launcher &L, double beta) {
   StageW sw{};
   sw.beta = beta;
-  launch(L, K_IMPL, KID_IMPLICIT, k_implicit<false>, 64, 0, sw);
+  launch_col5<false>(L, K_IMPL, sw);
   launch(L, K_IMPL3, KID_IMPLICIT, k_implicit3<false>, 64, 0, sw);
   launch(L, K_ADD_DU, KID_IMPLICIT, k_add_du<false>, BLK, 0, sw);
   HIPCHK(hipGetLastError());
@@ -4857,8 +5192,8 @@ int exo_implicit_column(exo_handle *h, int nx1, const double *w_col, double *du_
     HIPCHK(hipMemcpyAsync(da, area1, (nx1 + 1) * sizeof(double), hipMemcpyHostToDevice,
                           h->stream));
     HIPCHK(hipMemcpyAsync(dv, vol, nx1 * sizeof(double), hipMemcpyHostToDevice, h->stream));
-    ColIOShim io{dw, ddu, da, dv, nc1, NG};
-    hipLaunchKernelGGL(k_implicit_columns, dim3(1), dim3(64), 0, h->stream, io, 1, nx1, dt,
+    ColIOShim io{dw, ddu, da, dv, nc1, NG, true};
+    hipLaunchKernelGGL(k_implicit_columns, dim3(1), dim3(128), 0, h->stream, io, 1, nx1, dt,
                        h->g.gamma, h->g.grav, d);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(du_col, ddu, nw * sizeof(double), hipMemcpyDeviceToHost, h->stream));
@@ -4881,8 +5216,8 @@ int exo_implicit_columns_noalloc(exo_handle *h, int ncol, int nx1, const double 
           " doubles of coefficient scratch, above the fixed " +
           std::to_string(EXO_NOALLOC_SCRATCH_DOUBLES);
     double *scr = scratch_ptr();
-    ColIOShim io{w_cols, du_cols, area1, vol, nx1 + 2 * NG, NG};
-    hipLaunchKernelGGL(k_implicit_columns, dim3((unsigned)nblk), dim3(64), 0, h->stream, io,
+    ColIOShim io{w_cols, du_cols, area1, vol, nx1 + 2 * NG, NG, true};
+    hipLaunchKernelGGL(k_implicit_columns, dim3((unsigned)nblk), dim3(128), 0, h->stream, io,
                        ncol, nx1, dt, h->g.gamma, h->g.grav, scr);
     HIPCHK(hipGetLastError());
   });
