@@ -1825,14 +1825,14 @@ __device__ __forceinline__ void col5_solve_one(const IO &io, int is, int ie, dou
 // substitutes and wave 1 ends each level's state.  A column alone on its SIMD is
 // bound by latency, 11000 cycles a level by one wave, 7500 by two (assembly
 // 6100, elimination 5100, substitution 1300).  At 312 registers (no spills) a
-// SIMD takes one wave, a CU two blocks (COL5_CU), and a launch of more blocks
+// SIMD takes one wave, a CU two blocks (COL_CU), and a launch of more blocks
 // than that is faster by one wave a block, all 1024 places taken at once.  One
 // wave -> two: 6 x 16 x 16 x 16 82 -> 55 us, 6 x 48 x 48 x 48 254 -> 182, 6 x 64 x
 // 64 x 64 (384 blocks on 256 CUs) 398 -> 314; 6 x 80 x 80 x 32 (600 blocks) 253 ->
 // 296, 6 x 96 x 96 x 64 (864) 562 -> 607; 256 columns of 64 levels alone 298 ->
 // 193.  (Held to 256 registers for two waves a SIMD the assembly spills, and each
 // reload waits for the loads ahead: 6 x 96 x 96 x 64 750 us.)
-constexpr int COL5_CU = 2;
+constexpr int COL_CU = 2;
 constexpr int COL5_PAIRS = 40;
 constexpr int COL5_LDS = COL5_PAIRS * 64;  // dpairs: a level's rows, [pair][lane]
 constexpr int COL5_BK = 3;                 // levels of the backward sweep handed over at once
@@ -2226,7 +2226,6 @@ __device__ __forceinline__ void implicit3_body(const DGrid &g, const DState &st,
   ADDR(1) double *__restrict__ U = st.u;
   // coefficient scratch, [block][level][pair][lane]: the 12 doubles of a level
   // (a^-1 c row-major, then delta) as 6 pairs of 64 lanes x 16 B
-  typedef double dpair __attribute__((ext_vector_type(2)));
   ADDR(1) dpair *__restrict__ CFP =
       (ADDR(1) dpair *)st.coef + (size_t)lb * g.nx1 * 6 * 64 + threadIdx.x;
   auto cfp = [&](int i, int q2) -> ADDR(1) dpair * {
@@ -2440,6 +2439,275 @@ __global__ void __launch_bounds__(64) k_implicit3(const Inst *__restrict__ I_, W
   }
 }
 
+// The same by three waves a block of 64 columns: waves 1 and 2 assemble the rows
+// of every second level (b, a, c and the right-hand side: 30 doubles a lane,
+// through LDS), wave 0 eliminates the two levels before; in the backward sweep
+// wave 0 substitutes and the others end the levels' states.  Assembly is two
+// thirds of a level's work, so one assembling wave would hold the other up.  As
+// the 5x5 solve, a block is bound by latency and this form is for launches of at
+// most COL_CU blocks a CU (its 60 KB of LDS leave no place for a third).  One
+// wave -> three: 6 x 16 x 16 x 16 41 -> 25 us, 6 x 48 x 48 x 48 128 -> 85, 6 x 64 x
+// 64 x 47 (384 blocks on 256 CUs) 148 -> 131; 6 x 80 x 80 x 32 (600 blocks) 131 ->
+// 142, 6 x 96 x 96 x 64 (864) 315 -> 374.
+constexpr int COL3_A = 2;       // assembling waves
+constexpr int COL3_PAIRS = 15;  // of a level's rows
+constexpr int COL3_BK = 6;      // levels of the backward sweep handed over at once
+constexpr int COL3_LDS = 2 * COL3_A * COL3_PAIRS * 64;  // dpairs, [parity][level][pair][lane]
+static_assert((2 * COL3_BK + 1) * 3 <= 2 * COL3_LDS / 64, "the backward sweep's corrections");
+
+template <typename IO>
+__device__ __forceinline__ void col3_assemble(const IO &io, int is, int ie, double dt,
+                                              double gamma, double grav, dpair *lds, int lane,
+                                              int wa) {
+  double gm1c = (gamma - 1.) * 1. / 1.;
+  double gm1 = 0.5 * (gm1c + gm1c);
+  double k1 = qdiv(gm1c + 1, gm1c);
+  auto erow = [&](const double *w) { return qdiv(k1 * w[IPR], w[IDN]); };
+  auto face = [&](const double *wl, const double *wr) {
+    double prim[5];
+    roe_average(prim, gm1, wl, wr);
+    double cs = sqrt(qdiv((1. + (gamma - 1) * 1. / 1.) * prim[IPR], prim[IDN]));
+    return abs_a(prim, cs, gm1);
+  };
+  double ydt = qdiv(1., dt);
+  // the wave's next level, loaded a level ahead (past the top, the last level
+  // again: a load under a condition would be waited for)
+  double wn[3][5], dun[3], gr[4];
+  auto load = [&](int i) {
+    if (i > ie) i = ie;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) io.wraw(i - 1 + e, wn[e]);
+#pragma unroll
+    for (int n = 0; n < 3; ++n) dun[n] = io.du(i, SUB3[n]);
+    io.graw(i, gr);
+  };
+  load(is + wa);
+  for (int i0 = is, par = 0; i0 <= ie; i0 += COL3_A, par ^= 1) {
+    int i = i0 + wa < ie ? i0 + wa : ie;
+    double wm[5], w0[5], wp[5], rhs[3];
+#pragma unroll
+    for (int n = 0; n < 5; ++n) {
+      wm[n] = wn[0][n];
+      w0[n] = wn[1][n];
+      wp[n] = wn[2][n];
+    }
+#pragma unroll
+    for (int n = 0; n < 3; ++n) rhs[n] = div_rn(dun[n], dt, ydt);
+    double aleft, aright, vol;
+    io.geom(gr, aleft, aright, vol);
+    load(i0 + COL3_A + wa);
+    io.project(wm);
+    io.project(w0);
+    io.project(wp);
+    M5 Am = face(wm, w0), Ap = face(w0, wp);
+    double v2 = 2. * vol, yv2 = qdiv(1., v2);
+    M5 Jm = jac_e(gm1c, wm, erow(wm)), J0 = jac_e(gm1c, w0, erow(w0)),
+       Jp = jac_e(gm1c, wp, erow(wp));
+    double v[30];  // rows r of b, a and c and the right-hand side, r = 0, 1, 2
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        int R = SUB3[r], Q = SUB3[q];
+        v[10 * r + q] = div_rn(-(Am.a[R][Q] + Jm.a[R][Q]) * aleft, v2, yv2);
+        v[10 * r + 6 + q] = div_rn(-(Ap.a[R][Q] - Jp.a[R][Q]) * aright, v2, yv2);
+        double a = div_rn(Am.a[R][Q] * aleft + Ap.a[R][Q] * aright +
+                              (aright - aleft) * J0.a[R][Q],
+                          v2, yv2);
+        if (r == q) a += ydt;
+        if ((r == 1 && q == 0) || (r == 2 && q == 1)) a -= grav;
+        v[10 * r + 3 + q] = a;
+      }
+      v[10 * r + 9] = rhs[r];
+    }
+    if (i == is)  // reflecting bottom
+#pragma unroll
+      for (int e = 0; e < 9; ++e)
+        v[10 * (e / 3) + 3 + e % 3] += v[10 * (e / 3) + e % 3] * (e % 3 == 1 ? -1. : 1.);
+    if (i == ie)  // reflecting top
+#pragma unroll
+      for (int e = 0; e < 9; ++e)
+        v[10 * (e / 3) + 3 + e % 3] += v[10 * (e / 3) + 6 + e % 3] * (e % 3 == 1 ? -1. : 1.);
+#pragma unroll
+    for (int q2 = 0; q2 < COL3_PAIRS; ++q2)
+      lds[((par * COL3_A + wa) * COL3_PAIRS + q2) * 64 + lane] = dpair{v[2 * q2], v[2 * q2 + 1]};
+    __syncthreads();  // and wave 0 is done with the levels of the other parity
+  }
+}
+
+// Wave 0.  Coefficient scratch, [block][level][pair][lane]: the 12 doubles of a
+// level (a^-1 c row-major, then delta) as 6 pairs of 64 lanes x 16 B.
+__device__ __forceinline__ void col3_eliminate(int is, int ie, ADDR(1) dpair *__restrict__ CFP,
+                                               dpair *lds, int lane) {
+  auto cfp = [&](int i, int q2) -> ADDR(1) dpair * {
+    return CFP + ((size_t)(i - is) * 6 + q2) * 64;
+  };
+  M3 Aprev;
+  V3 dprev;
+  for (int i0 = is, par = 0; i0 <= ie; i0 += COL3_A, par ^= 1) {
+    __syncthreads();
+    for (int l = 0; l < COL3_A && i0 + l <= ie; ++l) {
+      int i = i0 + l;
+      double v[30];
+#pragma unroll
+      for (int q2 = 0; q2 < COL3_PAIRS; ++q2) {
+        dpair t = lds[((par * COL3_A + l) * COL3_PAIRS + q2) * 64 + lane];
+        v[2 * q2] = t.x;
+        v[2 * q2 + 1] = t.y;
+      }
+      M3 b, T, c;
+      V3 tv;
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          b.a[r][q] = v[10 * r + q];
+          T.a[r][q] = v[10 * r + 3 + q];
+          c.a[r][q] = v[10 * r + 6 + q];
+        }
+        tv.a[r] = v[10 * r + 9];
+      }
+      if (i > is) {
+        M3 ba = m3_mul(b, Aprev);
+        V3 bd = m3_mulv(b, dprev);
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+#pragma unroll
+          for (int q = 0; q < 3; ++q) T.a[r][q] = T.a[r][q] - ba.a[r][q];
+          tv.a[r] = tv.a[r] - bd.a[r];
+        }
+      }
+      M3 ainv = m3_inv(T);
+      dprev = m3_mulv(ainv, tv);
+      Aprev = m3_mul(ainv, c);
+      double cv[12];
+#pragma unroll
+      for (int e = 0; e < 9; ++e) cv[e] = Aprev.a[e / 3][e % 3];
+#pragma unroll
+      for (int n = 0; n < 3; ++n) cv[9 + n] = dprev.a[n];
+#pragma unroll
+      for (int q2 = 0; q2 < 6; ++q2)
+        __builtin_nontemporal_store(dpair{cv[2 * q2], cv[2 * q2 + 1]}, cfp(i, q2));
+    }
+  }
+  // backward substitution, level ie - t for t = 0, 1, ..; delta(ie) is final;
+  // COL3_BK levels are loaded ahead (36 of the 63 loads the vector-memory
+  // counter tracks), past the bottom the last level again
+  constexpr int PD = COL3_BK;
+  int nl = ie - is + 1;
+  double cq[PD][12];
+  auto bload = [&](int t, double *cv) {
+    int i = ie - t < is ? is : ie - t;
+#pragma unroll
+    for (int q2 = 0; q2 < 6; ++q2) {
+      dpair x = __builtin_nontemporal_load(cfp(i, q2));
+      cv[2 * q2] = x.x;
+      cv[2 * q2 + 1] = x.y;
+    }
+  };
+  // out: [parity of the piece][level][variable][lane], and delta(ie)
+  double *out = (double *)lds + lane;
+  V3 dnext = dprev;
+#pragma unroll
+  for (int n = 0; n < 3; ++n) out[(2 * PD * 3 + n) * 64] = dnext.a[n];
+#pragma unroll
+  for (int q = 0; q < PD; ++q) bload(1 + q, cq[q]);
+  for (int t0 = 1, par = 0; t0 < nl || t0 == 1; t0 += PD, par ^= 1) {
+#pragma unroll
+    for (int q = 0; q < PD; ++q) {
+      M3 A;
+#pragma unroll
+      for (int e = 0; e < 9; ++e) A.a[e / 3][e % 3] = cq[q][e];
+      V3 ad = m3_mulv(A, dnext);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) dnext.a[n] = cq[q][9 + n] - ad.a[n];
+      bload(t0 + q + PD, cq[q]);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) out[((par * PD + q) * 3 + n) * 64] = dnext.a[n];
+    }
+    __syncthreads();
+  }
+}
+
+// Waves 1 and 2 in the backward sweep: u += du of every second level, the
+// corrected (density, x1 momentum, energy) and the explicit transverse momenta;
+// with AVG on the stage's weighted average of u, formed here.  A level's state
+// is loaded a piece ahead.
+template <bool AVG, typename IO>
+__device__ __forceinline__ void col3_finish(const IO &io, int is, int ie, const dpair *lds,
+                                            int lane, int wa) {
+  constexpr int PD = COL3_BK, PW = PD / COL3_A;
+  int nl = ie - is + 1;
+  const double *in = (const double *)lds + lane;
+  struct Lev {
+    V5 u, u1;
+    double d2, d3;
+  } ue, uq[PW];
+  auto load = [&](int t, Lev &x) {
+    int i = ie - t < is ? is : ie - t;
+    io.uload(i, x.u, x.u1);
+    x.d2 = io.du(i, IVY);
+    x.d3 = io.du(i, IVZ);
+  };
+  auto end = [&](int i, const Lev &x, int e) {
+    if (!io.act) return;
+    double ub[5];
+#pragma unroll
+    for (int n = 0; n < 5; ++n)
+      ub[n] = AVG ? stage_avg(io.sw, x.u.a[n], io.first ? 0. : x.u1.a[n], io.at(io.U1, n, i))
+                  : x.u.a[n];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) *io.at(io.U, SUB3[n], i) = ub[SUB3[n]] + in[(e * 3 + n) * 64];
+    *io.at(io.U, IVY, i) = ub[IVY] + x.d2;
+    *io.at(io.U, IVZ, i) = ub[IVZ] + x.d3;
+  };
+  load(0, ue);
+#pragma unroll
+  for (int q = 0; q < PW; ++q) load(1 + q * COL3_A + wa, uq[q]);
+  __syncthreads();
+  if (wa == 0) end(ie, ue, 2 * PD);
+  int t0 = 1, par = 0;
+  for (; t0 + PD <= nl; t0 += PD, par ^= 1) {
+    if (t0 > 1) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PW; ++q) {
+      int l = q * COL3_A + wa;
+      Lev x = uq[q];
+      load(t0 + PD + l, uq[q]);
+      end(ie - t0 - l, x, par * PD + l);
+    }
+  }
+  if (t0 < nl) {
+    if (t0 > 1) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PW; ++q) {
+      int l = q * COL3_A + wa;
+      if (t0 + l < nl) end(ie - t0 - l, uq[q], par * PD + l);
+    }
+  }
+}
+
+template <bool AVG>
+__global__ void __launch_bounds__(64 * (1 + COL3_A)) __attribute__((amdgpu_waves_per_eu(2)))
+k_implicit3_three(const Inst *__restrict__ I_, Work w, StageW sw) {
+  __shared__ dpair lds[COL3_LDS];
+  int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  WORK_LOOP(w) {
+    WORK_INST(w);
+    auto io = col_io<AVG, const ADDR(1) double *>(g, st, lb, sw);
+    io.x1f = g.x1f;
+    io.x1v = g.x1v;
+    io.dx1f = g.dx1f;
+    if (wave == 0) {
+      col3_eliminate(g.is, g.ie, (ADDR(1) dpair *)st.coef + (size_t)lb * g.nx1 * 6 * 64 + lane,
+                     lds, lane);
+    } else {
+      col3_assemble(io, g.is, g.ie, sw.beta * st.dtv[0], g.gamma, g.grav, lds, lane, wave - 1);
+      col3_finish<AVG>(io, g.is, g.ie, lds, lane, wave - 1);
+    }
+    __syncthreads();
+  }
+}
 
 // u += du without the column solve (ImplicitHydroTasks with implicit_flag 0)
 // AVG (within a stage): u = the stage's weighted average + du
@@ -4243,15 +4511,22 @@ void launch_update(Launcher &L, int stage, int prim) {
   HIPCHK(hipGetLastError());
 }
 
-// The 5x5 column solve: by two waves a block of 64 columns while the device has
-// a place for every block at once (two of them a CU), else by one.
-bool col5_two(int nblk, int ncu) { return nblk <= COL5_CU * ncu; }
+// The column solves: by several waves a block of 64 columns while the device has
+// a place for every block at once (COL_CU of them a CU), else by one.
+bool col_split(int nblk, int ncu) { return nblk <= COL_CU * ncu; }
 template <bool AVG>
 void launch_col5(Launcher &L, int kind, const StageW &sw) {
-  if (col5_two((int)L.grid(kind), L.ncu))
+  if (col_split((int)L.grid(kind), L.ncu))
     launch(L, kind, KID_IMPLICIT, k_implicit_two<AVG>, 128, 0, sw);
   else
     launch(L, kind, KID_IMPLICIT, k_implicit<AVG>, 64, 0, sw);
+}
+template <bool AVG>
+void launch_col3(Launcher &L, int kind, const StageW &sw) {
+  if (col_split((int)L.grid(kind), L.ncu))
+    launch(L, kind, KID_IMPLICIT, k_implicit3_three<AVG>, 64 * (1 + COL3_A), 0, sw);
+  else
+    launch(L, kind, KID_IMPLICIT, k_implicit3<AVG>, 64, 0, sw);
 }
 
 // the stage's update and column correction after launch_fluxes(L, true): the
@@ -4268,7 +4543,7 @@ void launch_update_implicit(Launcher &L, int stage) {
   launch_fuse2<false, true>(L, K_FUSE2_MIX, KID_UPDATE, sw);
   launch_fuse2<true, true>(L, K_FUSE2_MIX_S, KID_UPDATE, sw);
   launch_col5<true>(L, K_IMPL_AVG, sw);
-  launch(L, K_IMPL3_AVG, KID_IMPLICIT, k_implicit3<true>, 64, 0, sw);
+  launch_col3<true>(L, K_IMPL3_AVG, sw);
   launch(L, K_ADD_DU_AVG, KID_IMPLICIT, k_add_du<true>, BLK, 0, sw);
   HIPCHK(hipGetLastError());
 }
@@ -4277,7 +4552,7 @@ void launch_implicit(Launcher &L, double beta) {
   StageW sw{};
   sw.beta = beta;
   launch_col5<false>(L, K_IMPL, sw);
-  launch(L, K_IMPL3, KID_IMPLICIT, k_implicit3<false>, 64, 0, sw);
+  launch_col3<false>(L, K_IMPL3, sw);
   launch(L, K_ADD_DU, KID_IMPLICIT, k_add_du<false>, BLK, 0, sw);
   HIPCHK(hipGetLastError());
 }

@@ -1,8 +1,9 @@
 """The column solves within and outside a stage against the oracle, bit for bit:
-level counts that leave every remainder of the three levels a piece of the
-backward sweep holds, panels whose columns leave a remainder in the last block of
-64, and both sides of the number of blocks (two a CU) from which the 5x5 solve
-takes one wave a block instead of two."""
+level counts that leave remainders of the three (5x5) and six (3x3) levels a
+piece of the backward sweep holds and of the two levels the 3x3 assembly takes
+at once, panels whose columns leave a remainder in the last block of
+64, and both sides of the number of blocks (two a CU) above which a block has one
+wave instead of several."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("implicit", [9, 1])
-@pytest.mark.parametrize("nx, nx1", [(4, 3), (4, 4), (6, 5), (8, 6), (10, 17), (72, 4), (74, 3),
+@pytest.mark.parametrize("nx, nx1", [(4, 3), (4, 4), (6, 5), (8, 6), (10, 17), (4, 8), (6, 10), (72, 4), (74, 3),
                                      (74, 5)])
 def test_column_solve_is_the_oracles(ex, orc, nx, nx1, implicit):
     cfg = atm_config(ex, nx=nx, nx1=nx1, implicit=implicit)
