@@ -168,6 +168,7 @@ __device__ __forceinline__ DState to_global(const State &h) {
 }
 
 constexpr int BLK = 256;
+constexpr int MAXNT = 4;  // passive scalars a configuration may have
 
 // Remap tables of an instance, made on the host from its descriptors: by ghost
 // cell [panel][side][depth][along] and by edge face [panel][side][along], each
@@ -453,7 +454,7 @@ struct GhostCell {
   int polar;
 };
 
-__device__ __forceinline__ GhostCell ghost_cell(const Inst &I, int q, bool vectors) {
+__device__ __forceinline__ GhostCell ghost_cell(const Inst &I, int q) {
   const ADDR(1) double *t = glb(I.gt) + q;
   const ADDR(1) int *ti = glb(I.gi) + q;
   size_t n = I.ngd;
@@ -464,15 +465,13 @@ __device__ __forceinline__ GhostCell ghost_cell(const Inst &I, int q, bool vecto
   c.yD = t[GT_YD * n];
   c.o0 = (unsigned)ti[GI_SRC0 * n];
   c.o1 = (unsigned)ti[GI_SRC1 * n];
-  if (vectors) {
-    c.sth = t[GT_STH * n];
-    c.ysth = t[GT_YSTH * n];
-    c.cths = t[GT_CTH * n];
-    c.ctht = t[GT_CTHT * n];
+  c.sth = t[GT_STH * n];
+  c.ysth = t[GT_YSTH * n];
+  c.cths = t[GT_CTH * n];
+  c.ctht = t[GT_CTHT * n];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) c.m[e] = t[(GT_MAP + e) * n];
-    c.polar = ti[GI_POLAR * n];
-  }
+  for (int e = 0; e < 8; ++e) c.m[e] = t[(GT_MAP + e) * n];
+  c.polar = ti[GI_POLAR * n];
   return c;
 }
 
@@ -523,47 +522,55 @@ __device__ __forceinline__ bool edge_thread(const DGrid &g, int nrow, int lb, in
 // the edge, whole lines.  6 x 96 x 96 x 64: 41 us a stage, 44 with lanes along
 // the levels everywhere and the maps' square roots and quotients in the kernel;
 // three depths or four levels a thread 54 and 45 us (fewer wavefronts).
-__device__ __forceinline__ void ghost_body(const DGrid &g, int lb, const Inst &I,
-                                           ADDR(1) double *arr, int nvar, bool vectors) {
+// The passive scalars take the same sources and weights and go along: a launch of
+// their own read the tables again and, on small spheres, cost its latency (6 x 26
+// x 26 x 19 with a tracer 10.8 -> 6.6 us a stage, 6 x 96 x 96 x 64 with two 58 ->
+// 57).
+__device__ __forceinline__ void ghost_body(const DGrid &g, const DState &st, int lb,
+                                           const Inst &I) {
   unsigned t = (unsigned)lb * BLK + threadIdx.x, N = g.N, ni = g.nx1;
   if (t >= (unsigned)I.ngd * ni) return;
   unsigned ps = t / (NG * N * ni), r = t - ps * (NG * N * ni);
   int p = (int)(ps / 4), side = (int)(ps % 4);
   unsigned f = side < 2 ? ni : N, q = r / f, lo = r - q * f, hi = q / NG;
   int d = (int)(q - hi * NG), a = (int)(side < 2 ? hi : lo), i = g.is + (int)(side < 2 ? lo : hi);
-  GhostCell c = ghost_cell(I, (int)((ps * NG + d) * N) + a, vectors);
+  GhostCell c = ghost_cell(I, (int)((ps * NG + d) * N) + a);
   int k, j;
   edge_cell(g, side, d, a, k, j);
   size_t ot = g.c(0, p, k, i, j), up = (size_t)i * g.jp, o0 = c.o0 + up, o1 = c.o1 + up;
   // every value is loaded before the first is stored (the compiler must take a
   // store for one that a later load may read)
-  double v0[5], v1[5];
+  double v0[5], v1[5], s0[MAXNT], s1[MAXNT];
 #pragma unroll
   for (int n = 0; n < 5; ++n) {
-    if (n >= nvar || (vectors && g.skipv(n))) continue;
-    v0[n] = arr[n * g.vstride + o0];
-    v1[n] = arr[n * g.vstride + o1];
+    if (g.skipv(n)) continue;
+    v0[n] = st.u[n * g.vstride + o0];
+    v1[n] = st.u[n * g.vstride + o1];
+  }
+#pragma unroll
+  for (int n = 0; n < MAXNT; ++n) {
+    if (n >= g.nt) continue;
+    s0[n] = st.s[n * g.vstride + o0];
+    s1[n] = st.s[n * g.vstride + o1];
   }
 #pragma unroll
   for (int n = 0; n < 5; ++n) {
-    if (n >= nvar || (vectors && (n == IVY || n == IVZ || g.skipv(n)))) continue;
-    arr[n * g.vstride + ot] = ghost_scalar(c, v0[n], v1[n]);
+    if (n == IVY || n == IVZ || g.skipv(n)) continue;
+    st.u[n * g.vstride + ot] = ghost_scalar(c, v0[n], v1[n]);
   }
-  if (vectors) {
-    double vy, vz;
-    ghost_vector(c, v0[IVY], v0[IVZ], v1[IVY], v1[IVZ], vy, vz);
-    arr[IVY * g.vstride + ot] = vy;
-    arr[IVZ * g.vstride + ot] = vz;
-  }
+  double vy, vz;
+  ghost_vector(c, v0[IVY], v0[IVZ], v1[IVY], v1[IVZ], vy, vz);
+  st.u[IVY * g.vstride + ot] = vy;
+  st.u[IVZ * g.vstride + ot] = vz;
+#pragma unroll
+  for (int n = 0; n < MAXNT; ++n)
+    if (n < g.nt) st.s[n * g.vstride + ot] = ghost_scalar(c, s0[n], s1[n]);
 }
 
-// which = 0: conserved variables (vectors remapped), 1: passive scalars
-__global__ void __launch_bounds__(BLK) k_ghost(const Inst *__restrict__ I_, Work w, int which) {
+__global__ void __launch_bounds__(BLK) k_ghost(const Inst *__restrict__ I_, Work w) {
   WORK_LOOP(w) {
     WORK_INST(w);
-    const Inst &I = I_[ii_];
-    if (which == 0) ghost_body(g, lb, I, st.u, g.nv, true);
-    else ghost_body(g, lb, I, st.s, g.nt, false);
+    ghost_body(g, st, lb, I_[ii_]);
   }
 }
 
@@ -1123,7 +1130,7 @@ struct RegFlux {
   const double *x2l, *x2r, *x1l, *x1r, *s2l, *s2r;
   const float *f2l, *f2r, *fs2l, *fs2r;
 };
-constexpr int RF_NT = 4;  // scalars register fluxes carry (the configuration's maximum)
+constexpr int RF_NT = MAXNT;  // scalars register fluxes carry (the configuration's maximum)
 
 // X2R: the fluxes of rf come from the caller's registers instead of the flux
 // arrays (FP64: x2, x1 and the scalars' x2; mixed: the FP32 x2 and scalar x2
@@ -3620,7 +3627,7 @@ __device__ __forceinline__ void sw_halo_body(const DGrid &g, const DState &st, i
   double v0[NG][3], v1[NG][3], cg[NG], in[NG][3], ci[NG];
 #pragma unroll
   for (int depth = 0; depth < NG; ++depth) {
-    gc[depth] = ghost_cell(I, ((p * 4 + side) * NG + depth) * g.N + a, true);
+    gc[depth] = ghost_cell(I, ((p * 4 + side) * NG + depth) * g.N + a);
     size_t o0 = (size_t)gc[depth].o0 + (size_t)i * g.jp;
     size_t o1 = (size_t)gc[depth].o1 + (size_t)i * g.jp;
     int k, j;
@@ -3991,7 +3998,7 @@ int kind_blocks(int kind, const Grid &g, bool mixed, int ngd, int ned, bool step
     case K_PRIM_REST: return ideal ? (int)grid1((size_t)6 * g.nc3 * g.nx1 * g.nc2) : 0;
     case K_PRIM_GHOST: return !ideal ? (int)grid1((size_t)6 * 4 * NG * g.N * g.nx1) : 0;
     case K_GHOST_U: return (int)grid1((size_t)ngd * g.nx1);
-    case K_GHOST_S: return g.nt ? (int)grid1((size_t)ngd * g.nx1) : 0;
+    case K_GHOST_S: return 0;  // the scalars go with K_GHOST_U
     case K_X1: return ideal && !mixed ? (int)grid1(cols, x1c) * 6 : 0;
     case K_X1_MIX: return ideal && mixed ? (int)grid1(cols, 64) * 6 : 0;
     // mixed shallow water takes FP64 edge states (its faces are taken about an
@@ -4398,8 +4405,7 @@ void launch_prim(Launcher &L, int kid) {
 }
 
 void launch_fill_ghosts(Launcher &L) {
-  launch(L, K_GHOST_U, KID_GHOST, k_ghost, BLK, 0, 0);
-  launch(L, K_GHOST_S, KID_GHOST, k_ghost, BLK, 0, 1);
+  launch(L, K_GHOST_U, KID_GHOST, k_ghost, BLK, 0);
   launch_prim(L, KID_PRIM);
   HIPCHK(hipGetLastError());
 }
@@ -4579,8 +4585,7 @@ void launch_dt(Launcher &L, double dt_fixed) {
 // ghost fill within a step: the stage update has written the primitive state
 // of the interior cells of shallow-water instances
 void launch_fill_ghosts_stage(Launcher &L) {
-  launch(L, K_GHOST_U, KID_GHOST, k_ghost, BLK, 0, 0);
-  launch(L, K_GHOST_S, KID_GHOST, k_ghost, BLK, 0, 1);
+  launch(L, K_GHOST_U, KID_GHOST, k_ghost, BLK, 0);
   launch(L, K_PRIM_REST, KID_PRIM, k_prim<EOS_IDEAL>, BLK, 0, DFLOOR, SFLOOR);
   launch(L, K_PRIM_GHOST, KID_PRIM, k_prim_ghost, BLK, 0, DFLOOR, SFLOOR);
   HIPCHK(hipGetLastError());
@@ -4669,7 +4674,7 @@ void tune_launcher(Launcher &L, int reps) {
           if (kind != K_PRIM) launch_prim(L, -1);
           switch (kind) {
             case K_PRIM: launch_prim(L, -1); break;
-            case K_GHOST_U: launch(L, K_GHOST_U, -1, k_ghost, BLK, 0, 0); break;
+            case K_GHOST_U: launch(L, K_GHOST_U, -1, k_ghost, BLK, 0); break;
             case K_X1: launch_x1(L, K_X1, -1); break;
             case K_X1_MIX: launch_x1(L, K_X1_MIX, -1); break;
             case K_EDGE: launch(L, K_EDGE, -1, k_edge_states, BLK, 0); break;
