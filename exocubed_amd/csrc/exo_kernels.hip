@@ -1478,8 +1478,11 @@ __device__ __forceinline__ void face2_update_body(const DGrid &g, const DState &
 // At most four wavefronts a SIMD: it waits for memory more than it issues, and for
 // a fifth the compiler gives up registers, and with them loads in flight (the
 // mixed form on 6 x 64 x 64 x 64, LMARS: 82 registers 89 us, up to 128 76 us).
+// With scalars at least three (the FP64 HLLC form took 189 registers, two a SIMD:
+// 6 x 64 x 64 x 47 with a tracer 130 -> 115 us, 44 B spilled); at four more (the mixed
+// form on 6 x 96 x 96 x 64 with two 328 -> 377 us).
 template <bool SCAL, bool MIX, int RK = -1>
-__global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(SCAL ? 2 : 4, 4)))
+__global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(SCAL ? 3 : 4, 4)))
 k_face2_update(const Inst *__restrict__ I_, Work w, StageW sw) {
   WORK_LOOP(w) {
     WORK_INST(w);
