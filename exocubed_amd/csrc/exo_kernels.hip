@@ -4641,10 +4641,32 @@ void launch_sums(Launcher &L, double *out) {
   HIPCHK(hipGetLastError());
 }
 
+// The time-step state of every instance of a launcher, put back when the
+// tuner ends or throws: k_dt writes it, and run again and again it would double
+// the previous dt, which bounds the next step's growth, away.
+struct KeepTimeStep {
+  Launcher &L;
+  std::vector<double> v;
+  explicit KeepTimeStep(Launcher &l) : L(l), v((size_t)2 * l.ninst) {
+    for (int i = 0; i < L.ninst; ++i)
+      HIPCHK(hipMemcpyAsync(&v[2 * i], L.h_inst[i].st.dtv, 2 * sizeof(double),
+                            hipMemcpyDeviceToHost, L.stream));
+    HIPCHK(hipStreamSynchronize(L.stream));
+  }
+  ~KeepTimeStep() {
+    for (int i = 0; i < L.ninst; ++i)
+      (void)hipMemcpyAsync(L.h_inst[i].st.dtv, &v[2 * i], 2 * sizeof(double),
+                           hipMemcpyHostToDevice, L.stream);
+    (void)hipStreamSynchronize(L.stream);
+  }
+};
+
 // Autotuner of the persistent launch width: for each launch kind that only
-// reads the conserved state (so repeating it changes nothing), time each
-// candidate width and keep the fastest.  Widths are multiples of the CU count.
+// reads the conserved state (so repeating it changes nothing; the CFL minimum
+// also writes the time-step state, which is put back), time each candidate
+// width and keep the fastest.  Widths are multiples of the CU count.
 void tune_launcher(Launcher &L, int reps) {
+  const KeepTimeStep keep(L);
   const int ncu = L.ncu;
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
