@@ -177,7 +177,7 @@ constexpr int MAXNT = 4;  // passive scalars a configuration may have
 // here from the descriptor's tangents with the maps' own expressions
 // (vec_rll_from_abp, vec_abp_from_rll), they leave the kernels a few products
 // where each map took four square roots and four to eight divisions.
-enum { GT_A = 0, GT_B, GT_D, GT_YD, GT_STH, GT_YSTH, GT_CTH, GT_CTHT, GT_MAP, GT_N = GT_MAP + 8 };
+enum { GT_A = 0, GT_B, GT_D, GT_STH, GT_CTH, GT_CTHT, GT_MAP, GT_N = GT_MAP + 8 };
 enum { GI_SRC0 = 0, GI_SRC1, GI_POLAR, GI_N };  // elements of variable 0, level 0
 enum { ET_MAP = 0, ET_N = 8 };
 enum { EI_SLOT = 0, EI_POLAR, EI_N };  // slot: target (panel * 4 + side) * 2^16 + along
@@ -449,7 +449,7 @@ __global__ void __launch_bounds__(BLK) k_prim_ghost(const Inst *__restrict__ I_,
 // cubed_sphere_utility.cpp:92-617): one thread per (ghost cell, i); the
 // descriptor carries the interpolation weights and vector-map points.
 struct GhostCell {
-  double A, B, D, yD, sth, ysth, cths, ctht, m[8];
+  double A, B, D, sth, cths, ctht, m[8];
   unsigned o0, o1;  // an instance that fits the memory has fewer than 2^31 elements a variable
   int polar;
 };
@@ -462,11 +462,9 @@ __device__ __forceinline__ GhostCell ghost_cell(const Inst &I, int q) {
   c.A = t[GT_A * n];
   c.B = t[GT_B * n];
   c.D = t[GT_D * n];
-  c.yD = t[GT_YD * n];
   c.o0 = (unsigned)ti[GI_SRC0 * n];
   c.o1 = (unsigned)ti[GI_SRC1 * n];
   c.sth = t[GT_STH * n];
-  c.ysth = t[GT_YSTH * n];
   c.cths = t[GT_CTH * n];
   c.ctht = t[GT_CTHT * n];
 #pragma unroll
@@ -475,15 +473,19 @@ __device__ __forceinline__ GhostCell ghost_cell(const Inst &I, int q) {
   return c;
 }
 
+// qdiv, not div_rn: a cell's state may hold infinities, which have to reach the
+// neighbour (div_rn makes NaNs of them, and the depth floor would hide those).
+// The quotients of one divisor share its reciprocal, and the time is the same: a
+// step of 6 x 24 x 24 or 6 x 48 x 48 x 3 shallow water within 1 % of div_rn's.
 __device__ __forceinline__ double ghost_scalar(const GhostCell &c, double v1, double v2) {
-  return div_rn(c.A * v1 + c.B * v2, c.D, c.yD);
+  return qdiv(c.A * v1 + c.B * v2, c.D);
 }
 
 // the covariant x2 / x3 components of a ghost cell from the two source cells
 __device__ __forceinline__ void ghost_vector(const GhostCell &c, double v1y, double v1z, double v2y,
                                              double v2z, double &vy, double &vz) {
   double y = ghost_scalar(c, v1y, v2y), z = ghost_scalar(c, v1z, v2z);
-  auto by2 = [&](double v) { return div_rn(div_rn(v, c.sth, c.ysth), c.sth, c.ysth); };
+  auto by2 = [&](double v) { return qdiv(qdiv(v, c.sth), c.sth); };
   double cy = by2(y) - by2(z * c.cths), cz = by2(z) - by2(y * c.cths);
   double ty, tz;
   frame_map(c.m, c.polar, cy, cz, ty, tz);
@@ -4289,8 +4291,8 @@ RemapTables remap_tables(const Setup &s, const Grid &g) {
     int lo = x2 ? g.js : g.ks, hi = x2 ? g.je : g.ke;
     int side = (x2 ? 0 : 2) + (at > hi ? 1 : 0), depth = at > hi ? at - hi - 1 : lo - 1 - at;
     size_t q = ((size_t)(d.tgt_panel * 4 + side) * NG + depth) * g.N + along;
-    const double v[8] = {d.A, d.B, d.D, 1.0 / d.D, d.sth_s, 1.0 / d.sth_s, d.cth_s, d.cth_t};
-    for (int e = 0; e < 8; ++e) r.gt[(GT_A + e) * ng + q] = v[e];
+    const double v[GT_MAP] = {d.A, d.B, d.D, d.sth_s, d.cth_s, d.cth_t};
+    for (int e = 0; e < GT_MAP; ++e) r.gt[(GT_A + e) * ng + q] = v[e];
     r.gi[GI_POLAR * ng + q] =
         map_factors(d.src_cy, d.src_cz, d.src_block, d.tgt_cy, d.tgt_cz, d.tgt_block, m);
     for (int e = 0; e < 8; ++e) r.gt[(GT_MAP + e) * ng + q] = m[e];
