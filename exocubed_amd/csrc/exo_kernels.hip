@@ -3340,17 +3340,25 @@ __global__ void __launch_bounds__(BLK) k_flux_h_mix(const Inst *__restrict__ I_,
 //     and by a block's latency: 6 x 48 x 48 x 3 takes 75 us a step instead of
 //     109, 6 x 24 x 24 80 instead of 115.
 //   * Large ones moved some 270 bytes a cell and stage (face fluxes out and in,
-//     u, u1 and w); here a stage reads its input (24 bytes) and, in stages 2
-//     and 3, the step's first state (24), writes 24, and reads 100 bytes of
-//     tables.  What is left is FP64 issue: 56 spheres of 24 to 182 cells a side
+//     u, u1 and w); here a stage has to read its input (24 bytes) and the
+//     primitive state (stage 1) or the step's first state (24), writes 24, and
+//     reads 100 bytes of tables.  What is left is FP64 issue: 56 spheres of 24 to 182 cells a side
 //     (2.3 M cells, Roe) take 0.84 ms a step instead of 1.04, the stage kernel
 //     0.217 ms, 0.17 of it the issue of its instructions.
-// A stage reads u and converts it on the way into LDS (12 % of the cells twice
-// or more, the tiles' margins), so the primitive state is written only by the
-// last one.  No stage may write what its neighbours' tiles read: stage 1 goes
+// Stages 2 and 3 convert u on the way into LDS (a tile its own 240 cells and up
+// to 186 of its neighbours': 1.5 to 1.75 conversions a cell), so the primitive
+// state is written only by the last one and read only by the first.  No stage
+// may write what its neighbours' tiles read: stage 1 goes
 // from u to u1, 2 from u1 to du, 3 from du back to u, which stages 2 and 3 read
 // at their own cell only, as the step's first state (SSPRK3's u1).  (du is
 // unused by shallow water otherwise; outside a step u1 is the stage register.)
+// The last stage of a call's last step (SW_LAST) leaves what the single phases
+// leave, for calls that follow: its face fluxes and, in u1, the step's first
+// state.  Within a call nobody reads them, and they are 72 bytes a cell: a single
+// step of 6 x 1024 x 1024, mixed, takes 1.32 ms with them and 1.22 without.  The
+// first stage takes the primitive state from memory, not from u, as the single
+// phases do: it may be older than u (no ghost fill since an update of u), and
+// then both panels of an edge face still see the same states.
 // A tile is 16 x 15 cells: its 511 faces are one for each of 512 threads or two
 // for each of 256, without a nearly empty pass after them (a 16 x 16 tile has
 // 544; it ran at 0.225 ms a stage of the batch above against 0.218, 32 x 7 cells
@@ -3364,6 +3372,9 @@ struct SwLds {
   double f3[3][SWTK + 1][SWTJ];          // x3 faces, the upper edge's included
 };
 __device__ __forceinline__ int sw_var(int q) { return q == 0 ? IDN : q == 1 ? IVY : IVZ; }
+
+// a step's first stage, its later ones, and the last of a call's last step
+enum { SW_FIRST, SW_LATER, SW_LAST };
 
 __device__ __forceinline__ ADDR(1) double *sw_in(const DState &st, int stage) {
   return stage == 0 ? st.u : stage == 1 ? st.u1 : st.du;
@@ -3493,7 +3504,7 @@ __device__ __forceinline__ void sw_coriolis(const DGrid &g, int p, int k, int j,
   out[IVZ] += s * (acc3 + acc2 * cth);
 }
 
-template <bool MIX, int RK, int NT>
+template <bool MIX, int RK, int NT, int PART>
 __device__ __forceinline__ void sw_stage_body(const DGrid &g, const DState &st, int lb,
                                               const StageW &sw, int stage, SwLds &l) {
   int N = g.N, ntj = (N + SWTJ - 1) / SWTJ, ntk = (N + SWTK - 1) / SWTK, ni = g.nx1;
@@ -3503,9 +3514,11 @@ __device__ __forceinline__ void sw_stage_body(const DGrid &g, const DState &st, 
   int i = g.is + r % ni, p = r / ni;
   int j0 = g.js + tj * SWTJ, k0 = g.ks + tk * SWTK;
   const int tid = threadIdx.x;
-  const ADDR(1) double *in = sw_in(st, stage);
-  ADDR(1) double *outp = sw_out(st, stage);
+  constexpr bool FIRST = PART == SW_FIRST;
+  const ADDR(1) double *in = FIRST ? st.u : sw_in(st, stage);
+  ADDR(1) double *outp = FIRST ? st.u1 : PART == SW_LAST ? st.u : sw_out(st, stage);
   size_t vs = g.vstride;
+  const ADDR(1) double *src = FIRST ? st.w : in;
   // the tile and its margins into LDS, one cell a thread: the tile, then left
   // and right, then lower and upper.  Cells past the panel's ghosts are no
   // stencil's, nor are the corners.
@@ -3523,8 +3536,8 @@ __device__ __forceinline__ void sw_stage_body(const DGrid &g, const DState &st, 
     int j = j0 + x, k = k0 + y;
     if (j < g.nc2 && k < g.nc3) {
       size_t c = g.c(0, p, k, i, j);
-      double h = in[IDN * vs + c], w2, w3;
-      sw_prim(h, in[IVY * vs + c], in[IVZ * vs + c], g.T(T_COSC, p, k, j), sw.dfloor, w2, w3);
+      double h = src[IDN * vs + c], w2 = src[IVY * vs + c], w3 = src[IVZ * vs + c];
+      if (!FIRST) sw_prim(h, w2, w3, g.T(T_COSC, p, k, j), sw.dfloor, w2, w3);
       l.w[0][y + NG][x + NG] = h;
       l.w[1][y + NG][x + NG] = w2;
       l.w[2][y + NG][x + NG] = w3;
@@ -3546,6 +3559,12 @@ __device__ __forceinline__ void sw_stage_body(const DGrid &g, const DState &st, 
       for (int q = 0; q < 3; ++q) {
         if (x3) l.f3[q][y][x] = fl[q];
         else l.f2[q][y][x] = fl[q];
+      }
+      // of a face between two tiles the one it is the first face of stores it
+      if (PART == SW_LAST && (x3 ? y < SWTK || k > g.ke : x < SWTJ || j > g.je)) {
+        ADDR(1) double *F = x3 ? st.flx[2] : st.flx[1];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) F[g.f(sw_var(q), p, k, i, j)] = fl[q];
       }
     }
   }
@@ -3573,8 +3592,9 @@ __device__ __forceinline__ void sw_stage_body(const DGrid &g, const DState &st, 
   for (int q = 0; q < 3; ++q) {
     int n = sw_var(q);
     // the stage register of the step's first state is 0 + u
-    double uv = in[n * vs + c];
-    double u = sw.first ? 0. + uv : sw.g1 * uv + sw.g2 * (0. + st.u[n * vs + c]);
+    double uv = in[n * vs + c], u1 = 0. + (FIRST ? uv : st.u[n * vs + c]);
+    double u = FIRST ? u1 : sw.g1 * uv + sw.g2 * u1;
+    if (PART == SW_LAST) st.u1[n * vs + c] = u1;
     double dflx = 0.;
     dflx += geo.a2r * l.f2[q][y][x + 1] - geo.a2l * l.f2[q][y][x];
     dflx += geo.a3r * l.f3[q][y + 1][x] - geo.a3l * l.f3[q][y][x];
@@ -3594,25 +3614,27 @@ __device__ __forceinline__ void sw_stage_body(const DGrid &g, const DState &st, 
   outp[IDN * vs + c] = h;  // with the floor, as the conversion writes it back
   outp[IVY * vs + c] = out[IVY];
   outp[IVZ * vs + c] = out[IVZ];
-  if (stage == 2) {
+  if (!FIRST && stage == 2) {
     st.w[IDN * vs + c] = h;
     st.w[IVY * vs + c] = w2;
     st.w[IVZ * vs + c] = w3;
   }
 }
 
-// RK: the Riemann solver of every instance of the launch, or -1.  NT: threads,
+// RK: the Riemann solver of every instance of the launch, or -1.  PART: SW_*; each
+// is a kernel of its own, as one for all three takes 99 to 103 registers where
+// five wavefronts a SIMD leave 96 (6 x 384 x 384 mixed 207 -> 216 us a step).  NT: threads,
 // 512 for launches that leave CUs without a tile, where a block's latency is
 // what counts (6 x 48 x 48 x 3, 216 tiles: 12.0 against 13.6 us, event times),
 // else 256, four blocks a CU in different phases (6 x 192 x 192 mixed, 936
 // tiles: 21.9 against 23.4 us; the batch 0.218 against 0.298 ms).
-template <bool MIX, int RK, int NT>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
+template <bool MIX, int RK, int NT, int PART>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 512 ? 4 : 5)))
 k_sw_stage(const Inst *__restrict__ I_, Work w, StageW sw, int stage) {
   __shared__ SwLds l;
   WORK_LOOP(w) {
     WORK_INST(w);
-    sw_stage_body<MIX, RK, NT>(g, st, lb, sw, stage, l);
+    sw_stage_body<MIX, RK, NT, PART>(g, st, lb, sw, stage, l);
     __syncthreads();  // the tile is refilled by the next block of the loop
   }
 }
@@ -4606,23 +4628,33 @@ void run_stage(Launcher &L, int stage) {
 }
 
 // one stage of the shallow-water instances whose step is k_sw_stage's (mode 1)
-void launch_sw(Launcher &L, int stage) {
+// last: of the last step of a call
+void launch_sw(Launcher &L, int stage, bool last) {
   int s0 = stage - 1;
   StageW sw{SS_DELTA[s0], SS_G1[s0], SS_G2[s0], SS_BETA[s0], s0 == 0 ? 1 : 0, 1, DFLOOR, SFLOOR};
   with_solver<EOS_SW>(L, [&](auto R) {
     constexpr int RK = decltype(R)::value;
-    if (L.nblk[1][K_SW] <= L.ncu)
-      launch(L, K_SW, KID_UPDATE, k_sw_stage<false, RK, 512>, 512, 0, sw, s0);
-    else launch(L, K_SW, KID_UPDATE, k_sw_stage<false, RK, 256>, 256, 0, sw, s0);
-    if (L.nblk[1][K_SW_MIX] <= L.ncu)
-      launch(L, K_SW_MIX, KID_UPDATE, k_sw_stage<true, RK, 512>, 512, 0, sw, s0);
-    else launch(L, K_SW_MIX, KID_UPDATE, k_sw_stage<true, RK, 256>, 256, 0, sw, s0);
+    auto tiles = [&](auto K) {
+      constexpr int PART = decltype(K)::value;
+      if (L.nblk[1][K_SW] <= L.ncu)
+        launch(L, K_SW, KID_UPDATE, k_sw_stage<false, RK, 512, PART>, 512, 0, sw, s0);
+      else launch(L, K_SW, KID_UPDATE, k_sw_stage<false, RK, 256, PART>, 256, 0, sw, s0);
+      if (L.nblk[1][K_SW_MIX] <= L.ncu)
+        launch(L, K_SW_MIX, KID_UPDATE, k_sw_stage<true, RK, 512, PART>, 512, 0, sw, s0);
+      else launch(L, K_SW_MIX, KID_UPDATE, k_sw_stage<true, RK, 256, PART>, 256, 0, sw, s0);
+    };
+    if (stage == 1) tiles(std::integral_constant<int, SW_FIRST>{});
+    else if (stage == 3 && last) tiles(std::integral_constant<int, SW_LAST>{});
+    else tiles(std::integral_constant<int, SW_LATER>{});
   });
   launch(L, K_SW_HALO, KID_GHOST, k_sw_halo, BLK, 0, DFLOOR, s0);
   HIPCHK(hipGetLastError());
 }
 
-void run_step(Launcher &L, double dt_fixed) {
+// last: the call's last step, after which the last stage's fluxes and the stage
+// register are there (k_sw_stage leaves them only then; every other kernel does
+// always).
+void run_step(Launcher &L, double dt_fixed, bool last) {
   struct Mode {  // back to the single phases' work list also when a launch throws
     Launcher &L;
     explicit Mode(Launcher &l) : L(l) { L.mode = 1; }
@@ -4631,9 +4663,12 @@ void run_step(Launcher &L, double dt_fixed) {
   launch_dt(L, dt_fixed);
   for (int stg = 1; stg <= 3; ++stg) {
     run_stage(L, stg);
-    launch_sw(L, stg);
+    launch_sw(L, stg, last);
   }
 }
+
+// whether the last step of a call differs from those before it
+bool last_differs(const Launcher &L) { return L.nblk[1][K_SW] + L.nblk[1][K_SW_MIX] > 0; }
 
 // compensated conserved totals of every instance into out[ninst][5] (device)
 void launch_sums(Launcher &L, double *out) {
@@ -5146,7 +5181,7 @@ void handle_graph(exo_handle *h, double dt_fixed) {
   h->graph = nullptr;
   HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
   try {
-    run_step(h->L, dt_fixed);
+    run_step(h->L, dt_fixed, false);
   } catch (...) {
     hipGraph_t gr = nullptr;
     (void)hipStreamEndCapture(h->stream, &gr);
@@ -5239,9 +5274,11 @@ int exo_step(exo_handle *h, int nsteps, double dt_fixed, double *dt_last) {
     if (!h->have_state) throw std::string("no state uploaded");
     if (nsteps > 1 && !h->L.prof) {  // replay a captured step (no per-kernel timing)
       handle_graph(h, dt_fixed);
-      for (int s = 0; s < nsteps; ++s) HIPCHK(hipGraphLaunch(h->exec, h->stream));
+      int replays = nsteps - (last_differs(h->L) ? 1 : 0);
+      for (int s = 0; s < replays; ++s) HIPCHK(hipGraphLaunch(h->exec, h->stream));
+      if (replays < nsteps) run_step(h->L, dt_fixed, true);
     } else {
-      for (int s = 0; s < nsteps; ++s) run_step(h->L, dt_fixed);
+      for (int s = 0; s < nsteps; ++s) run_step(h->L, dt_fixed, s == nsteps - 1);
     }
     if (dt_last) {
       double v[2];
@@ -5289,9 +5326,9 @@ int exo_step_redo(exo_handle *h, int nsteps, int max_redo, double *dt_last, int 
         // next step may grow to twice it (Mesh::NewTimeStep)
         double v[2] = {dt_redo, dt_redo};
         HIPCHK(hipMemcpyAsync(h->st.dtv, v, sizeof(v), hipMemcpyHostToDevice, h->stream));
-        run_step(h->L, dt_redo);
+        run_step(h->L, dt_redo, done == nsteps - 1);
       } else {
-        run_step(h->L, 0.0);
+        run_step(h->L, 0.0, done == nsteps - 1);
       }
       if (max_redo > 0) {
         if (state_valid(h)) {
@@ -5841,12 +5878,13 @@ int exo_batch_step(exo_batch *b, int nsteps, double dt_fixed) {
   return guarded(b, [&] {
     if (nsteps < 0) throw std::string("nsteps must be >= 0");
     batch_ready(b);
-    if (b->use_graph && !b->L.prof) {
+    int replays = nsteps - (last_differs(b->L) ? 1 : 0);
+    if (b->use_graph && !b->L.prof && replays > 0) {
       if (!b->exec || b->graph_dt_fixed != dt_fixed) {
         batch_free_graph(b);
         HIPCHK(hipStreamBeginCapture(b->L.stream, hipStreamCaptureModeThreadLocal));
         try {
-          run_step(b->L, dt_fixed);
+          run_step(b->L, dt_fixed, false);
         } catch (...) {
           hipGraph_t gr = nullptr;
           (void)hipStreamEndCapture(b->L.stream, &gr);
@@ -5857,9 +5895,10 @@ int exo_batch_step(exo_batch *b, int nsteps, double dt_fixed) {
         HIPCHK(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
         b->graph_dt_fixed = dt_fixed;
       }
-      for (int s = 0; s < nsteps; ++s) HIPCHK(hipGraphLaunch(b->exec, b->L.stream));
+      for (int s = 0; s < replays; ++s) HIPCHK(hipGraphLaunch(b->exec, b->L.stream));
+      if (replays < nsteps) run_step(b->L, dt_fixed, true);
     } else {
-      for (int s = 0; s < nsteps; ++s) run_step(b->L, dt_fixed);
+      for (int s = 0; s < nsteps; ++s) run_step(b->L, dt_fixed, s == nsteps - 1);
     }
     HIPCHK(hipStreamSynchronize(b->L.stream));
   });

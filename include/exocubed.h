@@ -101,7 +101,10 @@ EXO_API int exo_download_prim(exo_handle *h, double *w);
 EXO_API int exo_calc_fluxes(exo_handle *h);
 /* Copy the face fluxes of direction dir (0 = x1, 1 = x2, 2 = x3) to the host in
  * Athena's flux layout: x1 (NVAR, nc3, nc2, nc1+1), x2 (NVAR, nc3, nc2+1, nc1),
- * x3 (NVAR, nc3+1, nc2, nc1) per panel; only interior faces are defined. */
+ * x3 (NVAR, nc3+1, nc2, nc1) per panel; only interior faces are defined.
+ * They are those of the last exo_calc_fluxes, exo_stage or step (its last
+ * stage); the ideal gas's x2 fluxes those of the last exo_calc_fluxes, as a
+ * stage takes them up where they are formed. */
 EXO_API int exo_download_flux(exo_handle *h, int dir, double *out);
 /* Hydro::AddFluxDivergence(wght, u) followed by
  * GnomonicEquiangle::AddCoordTermsDivergence (gnomonic_equiangle.cpp:834-879)
