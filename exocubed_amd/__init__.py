@@ -30,12 +30,14 @@ LAUNCH_KINDS = ("prim", "ghost_u", "ghost_s", "x1", "x1_mix", "edge", "edge_mix"
                 "add_du_avg", "face2_update", "face_x2", "face2_update_s",
                 "face2_update_mix", "face2_update_mix_s", "sw_stage", "sw_stage_mix", "sw_halo",
                 "sw_edge")
+NKINDS = 30  # EXO_NKINDS: kinds with a shape; the others' widths follow the shapes
+NTUNED = NKINDS + len(LAUNCH_KINDS)
 
 
 def _tuning(caps):
-    n = len(LAUNCH_KINDS)
-    out = {k: int(c) for k, c in zip(LAUNCH_KINDS, caps[:n])}
-    out.update({k + "_shape": int(c) for k, c in zip(LAUNCH_KINDS, caps[n:]) if c})
+    out = {k: int(c) for k, c in zip(LAUNCH_KINDS[:NKINDS], caps)}
+    out.update({k: int(c) for k, c in zip(LAUNCH_KINDS[NKINDS:], caps[2 * NKINDS:])})
+    out.update({k + "_shape": int(c) for k, c in zip(LAUNCH_KINDS, caps[NKINDS:2 * NKINDS]) if c})
     return out
 
 
@@ -425,7 +427,7 @@ class Solver:
         """tuned persistent widths per launch kind, and "<kind>_shape" block
         shapes (waves per x1 block, levels per update thread) where not the
         default"""
-        caps = np.zeros(2 * len(LAUNCH_KINDS), dtype=np.int32)
+        caps = np.zeros(NTUNED, dtype=np.int32)
         self._chk(self.L.exo_tune(self.h, reps, caps.ctypes.data_as(C.c_void_p), len(caps)),
                   "exo_tune")
         return _tuning(caps)
@@ -461,14 +463,15 @@ class Batch:
         return out.reshape(len(self.members), 5)
 
     def tune(self, reps=3):
-        caps = np.zeros(2 * len(LAUNCH_KINDS), dtype=np.int32)
+        caps = np.zeros(NTUNED, dtype=np.int32)
         self._chk(self.L.exo_batch_tune(self.h, reps, caps.ctypes.data_as(C.c_void_p),
                                         len(caps)), "exo_batch_tune")
         return _tuning(caps)
 
     def set_caps(self, caps):
-        arr = np.array([caps.get(k, 0) for k in LAUNCH_KINDS] +
-                       [caps.get(k + "_shape", 0) for k in LAUNCH_KINDS], dtype=np.int32)
+        arr = np.array([caps.get(k, 0) for k in LAUNCH_KINDS[:NKINDS]] +
+                       [caps.get(k + "_shape", 0) for k in LAUNCH_KINDS[:NKINDS]] +
+                       [caps.get(k, 0) for k in LAUNCH_KINDS[NKINDS:]], dtype=np.int32)
         self._chk(self.L.exo_batch_set_caps(self.h, arr.ctypes.data_as(C.c_void_p), len(arr)),
                   "exo_batch_set_caps")
 

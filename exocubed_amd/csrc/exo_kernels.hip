@@ -3873,7 +3873,10 @@ __global__ void __launch_bounds__(256) k_layout(Grid g, double *host, double *de
 // handle, many for a batch)
 namespace {
 
-// launch kinds, each with its own block-prefix table over the instances
+// launch kinds, each with its own block-prefix table over the instances; their
+// order is the public one of the tuned arrays (exo_tune), so new ones come
+// last, and K_GHOST_S keeps its place though the scalars' ghosts go with
+// K_GHOST_U (it has no blocks)
 enum {
   K_PRIM = 0, K_GHOST_U, K_GHOST_S, K_X1, K_X1_MIX, K_EDGE, K_EDGE_MIX, K_FACE, K_FACE_MIX,
   K_UPD, K_UPD_MIX, K_IMPL, K_ADD_DU, K_CELLS, K_ONE, K_DT, K_EFLX, K_FACE_MIX_SW,
@@ -4028,7 +4031,7 @@ int kind_blocks(int kind, const Grid &g, bool mixed, int ngd, int ned, bool step
     case K_PRIM_REST: return ideal ? (int)grid1((size_t)6 * g.nc3 * g.nx1 * g.nc2) : 0;
     case K_PRIM_GHOST: return !ideal ? (int)grid1((size_t)6 * 4 * NG * g.N * g.nx1) : 0;
     case K_GHOST_U: return (int)grid1((size_t)ngd * g.nx1);
-    case K_GHOST_S: return 0;  // the scalars go with K_GHOST_U
+    case K_GHOST_S: return 0;
     case K_X1: return ideal && !mixed ? (int)grid1(cols, x1c) * 6 : 0;
     case K_X1_MIX: return ideal && mixed ? (int)grid1(cols, 64) * 6 : 0;
     // mixed shallow water takes FP64 edge states (its faces are taken about an
@@ -4773,7 +4776,6 @@ void tune_launcher(Launcher &L, int reps) {
   }
   // kinds sharing a shape with a tuned one (the other update-shaped kinds keep
   // the plain launch: they rewrite the state and cannot be repeated)
-  L.cap[K_GHOST_S] = L.cap[K_GHOST_U];
   L.cap[K_FACE_NF] = L.cap[K_FACE];
   L.prof = prof;
   HIPCHK(hipEventDestroy(e0));
@@ -5744,7 +5746,14 @@ int exo_conserved_sums(exo_handle *h, double *out5) {
 }  // extern "C"
 
 namespace {
-static_assert(K_NKIND == EXO_NKINDS, "EXO_NKINDS must count the launch kinds");
+// The arrays of exo_tune and exo_batch_set_caps: the widths of the kinds before
+// K_SW, their shapes, then the widths of the kinds from K_SW on, so that an array
+// kept from before these were added means the same.
+static_assert(K_SW == EXO_NKINDS && K_NKIND == EXO_NKINDS + EXO_NKINDS_STEP,
+              "EXO_NKINDS and EXO_NKINDS_STEP must count the launch kinds");
+constexpr int NTUNED = 2 * EXO_NKINDS + EXO_NKINDS_STEP;
+bool tuned_is_shape(int q) { return q >= EXO_NKINDS && q < 2 * EXO_NKINDS; }
+int tuned_kind(int q) { return q < EXO_NKINDS ? q : q - EXO_NKINDS; }
 
 // tuned widths and shapes per configuration of the instances of a launcher
 std::mutex g_tune_mu;
@@ -5765,6 +5774,19 @@ std::string tune_key(const std::vector<exo_handle *> &hs) {
   return k;
 }
 
+void report_tuning(const Launcher &L, int *caps, int ncaps) {
+  for (int q = 0; caps && q < ncaps && q < NTUNED; ++q)
+    caps[q] = (tuned_is_shape(q) ? L.shape : L.cap)[tuned_kind(q)];
+}
+
+void apply_tuning(Launcher &L, const int *caps, int ncaps) {
+  for (int q = 0; q < ncaps && q < NTUNED; ++q) {
+    int v = caps[q] > 0 ? caps[q] : 0;
+    if (tuned_is_shape(q)) set_shape(L, tuned_kind(q), v);
+    else L.cap[tuned_kind(q)] = v;
+  }
+}
+
 // tune a launcher, or apply the result of an earlier tuning of the same
 // configurations
 void tune_cached(Launcher &L, const std::vector<exo_handle *> &hs, int reps) {
@@ -5777,24 +5799,13 @@ void tune_cached(Launcher &L, const std::vector<exo_handle *> &hs, int reps) {
   }
   if (got.empty()) {
     tune_launcher(L, reps);
-    got.assign(2 * K_NKIND, 0);
-    for (int q = 0; q < K_NKIND; ++q) {
-      got[q] = L.cap[q];
-      got[K_NKIND + q] = L.shape[q];
-    }
+    got.resize(NTUNED);
+    report_tuning(L, got.data(), NTUNED);
     std::lock_guard<std::mutex> lock(g_tune_mu);
     g_tune_cache[key] = got;
   } else {
-    for (int q = 0; q < K_NKIND; ++q) {
-      set_shape(L, q, got[K_NKIND + q]);
-      L.cap[q] = got[q];
-    }
+    apply_tuning(L, got.data(), NTUNED);
   }
-}
-
-void report_tuning(const Launcher &L, int *caps, int ncaps) {
-  for (int q = 0; caps && q < ncaps && q < 2 * K_NKIND; ++q)
-    caps[q] = q < K_NKIND ? L.cap[q] : L.shape[q - K_NKIND];
 }
 }  // namespace
 extern "C" {
@@ -5928,11 +5939,7 @@ int exo_batch_set_caps(exo_batch *b, const int *caps, int ncaps) {
   return guarded(b, [&] {
     if (!caps) throw std::string("null caps");
     batch_free_graph(b);
-    for (int q = 0; q < ncaps && q < 2 * K_NKIND; ++q) {
-      int v = caps[q] > 0 ? caps[q] : 0;
-      if (q < K_NKIND) b->L.cap[q] = v;
-      else set_shape(b->L, q - K_NKIND, v);
-    }
+    apply_tuning(b->L, caps, ncaps);
   });
 }
 

@@ -160,14 +160,16 @@ EXO_API int exo_conserved_sums(exo_handle *h, double *out5);
  * state or only write the tendency (repeated launches change nothing): the
  * persistent launch width (the face kernels, the fused x2-face stage update
  * of instances without passive scalars, the primitive conversion, the ghost
- * remap, the CFL minimum), and the x1 sweep's block shape (waves per
- * 64-column block: 2, 4 or 8).
+ * remap, the CFL minimum), and the x1 sweep's block shape (waves per block: 2,
+ * 4 or 8; a block holds 64 columns in the mixed form, 16 or 8 in FP64).
  * Each candidate is timed `reps` times and the fastest kept; a configuration
  * tuned before in this process reuses its result without timing.  caps (may
  * be NULL) receives up to ncaps values: the width of each launch kind (0 = one
- * workgroup per block), then, from index EXO_NKINDS on, its shape (0 = the
- * default). */
-#define EXO_NKINDS 34
+ * workgroup per block), from index EXO_NKINDS on its shape (0 = the default),
+ * and from index 2 * EXO_NKINDS on the widths of the EXO_NKINDS_STEP kinds of
+ * the fused shallow-water step (stage, mixed stage, halo, panel-edge states). */
+#define EXO_NKINDS 30
+#define EXO_NKINDS_STEP 4
 EXO_API int exo_tune(exo_handle *h, int reps, int *caps, int ncaps);
 
 /* Device bytes exo_create allocates for this configuration (host only; 0 for
@@ -198,8 +200,8 @@ EXO_API int exo_batch_step(exo_batch *b, int nsteps, double dt_fixed);
 /* exo_conserved_sums of every member: out[member][5] */
 EXO_API int exo_batch_sums(exo_batch *b, double *out);
 /* exo_tune over the batch's launches (reused for a batch of the same member
- * configurations); exo_batch_set_caps sets widths, and from index EXO_NKINDS
- * on shapes, directly */
+ * configurations); exo_batch_set_caps sets an array of that layout directly;
+ * what it ends before keeps its value */
 EXO_API int exo_batch_tune(exo_batch *b, int reps, int *caps, int ncaps);
 EXO_API int exo_batch_set_caps(exo_batch *b, const int *caps, int ncaps);
 /* live kernel timing of the batch's launches (kernel ids as exo_profile_end;
