@@ -4095,7 +4095,7 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
     inst[i].ngd = (int)h->setup.ghosts.size();
     inst[i].ned = (int)h->setup.edges.size();
     L.lds_x1 = std::max(L.lds_x1, (size_t)(h->g.nc1 + 1) * 64 * sizeof(double));
-    if (!h->mixed) cols += (size_t)6 * h->g.N * h->g.N;
+    if (!h->mixed && h->g.eos == EOS_IDEAL) cols += (size_t)6 * h->g.N * h->g.N;
   }
   HIPCHK(hipGetDevice(&dev));
   HIPCHK(hipDeviceGetAttribute(&L.ncu, hipDeviceAttributeMultiprocessorCount, dev));
