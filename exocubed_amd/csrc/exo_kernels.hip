@@ -4630,27 +4630,42 @@ void run_stage(Launcher &L, int stage) {
   launch_fill_ghosts_stage(L);
 }
 
-// one stage of the shallow-water instances whose step is k_sw_stage's (mode 1)
-// last: of the last step of a call
-void launch_sw(Launcher &L, int stage, bool last) {
+// The work list in use until the end of a block, then the single phases' again,
+// also when a launch throws.
+struct ModeGuard {
+  Launcher &L;
+  ModeGuard(Launcher &l, int mode) : L(l) { L.mode = mode; }
+  ~ModeGuard() { L.mode = 0; }
+};
+
+// the tiles (K_SW or K_SW_MIX) of one stage of the shallow-water instances whose
+// step is k_sw_stage's (mode 1); last: of the last step of a call
+void launch_sw_tiles(Launcher &L, int kind, int stage, bool last) {
   int s0 = stage - 1;
   StageW sw{SS_DELTA[s0], SS_G1[s0], SS_G2[s0], SS_BETA[s0], s0 == 0 ? 1 : 0, 1, DFLOOR, SFLOOR};
   with_solver<EOS_SW>(L, [&](auto R) {
     constexpr int RK = decltype(R)::value;
-    auto tiles = [&](auto K) {
+    auto part = [&](auto K) {
       constexpr int PART = decltype(K)::value;
-      if (L.nblk[1][K_SW] <= L.ncu)
-        launch(L, K_SW, KID_UPDATE, k_sw_stage<false, RK, 512, PART>, 512, 0, sw, s0);
-      else launch(L, K_SW, KID_UPDATE, k_sw_stage<false, RK, 256, PART>, 256, 0, sw, s0);
-      if (L.nblk[1][K_SW_MIX] <= L.ncu)
-        launch(L, K_SW_MIX, KID_UPDATE, k_sw_stage<true, RK, 512, PART>, 512, 0, sw, s0);
-      else launch(L, K_SW_MIX, KID_UPDATE, k_sw_stage<true, RK, 256, PART>, 256, 0, sw, s0);
+      auto tiles = [&](auto M) {
+        constexpr bool MIX = decltype(M)::value;
+        if (L.nblk[1][kind] <= L.ncu)
+          launch(L, kind, KID_UPDATE, k_sw_stage<MIX, RK, 512, PART>, 512, 0, sw, s0);
+        else launch(L, kind, KID_UPDATE, k_sw_stage<MIX, RK, 256, PART>, 256, 0, sw, s0);
+      };
+      if (kind == K_SW) tiles(std::false_type{});
+      else tiles(std::true_type{});
     };
-    if (stage == 1) tiles(std::integral_constant<int, SW_FIRST>{});
-    else if (stage == 3 && last) tiles(std::integral_constant<int, SW_LAST>{});
-    else tiles(std::integral_constant<int, SW_LATER>{});
+    if (stage == 1) part(std::integral_constant<int, SW_FIRST>{});
+    else if (stage == 3 && last) part(std::integral_constant<int, SW_LAST>{});
+    else part(std::integral_constant<int, SW_LATER>{});
   });
-  launch(L, K_SW_HALO, KID_GHOST, k_sw_halo, BLK, 0, DFLOOR, s0);
+}
+
+void launch_sw(Launcher &L, int stage, bool last) {
+  launch_sw_tiles(L, K_SW, stage, last);
+  launch_sw_tiles(L, K_SW_MIX, stage, last);
+  launch(L, K_SW_HALO, KID_GHOST, k_sw_halo, BLK, 0, DFLOOR, stage - 1);
   HIPCHK(hipGetLastError());
 }
 
@@ -4658,11 +4673,7 @@ void launch_sw(Launcher &L, int stage, bool last) {
 // register are there (k_sw_stage leaves them only then; every other kernel does
 // always).
 void run_step(Launcher &L, double dt_fixed, bool last) {
-  struct Mode {  // back to the single phases' work list also when a launch throws
-    Launcher &L;
-    explicit Mode(Launcher &l) : L(l) { L.mode = 1; }
-    ~Mode() { L.mode = 0; }
-  } mode(L);
+  const ModeGuard mode(L, 1);
   launch_dt(L, dt_fixed);
   for (int stg = 1; stg <= 3; ++stg) {
     run_stage(L, stg);
@@ -4704,7 +4715,11 @@ struct KeepTimeStep {
 // Autotuner of the persistent launch width: for each launch kind that only
 // reads the conserved state (so repeating it changes nothing; the CFL minimum
 // also writes the time-step state, which is put back), time each candidate
-// width and keep the fastest.  Widths are multiples of the CU count.
+// width and keep the fastest.  Widths are multiples of the CU count.  A kind is
+// timed as a step launches it where a step does, else as the single phases do.
+// Of the fused shallow-water stages the second is repeated: it goes from u1 to
+// du, which nothing else of shallow water reads, and its halo from du to du and
+// the exchanged states, which are formed anew before each use.
 void tune_launcher(Launcher &L, int reps) {
   const KeepTimeStep keep(L);
   const int ncu = L.ncu;
@@ -4719,18 +4734,20 @@ void tune_launcher(Launcher &L, int reps) {
   launch_fluxes(L);
   StageW sw{1.0, 0.0, 1.0, 1.0, 1, 0, DFLOOR, SFLOOR};
   const int kinds[] = {K_PRIM, K_GHOST_U,  K_X1,          K_X1_MIX, K_EDGE,  K_EDGE_MIX,
-                       K_FACE, K_FACE_MIX, K_FACE_MIX_SW, K_DT,     K_FUSE2, K_FUSE2_MIX};
+                       K_FACE, K_FACE_MIX, K_FACE_MIX_SW, K_DT,     K_FUSE2, K_FUSE2_MIX,
+                       K_SW,   K_SW_MIX,   K_SW_HALO,     K_SW_EDGE};
   for (int kind : kinds) {
     std::vector<int> shapes = {0};  // the default first
     if (kind == K_X1 || kind == K_X1_MIX) shapes = {0, 2, 8};
     float best = 1e30f;
     int best_cap = 0, best_shape = 0;
+    int mode = kind != K_PRIM && L.nblk[1][kind] > 0;  // (a step has K_PRIM_REST)
     for (int sh : shapes) {
       set_shape(L, kind, sh);
-      if (L.nblk[0][kind] == 0) break;
+      if (L.nblk[mode][kind] == 0) break;
       std::vector<int> cands = {0};
       for (int m : {1, 2, 4, 8, 16})
-        if ((long long)m * ncu < L.nblk[0][kind]) cands.push_back(m * ncu);
+        if ((long long)m * ncu < L.nblk[mode][kind]) cands.push_back(m * ncu);
       for (int c : cands) {
         L.cap[kind] = c;
         for (int r = -1; r < reps; ++r) {  // r = -1 warms up
@@ -4740,6 +4757,7 @@ void tune_launcher(Launcher &L, int reps) {
           // warmed by the previous repetition (the conversion's own time is
           // the same for every candidate)
           if (kind != K_PRIM) launch_prim(L, -1);
+          const ModeGuard guard(L, mode);
           switch (kind) {
             case K_PRIM: launch_prim(L, -1); break;
             case K_GHOST_U: launch(L, K_GHOST_U, -1, k_ghost, BLK, 0); break;
@@ -4750,14 +4768,13 @@ void tune_launcher(Launcher &L, int reps) {
             case K_FACE: launch_face64<1>(L, K_FACE, -1); break;
             case K_FACE_MIX: launch_face_mix<1, false>(L, K_FACE_MIX, -1); break;
             case K_FACE_MIX_SW: launch_face_mix<1, true>(L, K_FACE_MIX_SW, -1); break;
-            case K_DT: {
-              Work none{nullptr, 0, 0};
-              k_dt<false><<<dim3(L.grid(K_DT)), dim3(BLK), 0, L.stream>>>(
-                  L.d_inst, L.work(K_DT), none, (int)L.grid(K_DT));
-              break;
-            }
+            case K_DT:
+            case K_SW_EDGE: launch_dt(L, 0.0); break;
             case K_FUSE2: launch_fuse2<false, false>(L, K_FUSE2, -1, sw); break;
             case K_FUSE2_MIX: launch_fuse2<false, true>(L, K_FUSE2_MIX, -1, sw); break;
+            case K_SW:
+            case K_SW_MIX: launch_sw_tiles(L, kind, 2, false); break;
+            case K_SW_HALO: launch(L, K_SW_HALO, -1, k_sw_halo, BLK, 0, DFLOOR, 1); break;
           }
         }
         HIPCHK(hipEventRecord(e1, L.stream));

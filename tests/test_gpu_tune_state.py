@@ -58,3 +58,31 @@ def test_tuned_batch_keeps_its_members_time_steps(ex):
         for p in pairs:
             p[0].close()
             p[1].close()
+
+
+@pytest.mark.parametrize("nx, mixed", [(34, False), (34, True), (128, False), (128, True)])
+def test_tuning_between_and_after_shallow_water_stages(ex, nx, mixed):
+    """the tuner repeats a fused stage and its halo: neither the stage register
+    nor the state may see it, and the tuned step is the untuned one's"""
+    cfg = sw_config(ex, nx=nx, nx1=2, rsolver=1)
+    cfg.precision = ex.PREC_MIXED if mixed else ex.PREC_FP64
+    g, twin = pair(ex, cfg)
+    for stage in (1, 2, 3):
+        g.tune(reps=1)
+        for m in (g, twin):
+            m.stage(stage, 2.0)
+    widths = g.tune(reps=1)
+    assert set(ex.LAUNCH_KINDS) <= set(widths)
+    assert g.step(3) == twin.step(3)
+    assert np.array_equal(g.download()[0], twin.download()[0])
+    assert np.array_equal(g.prim(), twin.prim())
+    g.close()
+    twin.close()
+    b = ex.Batch([pair(ex, cfg)[0], pair(ex, cfg)[0]])
+    b.set_caps({"sw_stage": 300, "sw_stage_mix": 300, "sw_halo": 5, "sw_edge": 3, "dt": 9})
+    b.step(2)
+    g = pair(ex, cfg)[0]
+    g.step(2)
+    for m in b.members:
+        assert np.array_equal(m.download()[0], g.download()[0])
+    b.close()
