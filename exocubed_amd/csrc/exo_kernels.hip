@@ -2812,14 +2812,17 @@ __device__ __forceinline__ void dt_body(const DGrid &g, const DState &st, int lb
     // as the next call finds them.  Minimum and count of blocks are kept in
     // DT_SLOTS lines, then once more over those: 1,728 blocks on one line took
     // 65 us on 6 x 96 x 96 x 64, 37 this way (42 with launches of their own
-    // for the reset and the result).  Only device-scope atomics touch
-    // the words, so waiting for each is order enough; a fence would write the
-    // caches back and drop them in every block (84 us).
+    // for the reset and the result).  A block's value has to be in before the
+    // block counts.  Only device-scope atomics touch the words, so it is enough
+    // that the first has returned before the second is issued: the empty
+    // statement takes its result, which the compiler waits for, and lets no
+    // access to memory past it.  A fence would write the caches back and drop
+    // them in every block (84 us).
     unsigned long long *top = (unsigned long long *)st.dtbits;
     int slot = lb % DT_SLOTS, slots = nblk < DT_SLOTS ? nblk : DT_SLOTS;
     auto last = [&](unsigned long long *q, unsigned long long v, int count) {
-      atomicMin(q, v);
-      __builtin_amdgcn_s_waitcnt(0);
+      unsigned long long before = atomicMin(q, v);
+      asm volatile("" ::"v"(before) : "memory");
       return atomicAdd(q + 1, 1ull) == (unsigned long long)(count - 1);
     };
     auto take = [&](unsigned long long *q) {  // the minimum; both words reset
