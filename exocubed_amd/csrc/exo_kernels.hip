@@ -635,7 +635,14 @@ size_t x1_lds(int nc1, int C) { return ((size_t)3 * nc1 + 2) * C; }
 // each; above, they read half a line of every row: 16 -> 8 columns, 6 x 32 x 32 x
 // 48 31 -> 26 us, 6 x 48 x 48 x 48 (3.4 blocks a CU) 51.6 -> 51.9, 6 x 64 x 64 x
 // 64 (6 a CU) 98 -> 107.
-constexpr int X1C = 16, X1C_FEW = 8, X1C_CU = 4;
+// With few levels, blocks of X1C columns leave most of their places for levels
+// empty (6 x 384 x 384 x 3: 4 faces on 16), and 64 columns, 4 levels at a time,
+// are faster where the launch has X1C_CU such blocks a CU as well: window -> 16
+// -> 64 columns, 6 x 384 x 384 x 3 420 -> 490 -> 258 us, 6 x 320 x 320 x 4 350 ->
+// 416 -> 216, 6 x 192 x 192 x 6 162 -> 163 -> 103; 16 -> 64 columns, 6 x 128 x 128 x
+// 20 140 -> 116, x 30 172 -> 177, 6 x 96 x 96 x 24 (3.4 such blocks a CU) 97 -> 96,
+// 6 x 64 x 64 x 20 (1.5) 44 -> 48.
+constexpr int X1C = 16, X1C_FEW = 8, X1C_FLAT = 64, X1C_CU = 4, X1_FLAT = 24;
 
 template <int W, int RK, int C>
 __device__ __forceinline__ void flux_x1_body(const DGrid &g, const DState &st, int lb, double *lds) {
@@ -766,6 +773,18 @@ k_flux_x1_few(const Inst *__restrict__ I_, Work w) {
   WORK_LOOP(w) {
     WORK_INST(w);
     flux_x1_body<W, RK, X1C_FEW>(g, st, lb, lds);
+    __syncthreads();  // the next block of the loop fills the LDS again
+  }
+}
+
+// and for one of many columns of few levels
+template <int W, int RK = -1>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4)))
+k_flux_x1_flat(const Inst *__restrict__ I_, Work w) {
+  extern __shared__ double lds[];
+  WORK_LOOP(w) {
+    WORK_INST(w);
+    flux_x1_body<W, RK, X1C_FLAT>(g, st, lb, lds);
     __syncthreads();  // the next block of the loop fills the LDS again
   }
 }
@@ -4086,7 +4105,8 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
   std::vector<int> tab((size_t)2 * K_NKIND * (n + 1));
   L.lds_x1 = L.lds_x1_fp64 = 0;
   int dev = 0;
-  size_t cols = 0;  // of the FP64 x1 sweep
+  size_t cols = 0;  // of the FP64 x1 sweep, and the levels of its highest ones
+  int levels = 0;
   for (int i = 0; i < n; ++i) {
     const exo_handle *h = hs[i];
     inst[i].g = h->g;
@@ -4098,11 +4118,15 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
     inst[i].ngd = (int)h->setup.ghosts.size();
     inst[i].ned = (int)h->setup.edges.size();
     L.lds_x1 = std::max(L.lds_x1, (size_t)(h->g.nc1 + 1) * 64 * sizeof(double));
-    if (!h->mixed && h->g.eos == EOS_IDEAL) cols += (size_t)6 * h->g.N * h->g.N;
+    if (!h->mixed && h->g.eos == EOS_IDEAL) {
+      cols += (size_t)6 * h->g.N * h->g.N;
+      levels = std::max(levels, h->g.nx1);
+    }
   }
   HIPCHK(hipGetDevice(&dev));
   HIPCHK(hipDeviceGetAttribute(&L.ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  L.x1c = cols < (size_t)X1C * X1C_CU * L.ncu ? X1C_FEW : X1C;
+  auto fill = [&](int c) { return cols >= (size_t)c * X1C_CU * L.ncu; };
+  L.x1c = !fill(X1C) ? X1C_FEW : levels <= X1_FLAT && fill(X1C_FLAT) ? X1C_FLAT : X1C;
   for (const exo_handle *h : hs)
     L.lds_x1_fp64 = std::max(L.lds_x1_fp64, x1_lds(h->g.nc1, L.x1c) * sizeof(double));
   L.eos = n > 0 ? hs[0]->g.eos : -1;
@@ -4468,7 +4492,8 @@ void launch_x1_w(Launcher &L, int kind, int kid) {
       launch(L, kind, kid, k_flux_x1_mix<W, decltype(R)::value>, 64 * W, L.lds_x1);
     });
   else if (L.x1c == X1C) launch(L, kind, kid, k_flux_x1<W>, 64 * W, L.lds_x1_fp64);
-  else launch(L, kind, kid, k_flux_x1_few<W>, 64 * W, L.lds_x1_fp64);
+  else if (L.x1c == X1C_FEW) launch(L, kind, kid, k_flux_x1_few<W>, 64 * W, L.lds_x1_fp64);
+  else launch(L, kind, kid, k_flux_x1_flat<W>, 64 * W, L.lds_x1_fp64);
 }
 
 void launch_x1(Launcher &L, int kind, int kid) {

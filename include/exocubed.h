@@ -160,8 +160,9 @@ EXO_API int exo_conserved_sums(exo_handle *h, double *out5);
  * state or only write the tendency (repeated launches change nothing): the
  * persistent launch width (the face kernels, the fused x2-face stage update
  * of instances without passive scalars, the primitive conversion, the ghost
- * remap, the CFL minimum, the fused shallow-water stage and its halo), and the x1 sweep's block shape (waves per block: 2,
- * 4 or 8; a block holds 64 columns in the mixed form, 16 or 8 in FP64).
+ * remap, the CFL minimum, the fused shallow-water stage and its halo), and the
+ * x1 sweep's block shape (waves per block: 2, 4 or 8; a block holds 64 columns
+ * in the mixed form, 8, 16 or 64 in FP64).
  * Each candidate is timed `reps` times and the fastest kept; a configuration
  * tuned before in this process reuses its result without timing.  caps (may
  * be NULL) receives up to ncaps values: the width of each launch kind (0 = one
