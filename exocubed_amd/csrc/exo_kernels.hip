@@ -5319,9 +5319,12 @@ extern "C" {
 int exo_step(exo_handle *h, int nsteps, double dt_fixed, double *dt_last) {
   return guarded(h, [&] {
     if (!h->have_state) throw std::string("no state uploaded");
-    if (nsteps > 1 && !h->L.prof) {  // replay a captured step (no per-kernel timing)
+    int replays = nsteps - (last_differs(h->L) ? 1 : 0);
+    // replay a captured step (no per-kernel timing); a single replay does not
+    // repay the capture
+    bool captured = h->exec && h->graph_dt_fixed == dt_fixed;
+    if (nsteps > 1 && !h->L.prof && (replays > 1 || captured)) {
       handle_graph(h, dt_fixed);
-      int replays = nsteps - (last_differs(h->L) ? 1 : 0);
       for (int s = 0; s < replays; ++s) HIPCHK(hipGraphLaunch(h->exec, h->stream));
       if (replays < nsteps) run_step(h->L, dt_fixed, true);
     } else {
