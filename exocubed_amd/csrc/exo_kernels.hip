@@ -623,8 +623,8 @@ __device__ __forceinline__ void psf_scan(const DGrid &g, const DState &st, int p
 // columns and four shares of the levels to a block, decomposed up to half of the
 // cells twice, waited for memory in the sum, and held 166 VGPRs: three waves a
 // SIMD, 864 blocks of 6 x 96 x 96 columns on 768 places.  Now four waves (127
-// VGPRs).  Bound by FP64 issue: 1390 VALU instructions a face, 0.13 of the
-// 0.19 ms.  Measured, window -> this: 6 x 96 x 96 x 64 234 -> 194 us, 6 x 64 x
+// VGPRs).  Bound by FP64 issue: 1480 VALU instructions a face, a SIMD's vector
+// ALU active 0.72 of the time.  Measured, window -> this: 6 x 96 x 96 x 64 234 -> 194 us, 6 x 64 x
 // 64 x 47 98 -> 67, 6 x 26 x 26 x 19 with a tracer 38 -> 14.  (Three or five
 // waves a SIMD, 32 columns, eight waves a block: 197 to 217 us.)
 // doubles of LDS: psf of nc1 + 1 faces, the perturbations of density and
@@ -3358,15 +3358,15 @@ __global__ void __launch_bounds__(BLK) k_flux_h_mix(const Inst *__restrict__ I_,
 // states), where the single phases take six (edge states, two face kernels,
 // update, ghost remap, ghost conversion), and the fluxes, the primitive state
 // and the stage register stay off memory.
-//   * Small spheres are bound by the launches, 4.7 us each in a replayed graph,
-//     and by a block's latency: 6 x 48 x 48 x 3 takes 75 us a step instead of
-//     109, 6 x 24 x 24 80 instead of 115.
+//   * Small spheres are bound by the chain of dependent loads and arithmetic of
+//     each launch, 8 to 11 us: 6 x 48 x 48 x 3 takes 68 us a step instead of
+//     109, 6 x 24 x 24 65 instead of 115.
 //   * Large ones moved some 270 bytes a cell and stage (face fluxes out and in,
 //     u, u1 and w); here a stage has to read its input (24 bytes) and the
 //     primitive state (stage 1) or the step's first state (24), writes 24, and
 //     reads 100 bytes of tables.  What is left is FP64 issue: 56 spheres of 24 to 182 cells a side
-//     (2.3 M cells, Roe) take 0.84 ms a step instead of 1.04, the stage kernel
-//     0.217 ms, 0.17 of it the issue of its instructions.
+//     (2.3 M cells, Roe) take 0.79 ms a step instead of 1.04, the stage kernel
+//     0.203 (first) and 0.220 ms, a SIMD's vector ALU active 0.73 of it.
 // Stages 2 and 3 convert u on the way into LDS (a tile its own 240 cells and up
 // to 186 of its neighbours': 1.5 to 1.75 conversions a cell), so the primitive
 // state is written only by the last one and read only by the first.  No stage

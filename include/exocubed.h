@@ -145,7 +145,9 @@ EXO_API int exo_sync(exo_handle *h);
 /* Live kernel timing: between begin and end every launch on the handle's stream
  * is bracketed by a HIP event pair; end returns the summed milliseconds and
  * launch counts per kernel id (0 prim, 1 ghost, 2 flux_x1, 3 edge_states,
- * 4 flux_x2, 5 flux_x3, 6 update, 7 implicit, 8 dt, 9 output). */
+ * 4 flux_x2, 5 flux_x3, 6 update, 7 implicit, 8 dt, 9 output).  Within a step
+ * the ideal gas's x2 faces and all of a stage of shallow water without scalars
+ * count as 6, that stage's halo as 1, its first panel-edge states with 8. */
 EXO_API int exo_profile_begin(exo_handle *h);
 EXO_API int exo_profile_end(exo_handle *h, double *ms, int *counts, int nkinds);
 
