@@ -4127,8 +4127,8 @@ void launcher_setup(Launcher &L, const std::vector<exo_handle *> &hs,
   HIPCHK(hipDeviceGetAttribute(&L.ncu, hipDeviceAttributeMultiprocessorCount, dev));
   auto fill = [&](int c) { return cols >= (size_t)c * X1C_CU * L.ncu; };
   L.x1c = !fill(X1C) ? X1C_FEW : levels <= X1_FLAT && fill(X1C_FLAT) ? X1C_FLAT : X1C;
-  for (const exo_handle *h : hs)
-    L.lds_x1_fp64 = std::max(L.lds_x1_fp64, x1_lds(h->g.nc1, L.x1c) * sizeof(double));
+  // (cols > 0: of the members that have the sweep, as others may be far taller)
+  if (cols > 0) L.lds_x1_fp64 = x1_lds(levels + 2 * NG, L.x1c) * sizeof(double);
   L.eos = n > 0 ? hs[0]->g.eos : -1;
   L.rs = n > 0 ? hs[0]->g.rs : -1;
   for (int i = 1; i < n; ++i) {

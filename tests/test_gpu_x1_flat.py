@@ -5,7 +5,7 @@ and every number of waves a block may have."""
 import numpy as np
 import pytest
 
-from helpers import atm_config
+from helpers import atm_config, sw_config
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +47,26 @@ def test_other_block_shapes(ex, waves):
     b.close()
     g.close()
     twin.close()
+
+
+def test_beside_far_taller_members(ex):
+    """the sweep's LDS is its own members': a batch with a tall mixed atmosphere
+    and many layers of water, each of which would ask for more than a CU has"""
+    mixed = atm_config(ex, nx=4, nx1=120)
+    mixed.precision = ex.PREC_MIXED
+    cfgs = [(atm_config(ex, nx=106, nx1=3), 1), (mixed, 1), (sw_config(ex, nx=4, nx1=300), 0)]
+    members, twins = [], []
+    for cfg, kind in cfgs:
+        u0, _ = ex.init_state(cfg, kind, 4)
+        for to in (members, twins):
+            m = ex.Solver(cfg)
+            m.upload(u0)
+            to.append(m)
+    b = ex.Batch(members)
+    b.step(2, 0.5)
+    for m, twin in zip(members, twins):
+        twin.step(2, 0.5)
+        assert np.array_equal(m.download()[0], twin.download()[0])
+    b.close()
+    for m in members + twins:
+        m.close()
